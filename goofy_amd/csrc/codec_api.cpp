@@ -69,8 +69,8 @@ void goofy_impl::quality_figures(const QualitySums& h, uint64_t pixels, goofy_qu
 {
     goofy_quality q{};
     q.pixels = pixels;
-    for (int i = 0; i < 4; ++i) q.sse_byte[i] = h.e[i];
-    q.sse_luma = (double)h.y100 / 10000.0;
+    for (int i = 0; i < 4; ++i) q.sse_byte[i] = h.sum[i];
+    q.sse_luma = (double)h.sum[4] / 10000.0;
     const double n = (double)q.pixels;
     // labels as in the reference harness: "r" = byte 2, "b" = byte 0
     q.mse_r = (double)q.sse_byte[2] / n;
@@ -92,24 +92,24 @@ void goofy_impl::quality_figures(const QualitySums& h, uint64_t pixels, goofy_qu
 
 extern "C" {
 
-// Device scratch of the quality sums, kept per device for reuse.  A call
-// returns its buffer only after synchronising its stream, so a buffer is never
-// shared by two calls in flight; no call frees one, because hipFree would wait
-// for every stream on the device (a quality check during serving would stall
-// the server's streams).
-// A quality call's buffers: device scratch (quality_scratch_bytes) and one
-// QualitySums of pinned host memory that the final-sum kernel writes.
+// Work areas of the quality calls, kept per device for reuse.  A call returns
+// its slot only after synchronising its stream, so a slot is never shared by
+// two calls in flight; no call frees one, because hipFree would wait for every
+// stream on the device (a quality check during serving would stall the
+// server's streams).
+// A slot: device work area (QualityAccum), pinned host memory for the words of
+// kQualityStripes launches, and whether the work area is known to be zero (not
+// when new, nor after a call that failed).
 struct QualitySlot {
     int device;
     void* d;
-    void* h;
+    QualityHost* h;
+    bool clean;
 };
 
 class QualityScratchPool {
 public:
-    static constexpr size_t kBytes = kQualityNoAllocBytes;
-
-    // A free slot of `device`, or a new one (device scratch and pinned host
+    // A free slot of `device`, or a new one (device work area and pinned host
     // memory allocated).  d == nullptr on failure.
     QualitySlot acquire(int device)
     {
@@ -122,11 +122,11 @@ public:
                     return s;
                 }
         }
-        QualitySlot s{device, nullptr, nullptr};
-        if (hipMalloc(&s.d, kBytes) != hipSuccess) return {device, nullptr, nullptr};
-        if (hipHostMalloc(&s.h, sizeof(QualitySums), hipHostMallocDefault) != hipSuccess) {
+        QualitySlot s{device, nullptr, nullptr, false};
+        if (hipMalloc(&s.d, sizeof(QualityAccum)) != hipSuccess) return {device, nullptr, nullptr, false};
+        if (hipHostMalloc((void**)&s.h, kQualityStripes * sizeof(QualityHost), hipHostMallocDefault) != hipSuccess) {
             (void)hipFree(s.d);
-            return {device, nullptr, nullptr};
+            return {device, nullptr, nullptr, false};
         }
         return s;
     }
@@ -147,34 +147,51 @@ static QualityScratchPool& quality_scratch_pool()
     return *pool;
 }
 
-// Runs `launch(scratch, host)` -- quality launches on `stream` whose last one
-// leaves the sums at offset 0 of scratch and at host (pinned) -- waits for the
-// stream and fills `out` with getMsePsnr's figures (Src/main.cpp:403-469).
+// Runs `launch(y0, rows, dest)` on `stream` for the stripes [y0, y0 + rows) of
+// `height` rows, at most max_rows each, waits for the stream and fills `out`
+// with getMsePsnr's figures (Src/main.cpp:403-469) from the stripes' sums.
 extern "C++" template <typename Launch>
-static int run_quality(uint64_t pixels, uint64_t units, hipStream_t stream, goofy_quality* out, Launch&& launch)
+static int run_quality(uint64_t pixels, uint32_t height, uint32_t max_rows, hipStream_t stream, goofy_quality* out,
+                       Launch&& launch)
 {
-    if (quality_scratch_bytes(units) > QualityScratchPool::kBytes) return fail(GOOFY_ERR_TOO_LARGE, "quality grid");
     DeviceInfo di;
     int rc = device_info(&di);
     if (rc != GOOFY_OK) return rc;
-    const QualitySlot slot = quality_scratch_pool().acquire(di.device);
-    if (!slot.d) return fail(GOOFY_ERR_OUT_OF_MEMORY, "quality scratch");
-    struct Release {  // on every path, the stream has drained before the slot is reused
+    struct Use {  // on every path, the stream has drained before the slot is reused
         QualitySlot slot;
         hipStream_t s;
-        ~Release()
+        bool done = false;
+        ~Use()
         {
-            (void)hipStreamSynchronize(s);
+            if (!slot.d) return;
+            if (!done) (void)hipStreamSynchronize(s);
+            slot.clean = done;
             quality_scratch_pool().release(slot);
         }
-    } guard{slot, stream};
-    hipError_t e = launch(slot.d, slot.h);
-    if (e != hipSuccess) return fail_hip(e, "quality kernel launch");
-    e = hipStreamSynchronize(stream);
-    if (e != hipSuccess) return fail_hip(e, "quality readback");
-    QualitySums h;
-    std::memcpy(&h, slot.h, sizeof h);
-    quality_figures(h, pixels, out);
+    } use{quality_scratch_pool().acquire(di.device), stream};
+    const QualitySlot& slot = use.slot;
+    if (!slot.d) return fail(GOOFY_ERR_OUT_OF_MEMORY, "quality scratch");
+    hipError_t e = hipSuccess;
+    if (!slot.clean && (e = hipMemsetAsync(slot.d, 0, sizeof(QualityAccum), stream)) != hipSuccess)
+        return fail_hip(e, "quality work area");
+    QualitySums sums{};
+    for (uint32_t y0 = 0; y0 < height;) {
+        uint32_t n = 0;
+        for (; n < kQualityStripes && y0 < height; ++n) {
+            const uint32_t rows = std::min(max_rows, height - y0);
+            e = launch(y0, rows, QualityDest{static_cast<QualityAccum*>(slot.d), slot.h + n, nullptr});
+            if (e != hipSuccess) return fail_hip(e, "quality kernel launch");
+            y0 += rows;
+        }
+        e = hipStreamSynchronize(stream);
+        if (e != hipSuccess) return fail_hip(e, "quality readback");
+        for (uint32_t i = 0; i < n; ++i) {
+            for (int k = 0; k < 5; ++k) sums.sum[k] += slot.h[i].word[k];
+            sums.sum[4] += slot.h[i].word[5] << 32;
+        }
+    }
+    use.done = true;
+    quality_figures(sums, pixels, out);
     return GOOFY_OK;
 }
 
@@ -186,18 +203,12 @@ int goofy_hip_quality_device(int format, const void* d_blocks, const void* d_sou
     int rc = check_image_device(format, d_source, d_blocks, width, height, pitch, true);
     if (rc != GOOFY_OK) return rc;
     if (width == 0 || height == 0) return fail(GOOFY_ERR_INVALID, "empty image");
-    const uint32_t bw = width / 4, bh = height / 4, max_rows = quality_stripe_rows(bw);
-    const uint64_t stripe_blocks = (uint64_t)bw * std::min(max_rows, bh);
-    return run_quality((uint64_t)width * height, stripe_blocks, (hipStream_t)stream, out, [&](void* scratch, void* host) {
-        hipError_t e = hipSuccess;
-        for (uint32_t y0 = 0; y0 < bh && e == hipSuccess;) {  // stripes beyond one launch's range
-            const uint32_t rows = std::min(max_rows, bh - y0);
-            e = launch_sqerr(format, static_cast<const uint8_t*>(d_blocks) + (size_t)y0 * bw * block_bytes(format),
-                             static_cast<const uint8_t*>(d_source) + (size_t)y0 * 4 * pitch, pitch, width, rows * 4,
-                             scratch, y0 > 0, host, (hipStream_t)stream);
-            y0 += rows;
-        }
-        return e;
+    const uint32_t bw = width / 4;
+    return run_quality((uint64_t)width * height, height / 4, quality_stripe_rows(bw), (hipStream_t)stream, out,
+                       [&](uint32_t y0, uint32_t rows, const QualityDest& dest) {
+        return launch_sqerr(format, static_cast<const uint8_t*>(d_blocks) + (size_t)y0 * bw * block_bytes(format),
+                            static_cast<const uint8_t*>(d_source) + (size_t)y0 * 4 * pitch, pitch, width, rows * 4,
+                            dest, false, (hipStream_t)stream);
     });
 }
 
@@ -226,8 +237,8 @@ int goofy_hip_quality_device_noalloc(int format, const void* d_blocks, const voi
     for (uint32_t y0 = 0; y0 < bh && e == hipSuccess;) {  // stripes beyond one launch's range
         const uint32_t rows = std::min(max_rows, bh - y0);
         e = launch_sqerr(format, static_cast<const uint8_t*>(d_blocks) + (size_t)y0 * bw * block_bytes(format),
-                         static_cast<const uint8_t*>(d_source) + (size_t)y0 * 4 * pitch, pitch, width, rows * 4, work,
-                         y0 > 0, nullptr, s);
+                         static_cast<const uint8_t*>(d_source) + (size_t)y0 * 4 * pitch, pitch, width, rows * 4,
+                         QualityDest{nullptr, nullptr, work}, y0 > 0, s);
         y0 += rows;
     }
     if (e != hipSuccess) return fail_hip(e, "quality kernel launch");
@@ -267,18 +278,11 @@ int goofy_hip_quality_images_device(const void* d_a, size_t pitch_a, const void*
     int rc = check_rgba_pair(d_a, pitch_a, d_b, pitch_b, width, height, 1);
     if (rc != GOOFY_OK) return rc;
     if (width == 0 || height == 0) return fail(GOOFY_ERR_INVALID, "empty image");
-    const uint32_t qw = width / 4, max_rows = quality_stripe_rows(qw);  // rows of qw 4-pixel units
-    const uint64_t stripe_units = (uint64_t)qw * std::min(max_rows, height);
-    return run_quality((uint64_t)width * height, stripe_units, (hipStream_t)stream, out, [&](void* scratch, void* host) {
-        hipError_t e = hipSuccess;
-        for (uint32_t y0 = 0; y0 < height && e == hipSuccess;) {
-            const uint32_t rows = std::min(max_rows, height - y0);
-            e = launch_sqerr_images(static_cast<const uint8_t*>(d_a) + (size_t)y0 * pitch_a, pitch_a,
-                                    static_cast<const uint8_t*>(d_b) + (size_t)y0 * pitch_b, pitch_b, width, rows,
-                                    scratch, y0 > 0, host, (hipStream_t)stream);
-            y0 += rows;
-        }
-        return e;
+    return run_quality((uint64_t)width * height, height, quality_stripe_rows(width / 4), (hipStream_t)stream, out,
+                       [&](uint32_t y0, uint32_t rows, const QualityDest& dest) {
+        return launch_sqerr_images(static_cast<const uint8_t*>(d_a) + (size_t)y0 * pitch_a, pitch_a,
+                                   static_cast<const uint8_t*>(d_b) + (size_t)y0 * pitch_b, pitch_b, width, rows,
+                                   dest, (hipStream_t)stream);
     });
 }
 

@@ -110,14 +110,42 @@ hipError_t launch_synth(const void* params, void* dst, uint32_t width, uint32_t 
                         hipStream_t stream);
 hipError_t launch_decode(int fmt, const void* blocks, void* dst, uint32_t width, uint32_t height, size_t pitch,
                          hipStream_t stream);
-// Quality sums: squared errors of bytes 0..3, and the sum of squared luma
-// differences times 10^4 (an exact integer with the harness's weights).  The
-// quality launchers take a device scratch buffer of quality_scratch_bytes():
-// the final sums at offset 0, one partial per workgroup from
-// kQualityPartialsOffset on.
+// Quality sums: squared errors of bytes 0..3, then the sum of squared luma
+// differences times 10^4 (an exact integer with the harness's weights).
 struct QualitySums {
-    unsigned long long e[4];
-    unsigned long long y100;
+    unsigned long long sum[5];
+};
+// The same sums as a pooled call's kernel passes them on: six words, the luma
+// sum in two (its low and high 32 bits, each summed by itself), every word
+// with a count of its contributions above kQualityCountBit.  A launch's sums
+// stay below that bit: at most 2^33.6 pixels (kQualityMaxLaunchUnits blocks)
+// of 255^2 < 2^16, and 1536 low words below 2^32.
+constexpr uint32_t kQualityWords = 6;
+constexpr uint32_t kQualityCountBit = 52;
+// Device work area of a pooled call, all zero between launches: the
+// workgroups' words spread over the slots (a line each), and their total.
+constexpr uint32_t kQualitySlots = 64;
+struct QualityAccum {
+    struct alignas(64) Line {
+        unsigned long long word[kQualityWords];
+    } slot[kQualitySlots], total;
+};
+// Pinned host memory: the words of one launch, without counts.
+struct QualityHost {
+    unsigned long long word[kQualityWords];
+};
+// A pooled call waits after this many stripes, each with a QualityHost.
+constexpr uint32_t kQualityStripes = 16;
+// Where a quality launch leaves its sums.  Pooled: the zeroed accum on the way
+// and *host (pinned) in the end.  Allocation-free (host null): work has the
+// final sums at offset 0 and one partial per workgroup from
+// kQualityPartialsOffset on; every partial the final kernel reads is written
+// by the launch before it, and the first stripe replaces the sums, so that
+// area needs no clearing between calls.
+struct QualityDest {
+    QualityAccum* accum;
+    QualityHost* host;
+    void* work;
 };
 constexpr size_t kQualityPartialsOffset = 64;
 constexpr uint32_t kQualityMaxGroups = 1536;
@@ -140,18 +168,14 @@ inline uint32_t quality_stripe_rows(uint64_t units_per_row)
     const uint64_t r = max_stripe_brows(units_per_row), cap = kQualityMaxLaunchUnits / (units_per_row ? units_per_row : 1);
     return (uint32_t)(r < cap ? r : cap);
 }
-// accumulate: add onto the sums already at offset 0 of `work` (later
-// stripes of one image on the same stream) instead of replacing them.
-// host_out: null, or pinned host memory for a copy of the sums at offset 0
-// (one QualitySums), valid once the stream has drained.  Every partial the
-// final kernel reads is written by the launch before it, and the first stripe
-// replaces the sums, so `work` needs no clearing between calls.
+// accumulate (allocation-free): add onto the sums already at offset 0 of the
+// work area (later stripes of one image on the same stream).
 hipError_t launch_sqerr(int fmt, const void* blocks, const void* src, size_t pitch, uint32_t width, uint32_t height,
-                        void* work, bool accumulate, void* host_out, hipStream_t stream);
+                        const QualityDest& dest, bool accumulate, hipStream_t stream);
 hipError_t launch_sqerr_images(const void* a, size_t pitch_a, const void* b, size_t pitch_b, uint32_t width,
-                               uint32_t height, void* work, bool accumulate, void* host_out, hipStream_t stream);
-// Size of the largest quality work area (kQualityMaxGroups partials), the
-// size of the allocation-free call's fixed device array.
+                               uint32_t height, const QualityDest& dest, hipStream_t stream);
+// Size of the allocation-free call's fixed device array (kQualityMaxGroups
+// partials).
 constexpr size_t kQualityNoAllocBytes = kQualityPartialsOffset + (size_t)kQualityMaxGroups * sizeof(QualitySums);
 // Device address of `device`'s copy of that array (the current device of the
 // calling thread), looked up once per device and kept.

@@ -404,6 +404,50 @@ def test_quality_images_closed_form(gpu):
     assert q["psnr_rgb"] == pytest.approx(10 * math.log10(768.0 ** 2 / 4.0), abs=1e-12)
 
 
+def test_quality_sums_finished_by_the_last_workgroup(gpu):
+    """The sums come together in 64 slots of a kept work area: grids of fewer
+    workgroups than slots, as many, one more, uneven and full slots (1536
+    workgroups, also with several units a lane), each call twice and larger
+    ones before smaller, so that a slot or a counter that one call leaves
+    behind shows in the next.  1024 pixels a row are one workgroup."""
+    from goofy_amd import hip
+    w = 1024
+    rng = np.random.default_rng(17)
+    a = rng.integers(0, 256, w * 4 * 1700, dtype=np.uint8)
+    b = rng.integers(0, 256, w * 4 * 1700, dtype=np.uint8)
+    da, db = hip.DeviceBuffer.from_array(a), hip.DeviceBuffer.from_array(b)
+    for h in (1700, 1, 1536, 2, 1535, 63, 129, 64, 65, 1):
+        print(f"quality grid of {min(h, 1536)} workgroups", flush=True)
+        sse, y100 = integer_sums(a[:w * 4 * h], b[:w * 4 * h])
+        for _ in range(2):
+            q = gpu.quality_images_device(da, db, w, h)
+            assert q["sse_byte"] == sse and q["sse_luma"] == y100 / 1e4, h
+
+
+def test_quality_call_refused_under_capture_leaves_no_trace(gpu):
+    """A quality call cannot be captured: it reports so, and the calls after
+    it, on the same kept work area, are right."""
+    import ctypes
+
+    from goofy_amd import hip
+    w, h = 256, 64
+    rng = np.random.default_rng(18)
+    a, b = (rng.integers(0, 256, w * h * 4, dtype=np.uint8) for _ in range(2))
+    da, db = hip.DeviceBuffer.from_array(a), hip.DeviceBuffer.from_array(b)
+    sse, _ = integer_sums(a, b)
+    assert gpu.quality_images_device(da, db, w, h)["sse_byte"] == sse
+    s = hip.Stream()
+    graph = ctypes.c_void_p()
+    assert hip._hip.hipStreamBeginCapture(ctypes.c_void_p(s.handle), 2) == 0  # relaxed
+    with pytest.raises(gpu.GoofyError) as e:
+        gpu.quality_images_device(da, db, w, h, stream=s)
+    hip._hip.hipStreamEndCapture(ctypes.c_void_p(s.handle), ctypes.byref(graph))
+    hip._hip.hipGetLastError()
+    assert e.value.status == gpu.ERR_HIP
+    for _ in range(2):
+        assert gpu.quality_images_device(da, db, w, h)["sse_byte"] == sse
+
+
 def test_quality_calls_from_threads_share_the_scratch_pool(gpu):
     """Quality calls on four threads and streams at once (the library keeps a
     pool of scratch buffers): every result equals the same call made alone."""
