@@ -20,7 +20,7 @@ Also reported:
   shapes);
 * the decoders, the RGB565 quality floor and the quality sums on the 8192^2
   image;
-* the batched workload: 4096 textures in one autotuned graph launch against
+* the batched workload: 4096 textures in one autotuned launch against
   4096 plain launches;
 * the serving workload: Poisson arrivals, p50/p99 latency, and capacity
   batched against one launch per request;
@@ -293,7 +293,7 @@ def bench_stress(g, hip, W, launches: int = 20):
 # ---- batched --------------------------------------------------------------------------------
 
 def bench_batch(g, hip, W, reps: int = 7, align: int = 16, per_texture: bool = True, widths=(0, 1 << 30)):
-    """The 4096-texture batch as one hipGraph replay, autotuned shape.  Rows
+    """The 4096-texture batch as one launch, autotuned shape.  Rows
     are `align`-byte aligned (16: the tight pitch width * 4); with
     per_texture the same textures also run as one plain launch each, for the
     speedup and a block-for-block comparison.  widths = [lo, hi): only the

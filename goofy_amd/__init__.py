@@ -381,7 +381,7 @@ def traffic_probe(dst, src, width: int, height: int, pitch: int, start_event=Non
 
 
 class Batch:
-    """Many device-resident textures encoded by one persistent-kernel launch (hipGraph replay)."""
+    """Many device-resident textures encoded by one kernel launch."""
 
     def __init__(self, textures: Sequence[dict], config: LaunchConfig | dict | None = None):
         arr = (TextureDesc * max(1, len(textures)))()

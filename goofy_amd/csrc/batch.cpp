@@ -5,13 +5,11 @@
 // prefix sum over ceil(blocks(t) / tile).  Tiles never straddle textures, so
 // a wave's loads stay contiguous and its format is uniform.  One kernel launch
 // walks the whole list (kernels.hip, k_encode_batch), one wave per tile or a
-// persistent grid of waves that each take a contiguous run of tiles; the
-// launch is captured once into a hipGraph and replayed.  The launch shape
-// (blocks per lane, workgroup size, persistent waves per CU, streaming hints)
-// comes from an
-// autotuner that times the candidates on the plan itself and caches the
-// winner per shape class for the process (and, with GOOFY_TUNE_CACHE=<file>,
-// across processes).
+// persistent grid of waves that each take a contiguous run of tiles.  The
+// launch shape (blocks per lane, workgroup size, persistent waves per CU,
+// streaming hints) comes from an autotuner that times the candidates on the
+// plan itself and caches the winner per shape class for the process (and, with
+// GOOFY_TUNE_CACHE=<file>, across processes).
 //
 // The reference has no batching: its driver encodes one image with one
 // nested loop (GoofyTC/goofy_tc.h:1514-1524).
@@ -45,18 +43,15 @@ struct goofy_batch {
     uint64_t blocks = 0, pixels = 0;
     bool alpha = false;  // holds DXT5 / ETC2 RGBA8 textures
     LaunchCfg cfg{};
-    hipStream_t capture_stream = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    // Recorded after every graph launch, on the caller's stream: the work-list
-    // is rewritten or freed only once the launches that read it have finished.
+    // Recorded by every launch's own dispatch: the work-list is rewritten or
+    // freed only once the launches that read it have finished.
     hipEvent_t launched = nullptr;
     bool launched_pending = false;
 };
 
 namespace {
 
-// Waits for the plan's last graph launch (which may be on a caller's
+// Waits for the plan's last launch (which may be on a caller's
 // non-blocking stream, which a synchronous copy does not wait for).
 int wait_launched(goofy_batch* b)
 {
@@ -65,17 +60,6 @@ int wait_launched(goofy_batch* b)
     if (e != hipSuccess) return fail_hip(e, "hipEventSynchronize(batch launch)");
     b->launched_pending = false;
     return GOOFY_OK;
-}
-
-void drop_graph(goofy_batch* b)
-{
-    if (b->exec) {
-        (void)wait_launched(b);
-        (void)hipGraphExecDestroy(b->exec);
-    }
-    if (b->graph) (void)hipGraphDestroy(b->graph);
-    b->exec = nullptr;
-    b->graph = nullptr;
 }
 
 // Rebuild the tile prefix sums for the plan's tile size and upload them.
@@ -127,37 +111,6 @@ int build_worklist(goofy_batch* b)
     }
     e = hipMemcpy(b->d_descs, host.data(), bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) return fail_hip(e, "hipMemcpy(work-list)");
-    drop_graph(b);
-    return GOOFY_OK;
-}
-
-int capture(goofy_batch* b)
-{
-    if (b->exec) return GOOFY_OK;
-    hipError_t e;
-    if (!b->capture_stream) {
-        e = hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking);
-        if (e != hipSuccess) return fail_hip(e, "hipStreamCreate");
-    }
-    e = hipStreamBeginCapture(b->capture_stream, hipStreamCaptureModeThreadLocal);
-    if (e != hipSuccess) return fail_hip(e, "hipStreamBeginCapture");
-    hipError_t le = launch_batch(b->cfg, b->d_descs, (uint32_t)b->descs.size(), b->ntiles, b->num_cus,
-                                 b->capture_stream, b->alpha);
-    hipGraph_t g = nullptr;
-    e = hipStreamEndCapture(b->capture_stream, &g);
-    if (le != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        return fail_hip(le, "batch kernel launch (capture)");
-    }
-    if (e != hipSuccess) return fail_hip(e, "hipStreamEndCapture");
-    hipGraphExec_t x = nullptr;
-    e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-    if (e != hipSuccess) {
-        (void)hipGraphDestroy(g);
-        return fail_hip(e, "hipGraphInstantiate");
-    }
-    b->graph = g;
-    b->exec = x;
     return GOOFY_OK;
 }
 
@@ -294,14 +247,22 @@ int goofy_batch_launch(goofy_batch* b, void* stream)
     clear_error();
     if (!b) return fail(GOOFY_ERR_INVALID, "null batch");
     if (b->ntiles == 0) return GOOFY_OK;
-    int rc = capture(b);
-    if (rc != GOOFY_OK) return rc;
-    hipError_t e = hipGraphLaunch(b->exec, (hipStream_t)stream);
-    if (e != hipSuccess) return fail_hip(e, "hipGraphLaunch");
+    const hipStream_t s = (hipStream_t)stream;
+    hipError_t e;
     if (!b->launched && (e = hipEventCreateWithFlags(&b->launched, hipEventDisableTiming)) != hipSuccess)
         return fail_hip(e, "hipEventCreate");
-    if ((e = hipEventRecord(b->launched, (hipStream_t)stream)) != hipSuccess) return fail_hip(e, "hipEventRecord");
-    b->launched_pending = true;
+    // One kernel: a plain launch.  A hipGraph of this one node cost the host
+    // 15-17 us a launch on MI355X (4 ms the first time), the kernel launch
+    // 2.8 us, and an event recorded behind it 5 us more than one that the
+    // kernel's own dispatch records.  A stream that is being captured takes
+    // the launch as a node, without the event.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();  // the launch says why
+    const bool eager = cap == hipStreamCaptureStatusNone;
+    e = launch_batch(b->cfg, b->d_descs, (uint32_t)b->descs.size(), b->ntiles, b->num_cus, s, b->alpha,
+                     eager ? b->launched : nullptr);
+    if (e != hipSuccess) return fail_hip(e, "batch kernel launch");
+    if (eager) b->launched_pending = true;
     return GOOFY_OK;
 }
 
@@ -344,9 +305,7 @@ int goofy_batch_set_config(goofy_batch* b, const goofy_launch_config* cfg)
     if (!cfg_valid(c)) return fail(GOOFY_ERR_INVALID, "invalid launch config");
     const bool retile = c.blocks_per_lane != b->cfg.blocks_per_lane;
     b->cfg = c;
-    if (retile) return build_worklist(b);
-    drop_graph(b);
-    return GOOFY_OK;
+    return retile ? build_worklist(b) : wait_launched(b);
 }
 
 int goofy_batch_autotune(goofy_batch* b, void* stream, int reps, goofy_launch_config* chosen, float* best_ms)
@@ -436,8 +395,6 @@ int goofy_batch_destroy(goofy_batch* b)
     if (!b) return GOOFY_OK;
     (void)wait_launched(b);
     if (b->launched) (void)hipEventDestroy(b->launched);
-    drop_graph(b);
-    if (b->capture_stream) (void)hipStreamDestroy(b->capture_stream);
     if (b->d_descs) (void)hipFree(b->d_descs);
     delete b;
     return GOOFY_OK;

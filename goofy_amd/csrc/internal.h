@@ -104,6 +104,9 @@ hipError_t launch_dual_alpha(uint32_t wg_waves, const void* src, size_t pitch, v
 // instance with all four formats; without, DXT1 / ETC1S only).
 hipError_t launch_batch(const LaunchCfg& cfg, const TexDesc* d_descs, uint32_t ntex, uint32_t ntiles, int num_cus,
                         hipStream_t stream, bool alpha = false);
+// The same with an event that the kernel's own dispatch records (or null).
+hipError_t launch_batch(const LaunchCfg& cfg, const TexDesc* d_descs, uint32_t ntex, uint32_t ntiles, int num_cus,
+                        hipStream_t stream, bool alpha, hipEvent_t done);
 hipError_t launch_batch_inline(const LaunchCfg& cfg, const InlineWorklist& wl, uint32_t ntex, uint32_t ntiles,
                                int num_cus, hipStream_t stream, bool alpha = false);
 hipError_t launch_synth(const void* params, void* dst, uint32_t width, uint32_t height, size_t pitch,

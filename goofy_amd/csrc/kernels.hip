@@ -398,26 +398,31 @@ hipError_t launch_dual_alpha(uint32_t wg_waves, const void* src, size_t pitch, v
 
 template <int BPL, bool ALPHA>
 static hipError_t batch_go(bool nt, dim3 grid, dim3 block, const TexDesc* d, const uint32_t* tb, uint32_t ntex,
-                           uint32_t ntiles, uint32_t tpw, uint32_t order, hipStream_t s)
+                           uint32_t ntiles, uint32_t tpw, uint32_t order, hipStream_t s, hipEvent_t done)
 {
     const uint32_t wpg = block.x / 64u;
-    if (nt)
-        hipLaunchKernelGGL((k_encode_batch<BPL, true, ALPHA>), grid, block, 0, s, d, tb, ntex, ntiles, tpw, order, wpg);
-    else
-        hipLaunchKernelGGL((k_encode_batch<BPL, false, ALPHA>), grid, block, 0, s, d, tb, ntex, ntiles, tpw, order, wpg);
+    const auto go = [&](auto kernel) {
+        if (done)
+            hipExtLaunchKernelGGL(kernel, grid, block, 0, s, nullptr, done, 0, d, tb, ntex, ntiles, tpw, order, wpg);
+        else
+            hipLaunchKernelGGL(kernel, grid, block, 0, s, d, tb, ntex, ntiles, tpw, order, wpg);
+    };
+    if (nt) go(k_encode_batch<BPL, true, ALPHA>);
+    else go(k_encode_batch<BPL, false, ALPHA>);
     return hipGetLastError();
 }
 
 template <int BPL>
 static hipError_t batch_nt(bool nt, bool alpha, dim3 grid, dim3 block, const TexDesc* d, const uint32_t* tb,
-                           uint32_t ntex, uint32_t ntiles, uint32_t tpw, uint32_t order, hipStream_t s)
+                           uint32_t ntex, uint32_t ntiles, uint32_t tpw, uint32_t order, hipStream_t s,
+                           hipEvent_t done)
 {
-    return alpha ? batch_go<BPL, true>(nt, grid, block, d, tb, ntex, ntiles, tpw, order, s)
-                 : batch_go<BPL, false>(nt, grid, block, d, tb, ntex, ntiles, tpw, order, s);
+    return alpha ? batch_go<BPL, true>(nt, grid, block, d, tb, ntex, ntiles, tpw, order, s, done)
+                 : batch_go<BPL, false>(nt, grid, block, d, tb, ntex, ntiles, tpw, order, s, done);
 }
 
 hipError_t launch_batch(const LaunchCfg& c, const TexDesc* d_descs, uint32_t ntex, uint32_t ntiles, int num_cus,
-                        hipStream_t stream, bool alpha)
+                        hipStream_t stream, bool alpha, hipEvent_t done)
 {
     if (ntiles == 0 || ntex == 0) return hipSuccess;
     const uint32_t* tb = worklist_tile_begin(d_descs, ntex);
@@ -427,11 +432,18 @@ hipError_t launch_batch(const LaunchCfg& c, const TexDesc* d_descs, uint32_t nte
     waves = (ntiles + tpw - 1) / tpw;
     const uint32_t wg = (uint32_t)c.wg_waves;
     const dim3 grid((uint32_t)((waves + wg - 1) / wg)), block(64u * wg);
+    const bool nt = c.nontemporal;
     switch (c.blocks_per_lane) {
-    case 1: return batch_nt<1>(c.nontemporal, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, c.tile_order, stream);
-    case 2: return batch_nt<2>(c.nontemporal, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, c.tile_order, stream);
-    default: return batch_nt<4>(c.nontemporal, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, c.tile_order, stream);
+    case 1: return batch_nt<1>(nt, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, c.tile_order, stream, done);
+    case 2: return batch_nt<2>(nt, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, c.tile_order, stream, done);
+    default: return batch_nt<4>(nt, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, c.tile_order, stream, done);
     }
+}
+
+hipError_t launch_batch(const LaunchCfg& c, const TexDesc* d_descs, uint32_t ntex, uint32_t ntiles, int num_cus,
+                        hipStream_t stream, bool alpha)
+{
+    return launch_batch(c, d_descs, ntex, ntiles, num_cus, stream, alpha, nullptr);
 }
 
 template <int BPL, bool ALPHA>

@@ -257,8 +257,7 @@ GOOFY_HIP_API int goofy_hip_traffic_probe(void* d_out, const void* d_input, unsi
 /* ---- batched encode: many textures, one launch -----------------------------
  * A plan flattens the block work-lists of n device-resident textures (each
  * its own size, pitch and format) into one wave-tile list and encodes all of
- * them with one kernel launch, captured once into a hipGraph.  The launch
- * runs one wave per tile, or a persistent grid (waves_per_cu > 0) in which
+ * them with one kernel launch.  The launch runs one wave per tile, or a persistent grid (waves_per_cu > 0) in which
  * each wave takes a contiguous run of tiles; the autotuner times both. */
 typedef struct goofy_texture_desc {
     const void* src;     /* device RGBA8, 16-byte aligned */
@@ -277,7 +276,8 @@ typedef struct goofy_batch goofy_batch;
  * themselves stay owned by the caller). */
 GOOFY_HIP_API int goofy_batch_create(const goofy_texture_desc* textures, size_t count,
                                      const goofy_launch_config* cfg, goofy_batch** out);
-/* Enqueue the whole batch on `stream` (replays the captured graph). */
+/* Enqueue the whole batch on `stream`: one kernel launch (a node of the graph
+ * when the stream is being captured). */
 GOOFY_HIP_API int goofy_batch_launch(goofy_batch* batch, void* stream);
 /* Same work as individual launches (one plain kernel per texture, or per
  * horizontal stripe for textures beyond one launch's index range), for

@@ -428,6 +428,57 @@ def test_batch_vs_oracle_and_configs(gpu, oracle):
     b.close()
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2])  # global, thread-local, relaxed capture
+def test_batch_captured_then_replayed_and_reshaped(gpu, oracle, mode):
+    """A batch launch on a capturing stream becomes a node of the caller's
+    graph; replays with eager work between them give the blocks, the plan can
+    be launched and reshaped afterwards, and launches on two streams with no
+    wait before the reshape are waited for by it."""
+    import ctypes
+
+    from goofy_amd import hip
+    sizes = [(64, 64), (68, 20), (260, 132), (1028, 4)]
+    items, want = [], []
+    for i, (w, h) in enumerate(sizes):
+        img = gpu.synth_host(0, 40 + i, i, 12, w, h)
+        fmt = i & 1
+        items.append(dict(src=hip.DeviceBuffer.from_array(img), dst=hip.DeviceBuffer((w // 4) * (h // 4) * 8, fill=0xCD),
+                          width=w, height=h, format=fmt))
+        want.append(oracle.compress_blocks(fmt, img, w, h, w * 4))
+    b = gpu.Batch(items)
+
+    def check(tag):
+        hip.synchronize()
+        for it, wv in zip(items, want):
+            assert np.array_equal(it["dst"].download(), wv), tag
+            it["dst"].fill(0xCD)
+        hip.synchronize()
+
+    rt, s, s2 = hip._hip, hip.Stream(), hip.Stream()
+    graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+    hip.synchronize()
+    assert rt.hipStreamBeginCapture(ctypes.c_void_p(s.handle), mode) == 0
+    b.launch(s)
+    assert rt.hipStreamEndCapture(ctypes.c_void_p(s.handle), ctypes.byref(graph)) == 0
+    assert rt.hipGraphInstantiate(ctypes.byref(run), graph, None, None, 0) == 0
+    for r in range(3):
+        say(f"batch captured, mode {mode}, replay {r}")
+        assert rt.hipGraphLaunch(run, ctypes.c_void_p(s.handle)) == 0
+        check(f"replay {r}")
+        b.launch()  # eager work between the replays
+        check(f"eager {r}")
+    assert rt.hipGraphExecDestroy(run) == 0 and rt.hipGraphDestroy(graph) == 0
+    for bpl in (2, 1):
+        b.launch(s)
+        b.launch(s2)
+        b.config = dict(blocks_per_lane=bpl, wg_waves=4, waves_per_cu=0, nontemporal=1, tile_order=0)
+        b.launch(s2)
+        check(f"reshaped {bpl}")
+    b.close()
+    s.destroy()
+    s2.destroy()
+
+
 def test_batch_full_workload(gpu, oracle):
     """The 4096-texture workload: batch output equals per-texture launches on
     every texture, and the oracle on a sample of textures."""
