@@ -76,7 +76,8 @@ int device_info(DeviceInfo* out)
 
 // Measured on MI355X (8192^2, both formats): one block per lane with
 // streaming (non-temporal) loads and stores is fastest; 1-4 wave workgroups
-// are within noise of each other, 4 blocks per lane loses ~10%.
+// are within noise of each other, 4 blocks per lane loses ~10%.  Large launches
+// into the 8-byte formats and batches start from this in wide_cfg.
 // One block per lane, streaming, linear tile order, and the largest
 // workgroup (8, 4, 2 or 1 waves) that still leaves two workgroups per CU.
 // 8-wave workgroups are the fastest shape on large images (on the 8192^2
@@ -310,7 +311,7 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
             copy_rows(in, input + (size_t)r0 * 4 * stride, stride, row_bytes, rows * 4);
             e = dual_alpha ? launch_dual_alpha((uint32_t)cfg.wg_waves, in, row_bytes, out, out + n, bw, bw * rows,
                                                ctx->stream)
-                : dual     ? launch_dual((uint32_t)cfg.wg_waves, in, row_bytes, out, out + n, bw, bw * rows, ctx->stream)
+                : dual     ? launch_dual(cfg, in, row_bytes, out, out + n, bw, bw * rows, ctx->stream)
                            : launch_plain(fmt, cfg, in, row_bytes, out, bw, bw * rows, ctx->stream);
         }
         if (e == hipSuccess) e = hipEventRecord(ctx->out_ready[0], ctx->stream);
@@ -341,7 +342,7 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
         uint8_t* second = static_cast<uint8_t*>(kout) + n;
         e = dual_alpha ? launch_dual_alpha((uint32_t)cfg.wg_waves, kin, row_bytes, kout, second, bw, bw * rows,
                                            ctx->stream)
-            : dual     ? launch_dual((uint32_t)cfg.wg_waves, kin, row_bytes, kout, second, bw, bw * rows, ctx->stream)
+            : dual     ? launch_dual(cfg, kin, row_bytes, kout, second, bw, bw * rows, ctx->stream)
                        : launch_plain(fmt, cfg, kin, row_bytes, kout, bw, bw * rows, ctx->stream);
         if (e != hipSuccess) break;
         if ((e = hipMemcpyAsync(ctx->h_out[s], ctx->d_out[s], outs * n, hipMemcpyDeviceToHost, ctx->stream)) !=
@@ -395,7 +396,7 @@ static int compress_device(int fmt, void* d_result, const void* d_input, unsigne
     for (uint32_t y0 = 0; y0 < bh;) {
         const uint32_t rows = std::min(max_rows, bh - y0);
         const uint32_t nb = rows * bw;  // <= 0xFFFFFFFF by max_stripe_brows
-        const LaunchCfg c = ucfg ? cfg : auto_cfg(nb, num_cus);
+        const LaunchCfg c = ucfg ? cfg : plain_cfg(fmt, nb, num_cus);
         hipError_t e = launch_plain(fmt, c, static_cast<const uint8_t*>(d_input) + (size_t)y0 * 4 * pitch, pitch,
                                     static_cast<uint8_t*>(d_result) + (size_t)y0 * bw * bb, bw, nb,
                                     (hipStream_t)stream, y0 == 0 ? (hipEvent_t)ev_start : nullptr,
@@ -524,14 +525,15 @@ static int compress_device_pair(bool alpha, void* d_a, void* d_b, const void* d_
         const uint32_t rows = std::min(max_rows, bh - y0);
         const uint32_t nb = rows * bw;
         const size_t out_off = (size_t)y0 * bw * bb;
-        const uint32_t wg = (uint32_t)auto_cfg(nb, di.num_cus).wg_waves;
         const uint8_t* in = static_cast<const uint8_t*>(d_input) + (size_t)y0 * 4 * pitch;
         uint8_t* a = static_cast<uint8_t*>(d_a) + out_off;
         uint8_t* b = static_cast<uint8_t*>(d_b) + out_off;
         hipEvent_t e0 = y0 == 0 ? (hipEvent_t)start_event : nullptr;
         hipEvent_t e1 = y0 + rows == bh ? (hipEvent_t)stop_event : nullptr;
-        hipError_t e = alpha ? launch_dual_alpha(wg, in, pitch, a, b, bw, nb, (hipStream_t)stream, e0, e1)
-                             : launch_dual(wg, in, pitch, a, b, bw, nb, (hipStream_t)stream, e0, e1);
+        hipError_t e = alpha ? launch_dual_alpha((uint32_t)auto_cfg(nb, di.num_cus).wg_waves, in, pitch, a, b, bw, nb,
+                                                 (hipStream_t)stream, e0, e1)
+                             : launch_dual(wide_cfg(nb, di.num_cus), in, pitch, a, b, bw, nb, (hipStream_t)stream, e0,
+                                           e1);
         if (e != hipSuccess) return fail_hip(e, "dual encode kernel launch");
         y0 += rows;
     }

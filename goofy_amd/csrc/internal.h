@@ -33,13 +33,22 @@ struct LaunchCfg {
     int wg_waves;         // waves per workgroup: 1, 2, 4 or 8
     int waves_per_cu;     // persistent grid size (0 = one wave per tile, no persistence)
     int nontemporal;      // 1 = streaming (non-temporal) loads and stores
-    int tile_order;       // 0 = linear, 1 = XCD-contiguous (kXcdCount groups of workgroups)
+    int tile_order;       // 0 = linear, 1 = runs of kXcdRunTiles tiles per XCD
 };
 
 // The dispatcher hands workgroup b to XCD b % 8.  With tile_order 1, kernels
-// renumber workgroups so that each XCD's workgroups take one contiguous
-// eighth of the tiles, in order.
+// renumber workgroups so that each XCD takes runs of 128 waves' work (a run is
+// 512 KiB of pixels with one block per lane; xcd_workgroup in tile_io.h).
+// Runs of 64 to 512 waves measured alike on batches of 128 to 4096 textures;
+// one run per XCD (a contiguous eighth each) was 3-4% slower than them on 4096
+// textures and 12% on 512, whose XCDs then end at different times.
 constexpr uint32_t kXcdCount = 8;
+constexpr uint32_t kXcdRunTiles = 128;
+// The kernels' order argument: 0, or 1 + log2 of the run in workgroups.
+inline uint32_t order_arg(const LaunchCfg& c)
+{
+    return c.tile_order ? 1u + (uint32_t)__builtin_ctz(kXcdRunTiles / (uint32_t)c.wg_waves) : 0u;
+}
 
 inline LaunchCfg to_cfg(const goofy_launch_config& u)
 {
@@ -95,7 +104,8 @@ inline uint32_t max_stripe_brows(uint64_t bw)
 // Kernel launchers (kernels.hip).
 hipError_t launch_plain(int fmt, const LaunchCfg& cfg, const void* src, size_t pitch, void* dst, uint32_t bw,
                         uint32_t nblocks, hipStream_t stream, hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
-hipError_t launch_dual(uint32_t wg_waves, const void* src, size_t pitch, void* dst_dxt1, void* dst_etc1, uint32_t bw,
+// cfg: workgroup size and tile order (one block per lane, streaming).
+hipError_t launch_dual(const LaunchCfg& cfg, const void* src, size_t pitch, void* dst_dxt1, void* dst_etc1, uint32_t bw,
                        uint32_t nblocks, hipStream_t stream, hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 hipError_t launch_dual_alpha(uint32_t wg_waves, const void* src, size_t pitch, void* dst_dxt5, void* dst_etc2,
                              uint32_t bw, uint32_t nblocks, hipStream_t stream, hipEvent_t start = nullptr,
@@ -207,6 +217,34 @@ inline int tile_blocks(const LaunchCfg& c) { return 64 * c.blocks_per_lane; }
 // Default launch shape for a launch of `blocks` 4x4 blocks on a device with
 // num_cus compute units (used wherever the caller gives no shape).
 LaunchCfg auto_cfg(uint64_t blocks, int num_cus);
+// The default for a launch that reads large amounts of pixels and is bound by
+// that: batches, and images into the 8-byte formats.  Above 64 MiB of pixels
+// (16384 tiles) tiles go to the XCDs in runs, in workgroups of 4 waves, or 8
+// from 1 GiB on; smaller launches keep auto_cfg's shape.  Measured in us per
+// launch, linear order in 8-wave workgroups -> this: batches of 128 / 1024 /
+// 4096 textures 34.6 -> 32.6, 282 -> 262, 1090 -> 1006; DXT1 6000x4000
+// 18.9 -> 18.8, 8192^2 47.9 -> 46.9, 16384^2 189.5 -> 178.5 (its 65792-byte
+// pitch 195.9 -> 187.2), DXT1 + ETC1S 8192^2 54.7 -> 52.7; but 4096^2
+// 13.4 -> 13.8 and 2048^2 5.0 -> 5.4.  A 2048-texture batch of 660k tiles took
+// 478 us in 8-wave workgroups and 490 in 4-wave ones, an 8192^2 image 47.1 and
+// 46.9.
+inline LaunchCfg wide_cfg(uint64_t blocks, int num_cus)
+{
+    LaunchCfg c = auto_cfg(blocks, num_cus);
+    const uint64_t tiles = (blocks + 63u) / 64u;
+    if (tiles > 16384u) {
+        c.wg_waves = tiles < 262144u ? 4 : 8;
+        c.tile_order = 1;
+    }
+    return c;
+}
+// The default for one image of a format.  The 16-byte formats, half bound by
+// their arithmetic, gained up to 3% from runs at some sizes and lost 2% at
+// others: they stay linear.
+inline LaunchCfg plain_cfg(int format, uint64_t blocks, int num_cus)
+{
+    return format >= GOOFY_FORMAT_DXT5 ? auto_cfg(blocks, num_cus) : wide_cfg(blocks, num_cus);
+}
 bool cfg_valid(const LaunchCfg& c);
 
 }  // namespace goofy_impl

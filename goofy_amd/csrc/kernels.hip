@@ -155,12 +155,8 @@ __device__ __forceinline__ void encode_tile(const uint8_t* __restrict__ src, uin
     }
 }
 
-// Index of this wave in the launch.  With order 1 the workgroups are
-// renumbered so that those the dispatcher places on XCD x (b % 8 == x) take
-// the x-th contiguous share of the launch, in order: each XCD then streams
-// through one contiguous region instead of every eighth workgroup's tiles.
-// A bijection on [0, gridDim.x): r = n % 8 XCDs hold q + 1 workgroups, the
-// rest q.  All operands are wave-uniform (scalar unit).
+// Index of this wave in the launch, with the workgroups renumbered by `order`
+// (xcd_workgroup in tile_io.h).
 // wpg = waves per workgroup.  The batch kernels take it as an argument; the
 // others read blockDim.x, a 16-bit field of the dispatch packet, which this
 // target reads with a vector load at the head of every wave.  Measured both
@@ -170,13 +166,7 @@ __device__ __forceinline__ void encode_tile(const uint8_t* __restrict__ src, uin
 // 2-3% faster.
 __device__ __forceinline__ uint32_t wave_index(uint32_t order, uint32_t wpg)
 {
-    uint32_t b = blockIdx.x;
-    if (order) {
-        const uint32_t n = gridDim.x, q = n / kXcdCount, r = n % kXcdCount;
-        const uint32_t x = b % kXcdCount, k = b / kXcdCount;
-        b = x < r ? x * (q + 1u) + k : r * (q + 1u) + (x - r) * q + k;
-    }
-    return __builtin_amdgcn_readfirstlane(b * wpg + (threadIdx.x >> 6));
+    return __builtin_amdgcn_readfirstlane(xcd_workgroup(order) * wpg + (threadIdx.x >> 6));
 }
 
 __device__ __forceinline__ uint32_t wave_index(uint32_t order) { return wave_index(order, blockDim.x >> 6); }
@@ -197,9 +187,9 @@ __global__ __launch_bounds__(512) void k_encode_plain(const uint8_t* __restrict_
 // launches.  One block per lane, streaming loads and stores.
 __global__ __launch_bounds__(512) void k_encode_dual(const uint8_t* __restrict__ src, uint64_t pitch,
                                                      uint8_t* __restrict__ dst_dxt1, uint8_t* __restrict__ dst_etc1,
-                                                     uint32_t bw, uint32_t nblocks, uint64_t magic)
+                                                     uint32_t bw, uint32_t nblocks, uint64_t magic, uint32_t order)
 {
-    const uint32_t first = wave_index(0u) * 64u, lane = threadIdx.x & 63u;
+    const uint32_t first = wave_index(order) * 64u, lane = threadIdx.x & 63u;
     u32x4 v[1][4];
     load_tile<1, true>(src, pitch, bw, magic, nblocks, first, lane, v);
     if (first + lane >= nblocks) return;
@@ -333,7 +323,7 @@ static hipError_t plain_bpl(const LaunchCfg& c, dim3 grid, dim3 block, const voi
                             hipEvent_t e1)
 {
     const bool nt = c.nontemporal != 0;
-    const uint32_t o = (uint32_t)c.tile_order;
+    const uint32_t o = order_arg(c);
     switch (c.blocks_per_lane) {
     case 1:
         return nt ? plain_go<FMT, 1, true>(grid, block, src, pitch, dst, bw, nblocks, magic, o, s, e0, e1)
@@ -364,19 +354,19 @@ hipError_t launch_plain(int fmt, const LaunchCfg& c, const void* src, size_t pit
     }
 }
 
-hipError_t launch_dual(uint32_t wg_waves, const void* src, size_t pitch, void* dst_dxt1, void* dst_etc1, uint32_t bw,
+hipError_t launch_dual(const LaunchCfg& c, const void* src, size_t pitch, void* dst_dxt1, void* dst_etc1, uint32_t bw,
                        uint32_t nblocks, hipStream_t stream, hipEvent_t start, hipEvent_t stop)
 {
     if (nblocks == 0) return hipSuccess;
-    const uint32_t ntiles = (nblocks + 63u) / 64u;
-    const dim3 grid((ntiles + wg_waves - 1u) / wg_waves), block(64u * wg_waves);
+    const uint32_t ntiles = (nblocks + 63u) / 64u, wg = (uint32_t)c.wg_waves, order = order_arg(c);
+    const dim3 grid((ntiles + wg - 1u) / wg), block(64u * wg);
     const uint64_t magic = div_magic(bw);
     if (start || stop)
         hipExtLaunchKernelGGL(k_encode_dual, grid, block, 0, stream, start, stop, 0, (const uint8_t*)src,
-                              (uint64_t)pitch, (uint8_t*)dst_dxt1, (uint8_t*)dst_etc1, bw, nblocks, magic);
+                              (uint64_t)pitch, (uint8_t*)dst_dxt1, (uint8_t*)dst_etc1, bw, nblocks, magic, order);
     else
         hipLaunchKernelGGL(k_encode_dual, grid, block, 0, stream, (const uint8_t*)src, (uint64_t)pitch,
-                           (uint8_t*)dst_dxt1, (uint8_t*)dst_etc1, bw, nblocks, magic);
+                           (uint8_t*)dst_dxt1, (uint8_t*)dst_etc1, bw, nblocks, magic, order);
     return hipGetLastError();
 }
 
@@ -434,9 +424,9 @@ hipError_t launch_batch(const LaunchCfg& c, const TexDesc* d_descs, uint32_t nte
     const dim3 grid((uint32_t)((waves + wg - 1) / wg)), block(64u * wg);
     const bool nt = c.nontemporal;
     switch (c.blocks_per_lane) {
-    case 1: return batch_nt<1>(nt, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, c.tile_order, stream, done);
-    case 2: return batch_nt<2>(nt, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, c.tile_order, stream, done);
-    default: return batch_nt<4>(nt, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, c.tile_order, stream, done);
+    case 1: return batch_nt<1>(nt, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, order_arg(c), stream, done);
+    case 2: return batch_nt<2>(nt, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, order_arg(c), stream, done);
+    default: return batch_nt<4>(nt, alpha, grid, block, d_descs, tb, ntex, ntiles, tpw, order_arg(c), stream, done);
     }
 }
 
@@ -480,9 +470,9 @@ hipError_t launch_batch_inline(const LaunchCfg& c, const InlineWorklist& wl, uin
     const uint32_t wg = (uint32_t)c.wg_waves;
     const dim3 grid((uint32_t)((waves + wg - 1) / wg)), block(64u * wg);
     switch (c.blocks_per_lane) {
-    case 1: return batch_inline_nt<1>(c.nontemporal, alpha, grid, block, wl, ntex, ntiles, tpw, c.tile_order, stream);
-    case 2: return batch_inline_nt<2>(c.nontemporal, alpha, grid, block, wl, ntex, ntiles, tpw, c.tile_order, stream);
-    default: return batch_inline_nt<4>(c.nontemporal, alpha, grid, block, wl, ntex, ntiles, tpw, c.tile_order, stream);
+    case 1: return batch_inline_nt<1>(c.nontemporal, alpha, grid, block, wl, ntex, ntiles, tpw, order_arg(c), stream);
+    case 2: return batch_inline_nt<2>(c.nontemporal, alpha, grid, block, wl, ntex, ntiles, tpw, order_arg(c), stream);
+    default: return batch_inline_nt<4>(c.nontemporal, alpha, grid, block, wl, ntex, ntiles, tpw, order_arg(c), stream);
     }
 }
 

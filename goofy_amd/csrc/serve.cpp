@@ -238,7 +238,7 @@ bool goofy_server::launch_group(Slot& s, std::vector<Req>& group)
         if (auto_shape) {  // the shape follows the group's size
             uint64_t blocks = 0;
             for (const Req& q : group) blocks += (uint64_t)(q.r.width / 4) * (q.r.height / 4);
-            L = auto_cfg(blocks, num_cus);
+            L = wide_cfg(blocks, num_cus);
         }
         const uint64_t tile = (uint64_t)tile_blocks(L);
         uint32_t tiles = 0;
@@ -269,7 +269,7 @@ bool goofy_server::launch_group(Slot& s, std::vector<Req>& group)
     } else {
         for (Req& q : group) {
             const uint32_t bw = q.r.width / 4, nb = bw * (q.r.height / 4);
-            e = launch_plain(q.r.format, auto_shape ? auto_cfg(nb, num_cus) : launch, q.r.src, q.r.pitch,
+            e = launch_plain(q.r.format, auto_shape ? plain_cfg(q.r.format, nb, num_cus) : launch, q.r.src, q.r.pitch,
                              arena.base() + q.arena_off, bw, nb, s.stream);
             if (e != hipSuccess) break;
         }

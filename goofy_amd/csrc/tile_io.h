@@ -16,7 +16,30 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "internal.h"
+
 namespace goofy_impl {
+
+// This workgroup's place in the launch.  The dispatcher hands workgroup b to
+// XCD b % 8, so with order 0 each XCD works on every eighth workgroup's tiles.
+// With order = 1 + log2(run) the workgroups are renumbered in spans of 8 runs:
+// XCD x takes the x-th run of each span, `run` workgroups that follow one
+// another, so that neighbouring tiles (whose rows share 128-byte lines at
+// their ends) and pages meet in one XCD's L2 and TLB, while all XCDs move
+// through the launch together.  The last, incomplete span keeps its order.  A
+// bijection on [0, gridDim.x); all operands are wave-uniform (scalar unit).
+__device__ __forceinline__ uint32_t xcd_workgroup(uint32_t order)
+{
+    uint32_t b = blockIdx.x;
+    if (order) {
+        const uint32_t lg = order - 1u, span = kXcdCount << lg;
+        if (b < (gridDim.x & ~(span - 1u))) {
+            const uint32_t x = b % kXcdCount, k = b / kXcdCount;  // the k-th workgroup of XCD x
+            b = (((k >> lg) * kXcdCount + x) << lg) + (k & ((1u << lg) - 1u));
+        }
+    }
+    return b;
+}
 
 // Buffer resource over `base` (raw: no stride, no swizzle; dword 3 as for
 // every gfx9 raw buffer).  Wave-uniform: it lives in four scalar registers.

@@ -121,16 +121,17 @@ typedef struct goofy_launch_config {
     int wg_waves;        /* waves per workgroup: 1, 2, 4 or 8 */
     int waves_per_cu;    /* persistent grid: waves per CU (0 = one wave per tile) */
     int nontemporal;     /* 1 = streaming loads/stores */
-    int tile_order;      /* 0 = linear wave->tile order; 1 = XCD-contiguous: the
+    int tile_order;      /* 0 = linear wave->tile order; 1 = by XCD: the
                             workgroups the dispatcher places on each of the 8
-                            XCDs (workgroup b on XCD b % 8) take one contiguous
-                            eighth of the tiles */
+                            XCDs (workgroup b on XCD b % 8) take contiguous
+                            runs of 128 waves' tiles, run by run in turn */
 } goofy_launch_config;
 
 /* As goofy_hip_compress_device with an explicit launch shape.  NULL = the
  * default shape, sized to the launch: one block per lane, streaming loads and
  * stores, linear tile order, and the largest workgroup of 8, 4, 2 or 1 waves
- * that still gives at least two workgroups per CU. */
+ * that still gives at least two workgroups per CU; for DXT1 and ETC1S above 64
+ * MiB of pixels tile order 1, in workgroups of 4 waves, or 8 from 1 GiB on. */
 GOOFY_HIP_API int goofy_hip_compress_device_cfg(int format, void* d_result, const void* d_input, unsigned int width,
                                                 unsigned int height, size_t pitch, void* stream,
                                                 const goofy_launch_config* cfg);

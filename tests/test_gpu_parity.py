@@ -336,6 +336,45 @@ def test_launch_configs_vs_oracle(gpu, oracle, bpl, wg, nt, order):
         assert np.array_equal(encode_dev(gpu, fmt, src, w, h, pitch, cfg), oracle.compress_blocks(fmt, img, w, h, pitch))
 
 
+@pytest.mark.parametrize("w,h", [(4096, 4096), (4096, 4100), (4100, 4100), (2052, 8500), (260, 65532)])
+def test_runs_per_xcd_match_linear_order(gpu, w, h):
+    """From 16384 tiles of 64 blocks on the default shape takes tiles in runs
+    per XCD: sizes at and above that limit, with a last span of workgroups
+    that is incomplete, and explicit shapes of every workgroup size, against
+    the linear order (which the other tests hold against the oracle)."""
+    from goofy_amd import hip
+    say(f"runs per XCD {w}x{h}: {(w // 4) * (h // 4) / 64:.1f} tiles")
+    src = dev_buffer(w * h * 4)
+    gpu.synth_device(1, 77, 0, 12, src, w, h)
+    n = (w // 4) * (h // 4) * 8
+    a, b = dev_buffer(n), dev_buffer(n)
+    linear = dict(blocks_per_lane=1, wg_waves=8, waves_per_cu=0, nontemporal=1, tile_order=0)
+    want = []
+    for fmt in (W.DXT1, W.ETC1):
+        gpu.compress_device(fmt, a, src, w, h, w * 4, config=linear)
+        hip.synchronize()
+        want.append(a.download())
+        for cfg in [None] + [dict(linear, wg_waves=wg, tile_order=1) for wg in (1, 2, 4, 8)]:
+            a.fill(0xCD)
+            gpu.compress_device(fmt, a, src, w, h, w * 4, config=cfg)
+            hip.synchronize()
+            assert np.array_equal(a.download(), want[fmt]), (fmt, cfg)
+    a.fill(0xCD)
+    b.fill(0xCD)
+    gpu.compress_device_dual(a, b, src, w, h, w * 4)
+    hip.synchronize()
+    assert np.array_equal(a.download(), want[0]) and np.array_equal(b.download(), want[1])
+    plan = gpu.Batch([dict(src=src, dst=d, width=w, height=h, format=f) for f, d in ((W.DXT1, a), (W.ETC1, b))])
+    for cfg in [None] + [dict(linear, wg_waves=wg, tile_order=1, waves_per_cu=p) for wg, p in ((1, 0), (8, 0), (4, 40))]:
+        a.fill(0xCD)
+        b.fill(0xCD)
+        if cfg:
+            plan.config = cfg
+        plan.launch()
+        hip.synchronize()
+        assert np.array_equal(a.download(), want[0]) and np.array_equal(b.download(), want[1]), cfg
+
+
 def test_tune_device_picks_a_valid_shape(gpu, oracle):
     w, h, pitch = 2048, 1024, 2048 * 4 + 256
     img = gpu.synth_host(0, 99, 0, 12, w, h, pitch, fill=0)
