@@ -8,6 +8,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <condition_variable>
 #include <cstring>
 #include <deque>
@@ -113,13 +114,25 @@ bool cfg_valid(const LaunchCfg& c)
 // upload stream never waits on the device.  (On a single stream each upload
 // is ordered behind the previous chunk's kernel and download; on MI355X the
 // 8192^2 call took 6.6 ms that way and 5.5 ms with the uploads apart, at the
-// link's measured host-to-device ceiling.)  A one-chunk image stays on one
-// stream.  Row copies of large chunks are split over a small persistent thread
-// pool.  Contexts (stream, events, device and pinned buffers) come from a
-// process-wide pool: concurrent callers never share one, and nothing is freed
-// at thread exit (the HIP runtime may already be gone then).
+// link's measured host-to-device ceiling.)  Row copies of large chunks are
+// split over a small persistent thread pool.  An image of one chunk goes
+// through a fed kernel instead (encode_one_chunk).  Contexts (stream, events, device
+// and pinned buffers) come from a process-wide pool: concurrent callers never
+// share one, and nothing is freed at thread exit (the HIP runtime may already
+// be gone then).
 
 constexpr int kSlots = 3;
+constexpr uint64_t kFeedPatience = 2000000;  // 20 ms in 10 ns ticks
+
+// Whether a launch returns only when its kernel has ended.
+static bool launches_block()
+{
+    for (const char* name : {"HIP_LAUNCH_BLOCKING", "AMD_SERIALIZE_KERNEL"}) {
+        const char* v = std::getenv(name);
+        if (v && *v && std::strcmp(v, "0") != 0) return true;
+    }
+    return false;
+}
 
 struct StagingCtx {
     int device = -1;
@@ -132,6 +145,9 @@ struct StagingCtx {
     void* h_in[kSlots] = {};
     void* h_out[kSlots] = {};
     size_t in_cap = 0, out_cap = 0;
+    HostFeed* feed = nullptr;     // fed kernels: the marks of the parts,
+    uint64_t call = 0;            // the number of the last launch
+    bool stage_first = launches_block();
 };
 
 class StagingPool {
@@ -179,6 +195,11 @@ static int ensure_ctx(StagingCtx* c, size_t in_bytes, size_t out_bytes)
                 return fail_hip(e, "hipEventCreate");
         }
     }
+    if (!c->feed) {
+        if ((e = hipHostMalloc((void**)&c->feed, sizeof(HostFeed), hipHostMallocCoherent)) != hipSuccess)
+            return fail_hip(e, "hipHostMalloc(staging)");
+        *c->feed = HostFeed{};
+    }
     if (c->in_cap < in_bytes || c->out_cap < out_bytes) {
         (void)hipStreamSynchronize(c->in_stream);
         (void)hipStreamSynchronize(c->stream);
@@ -194,8 +215,9 @@ static int ensure_ctx(StagingCtx* c, size_t in_bytes, size_t out_bytes)
         for (int i = 0; i < kSlots; ++i) {
             if ((e = hipMalloc(&c->d_in[i], ni)) != hipSuccess || (e = hipMalloc(&c->d_out[i], no)) != hipSuccess)
                 return fail_hip(e, "hipMalloc(staging)");
-            if ((e = hipHostMalloc(&c->h_in[i], ni, hipHostMallocDefault)) != hipSuccess ||
-                (e = hipHostMalloc(&c->h_out[i], no, hipHostMallocDefault)) != hipSuccess)
+            // coherent: a fed kernel reads rows that are written while it runs
+            if ((e = hipHostMalloc(&c->h_in[i], ni, hipHostMallocCoherent)) != hipSuccess ||
+                (e = hipHostMalloc(&c->h_out[i], no, hipHostMallocCoherent)) != hipSuccess)
                 return fail_hip(e, "hipHostMalloc(staging)");
         }
         c->in_cap = ni;
@@ -225,18 +247,91 @@ static void copy_rows(uint8_t* dst, const uint8_t* src, size_t stride, size_t ro
     });
 }
 
-// fmt: one format into `result`, or kHostDual: DXT1 into `result` and ETC1S
-// into `result2` from one pass over the image, or kHostDualAlpha: DXT5 and
-// ETC2 RGBA8 the same way.
-constexpr int kHostDual = 1 << 16;
-constexpr int kHostDualAlpha = (1 << 16) + 1;
+// Marks every part of a launched image on the way out: all are marked already
+// unless the staging was left by an exception.
+struct FeedGuard {
+    HostFeed* feed;
+    uint64_t call;
+    unsigned parts;
+    void mark(unsigned p) const { __atomic_store_n(&feed->part[p].staged, call, __ATOMIC_RELEASE); }
+    ~FeedGuard()
+    {
+        for (unsigned p = 0; p < parts; ++p) mark(p);
+    }
+};
 
+// One launch of a format or pair over an image, or chunk of one, whose rows
+// are row_bytes apart: blocks to `out`, a pair's second format to `out2`.
+static hipError_t launch_any(int fmt, const LaunchCfg& cfg, const void* in, size_t row_bytes, void* out, void* out2,
+                             uint32_t bw, uint32_t nblocks, hipStream_t stream)
+{
+    return fmt == kFeedDualAlpha
+               ? launch_dual_alpha((uint32_t)cfg.wg_waves, in, row_bytes, out, out2, bw, nblocks, stream)
+           : fmt == kFeedDual ? launch_dual(cfg, in, row_bytes, out, out2, bw, nblocks, stream)
+                              : launch_plain(fmt, cfg, in, row_bytes, out, bw, nblocks, stream);
+}
+
+// Encodes an image of one chunk (up to about 8 MiB) into ctx->h_out[0].  The
+// kernel reads the pinned staging copy over PCIe and writes its blocks to
+// pinned memory over PCIe: the copy engines' set-up and synchronisation weigh
+// more than the copy (512x512: 82 us through them).
+//   From 128 KiB on a fed kernel (k_encode_fed) is launched before anything is
+// staged and reads the parts while the host still writes the next ones, so the
+// launch and the copy are hidden behind the link: 512x512 43.7 us, 1024x1024
+// 116 us, against 55 and 146 us with one launch per 512 KiB staged.  Below
+// that the kernel's look at the mark, over PCIe, costs more than it hides
+// (64x64: 19.4 against 17.0 us): staged first, one plain launch.  Images of
+// more chunks keep the DMA pipeline, which reaches 52-56 GB/s on their chunks,
+// kernels 49.
+//   Between the fed launch and the mark of the last part the host calls
+// nothing that could wait for the device, so the kernel's wait ends whatever
+// other threads and streams do.  Should this thread stand still for `patience`
+// ticks the kernel ends unfinished, and the image, by then all staged, is
+// encoded by a plain launch.  Where a launch returns only after its kernel the
+// image is staged first, too.
+static hipError_t encode_one_chunk(StagingCtx* ctx, int fmt, const LaunchCfg& cfg, const uint8_t* input,
+                                   unsigned stride, uint32_t bw, uint32_t bh, size_t out_bytes, uint64_t patience)
+{
+    const size_t row_bytes = (size_t)bw * 16, bytes = row_bytes * 4 * bh;
+    uint8_t* const in = static_cast<uint8_t*>(ctx->h_in[0]);
+    uint8_t* const out = static_cast<uint8_t*>(ctx->h_out[0]);
+    const auto plain = [&]() -> hipError_t {
+        const hipError_t e = launch_any(fmt, cfg, in, row_bytes, out, out + out_bytes, bw, bw * bh, ctx->stream);
+        return e == hipSuccess ? hipStreamSynchronize(ctx->stream) : e;
+    };
+    if (bytes < (128u << 10) || ctx->stage_first) {
+        copy_rows(in, input, stride, row_bytes, bh * 4);
+        return plain();
+    }
+    // parts of whole block rows, about 64 KiB or a thirty-second of the image
+    const unsigned want = (unsigned)std::min<size_t>(kFeedParts, bytes >> 16);
+    const unsigned prows = (bh + want - 1) / want, parts = (bh + prows - 1) / prows;
+    const uint64_t call = ++ctx->call;
+    hipError_t e = launch_fed(fmt, in, row_bytes, out, out + out_bytes, bw, bw * bh, ctx->feed, call, bw * prows,
+                              patience, ctx->stream);
+    if (e != hipSuccess) return e;
+    {
+        const FeedGuard guard{ctx->feed, call, parts};
+        for (unsigned p = 0; p < parts; ++p) {
+            const size_t r0 = (size_t)p * prows, rows = std::min<size_t>(prows, bh - r0);
+            copy_rows(in + r0 * 4 * row_bytes, input + r0 * 4 * stride, stride, row_bytes, (unsigned)rows * 4);
+            guard.mark(p);
+        }
+    }
+    if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return e;
+    return ctx->feed->gave_up == call ? plain() : hipSuccess;
+}
+
+// fmt: one format into `result`, or kFeedDual: DXT1 into `result` and ETC1S
+// into `result2` from one pass over the image, or kFeedDualAlpha: DXT5 and
+// ETC2 RGBA8 the same way.
 static int compress_host(int fmt, unsigned char* result, const unsigned char* input, unsigned width,
-                         unsigned height, unsigned stride, unsigned char* result2 = nullptr)
+                         unsigned height, unsigned stride, unsigned char* result2 = nullptr,
+                         uint64_t patience = kFeedPatience)
 {
     clear_error();
-    const bool dual_alpha = fmt == kHostDualAlpha;
-    const bool dual = fmt == kHostDual || dual_alpha;
+    const bool dual_alpha = fmt == kFeedDualAlpha;
+    const bool dual = fmt == kFeedDual || dual_alpha;
     if (!format_valid(fmt) && !dual) return fail(GOOFY_ERR_INVALID, "unknown format");
     // Same checks, same order as the reference (GoofyTC/goofy_tc.h:1500-1508).
     if (width % 16 != 0) return fail(GOOFY_ERR_WIDTH, "width must be a multiple of 16");
@@ -269,60 +364,31 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
     const LaunchCfg cfg = auto_cfg((uint64_t)bw * cb, di.num_cus);
     hipError_t e = hipSuccess;
 
-    auto finish_chunk = [&](unsigned k) -> hipError_t {
+    // Copies chunk k's blocks from its slot to the caller.
+    auto collect = [&](unsigned k) {
         const int s = (int)(k % kSlots);
-        const unsigned rows = std::min(cb, bh - k * cb);
-        hipError_t r = hipEventSynchronize(ctx->out_ready[s]);
-        if (r != hipSuccess) return r;
-        const size_t n = (size_t)rows * bw * bb;
+        const size_t n = (size_t)std::min(cb, bh - k * cb) * bw * bb;
         std::memcpy(result + (size_t)k * cb * bw * bb, ctx->h_out[s], n);
         if (dual) std::memcpy(result2 + (size_t)k * cb * bw * bb, static_cast<uint8_t*>(ctx->h_out[s]) + n, n);
-        return hipSuccess;
+    };
+    if (nchunks == 1) {
+        if ((e = encode_one_chunk(ctx, fmt, cfg, input, stride, bw, bh, (size_t)bw * bh * bb, patience)) != hipSuccess) {
+            (void)hipStreamSynchronize(ctx->stream);
+            return fail_hip(e, "drop-in one-chunk launch");
+        }
+        collect(0);
+        return GOOFY_OK;
+    }
+    auto finish_chunk = [&](unsigned k) -> hipError_t {
+        hipError_t r = hipEventSynchronize(ctx->out_ready[k % kSlots]);
+        if (r == hipSuccess) collect(k);
+        return r;
     };
 
     // Chunk k uses slot k % kSlots.  Chunk k-kSlots, the slot's previous user,
     // was collected by finish_chunk in an earlier iteration, so its upload,
     // kernel and download are complete and the slot is free on both sides.
-    // An image of one chunk (up to about 8 MiB) is not copied to the device:
-    // the kernels read the pinned staging copy and write the pinned output
-    // over PCIe themselves (zero-copy), which saves the two DMA transfers'
-    // set-up and synchronisation -- at 512x512, 66 against 82 us.
-    const bool two_streams = nchunks > 1;
-    const bool zero_copy = nchunks == 1;
-    if (zero_copy) {
-        // The host stages the image in up to 8 parts of at least 512 KiB, and
-        // each part's kernel is launched as soon as its rows are staged: the
-        // GPU reads part p over PCIe while the host copies part p+1.  One
-        // stream, one synchronisation (finish_chunk).  At 512x512, 2 parts took
-        // 0.052-0.054 ms, 4 parts of 256 KiB 0.054-0.055 and 8 parts 0.064-0.066
-        // (each launch costs the host a few microseconds); at 1024x1024, 8
-        // parts took 0.145 ms against 0.151 for 4.  The kernels read PCIe at
-        // about 35 GB/s against the copy engines' 41-55, so larger images keep
-        // the DMA pipeline (at 2896x2896 zero-copy took 1.01 ms against 0.81).
-        uint8_t* const hin = static_cast<uint8_t*>(ctx->h_in[0]);
-        uint8_t* const hout = static_cast<uint8_t*>(ctx->h_out[0]);
-        const size_t n = (size_t)bw * bh * bb;  // bytes of one format's blocks
-        const unsigned parts = (unsigned)std::min<size_t>(8, std::max<size_t>(1, (row_bytes * 4 * bh) >> 19));
-        const unsigned prows = (bh + parts - 1) / parts;
-        for (unsigned r0 = 0; r0 < bh && e == hipSuccess; r0 += prows) {
-            const unsigned rows = std::min(prows, bh - r0);
-            uint8_t* const in = hin + (size_t)r0 * 4 * row_bytes;
-            uint8_t* const out = hout + (size_t)r0 * bw * bb;
-            copy_rows(in, input + (size_t)r0 * 4 * stride, stride, row_bytes, rows * 4);
-            e = dual_alpha ? launch_dual_alpha((uint32_t)cfg.wg_waves, in, row_bytes, out, out + n, bw, bw * rows,
-                                               ctx->stream)
-                : dual     ? launch_dual(cfg, in, row_bytes, out, out + n, bw, bw * rows, ctx->stream)
-                           : launch_plain(fmt, cfg, in, row_bytes, out, bw, bw * rows, ctx->stream);
-        }
-        if (e == hipSuccess) e = hipEventRecord(ctx->out_ready[0], ctx->stream);
-        if (e == hipSuccess) e = finish_chunk(0);
-        if (e != hipSuccess) {
-            (void)hipStreamSynchronize(ctx->stream);
-            return fail_hip(e, "drop-in zero-copy launch");
-        }
-        return GOOFY_OK;
-    }
-    hipStream_t up = two_streams ? ctx->in_stream : ctx->stream;
+    const hipStream_t up = ctx->in_stream;
     unsigned collected = 0;  // chunks [0, collected) are in `result`
     for (unsigned k = 0; k < nchunks && e == hipSuccess; ++k) {
         const int s = (int)(k % kSlots);
@@ -334,16 +400,11 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
         if ((e = hipMemcpyAsync(ctx->d_in[s], ctx->h_in[s], row_bytes * 4 * rows, hipMemcpyHostToDevice, up)) !=
             hipSuccess)
             break;
-        if (two_streams) {
-            if ((e = hipEventRecord(ctx->h2d_done[s], up)) != hipSuccess) break;
-            if ((e = hipStreamWaitEvent(ctx->stream, ctx->h2d_done[s], 0)) != hipSuccess) break;
-        }
+        if ((e = hipEventRecord(ctx->h2d_done[s], up)) != hipSuccess) break;
+        if ((e = hipStreamWaitEvent(ctx->stream, ctx->h2d_done[s], 0)) != hipSuccess) break;
         const size_t n = (size_t)bw * rows * bb;
         uint8_t* second = static_cast<uint8_t*>(kout) + n;
-        e = dual_alpha ? launch_dual_alpha((uint32_t)cfg.wg_waves, kin, row_bytes, kout, second, bw, bw * rows,
-                                           ctx->stream)
-            : dual     ? launch_dual(cfg, kin, row_bytes, kout, second, bw, bw * rows, ctx->stream)
-                       : launch_plain(fmt, cfg, kin, row_bytes, kout, bw, bw * rows, ctx->stream);
+        e = launch_any(fmt, cfg, kin, row_bytes, kout, second, bw, bw * rows, ctx->stream);
         if (e != hipSuccess) break;
         if ((e = hipMemcpyAsync(ctx->h_out[s], ctx->d_out[s], outs * n, hipMemcpyDeviceToHost, ctx->stream)) !=
             hipSuccess)
@@ -451,6 +512,15 @@ int goofy_hip_compress(int format, unsigned char* result, const unsigned char* i
     return compress_host(format, result, input, width, height, stride);
 }
 
+// goofy_hip_compress with another limit for a fed kernel's wait (10 ns ticks):
+// for the test of a host that stages too late.
+GOOFY_HIP_API int goofy_impl_compress_with_patience(int format, unsigned char* result, const unsigned char* input,
+                                                    unsigned int width, unsigned int height, unsigned int stride,
+                                                    uint64_t patience)
+{
+    return compress_host(format, result, input, width, height, stride, nullptr, patience);
+}
+
 int goofy_hip_compress_dxt1(unsigned char* result, const unsigned char* input, unsigned int width, unsigned int height,
                             unsigned int stride)
 {
@@ -499,7 +569,7 @@ int goofy_hip_compress_device_timed(int format, void* d_result, const void* d_in
 int goofy_hip_compress_dual(unsigned char* result_dxt1, unsigned char* result_etc1, const unsigned char* input,
                             unsigned int width, unsigned int height, unsigned int stride)
 {
-    return compress_host(kHostDual, result_dxt1, input, width, height, stride, result_etc1);
+    return compress_host(kFeedDual, result_dxt1, input, width, height, stride, result_etc1);
 }
 
 static int compress_device_pair(bool alpha, void* d_a, void* d_b, const void* d_input, unsigned int width,
@@ -559,7 +629,7 @@ int goofy_hip_compress_device_dual_alpha(void* d_dxt5, void* d_etc2, const void*
 int goofy_hip_compress_dual_alpha(unsigned char* result_dxt5, unsigned char* result_etc2, const unsigned char* input,
                                   unsigned int width, unsigned int height, unsigned int stride)
 {
-    return compress_host(kHostDualAlpha, result_dxt5, input, width, height, stride, result_etc2);
+    return compress_host(kFeedDualAlpha, result_dxt5, input, width, height, stride, result_etc2);
 }
 
 int goofy_hip_tune_device(int format, void* d_result, const void* d_input, unsigned int width, unsigned int height,

@@ -110,6 +110,25 @@ hipError_t launch_dual(const LaunchCfg& cfg, const void* src, size_t pitch, void
 hipError_t launch_dual_alpha(uint32_t wg_waves, const void* src, size_t pitch, void* dst_dxt5, void* dst_etc2,
                              uint32_t bw, uint32_t nblocks, hipStream_t stream, hipEvent_t start = nullptr,
                              hipEvent_t stop = nullptr);
+// The drop-in's kernel, which encodes an image in pinned host memory while
+// the host is still staging it there.  HostFeed (pinned, coherent): the word
+// of a part holds the number of the call whose rows are staged in it, written
+// after them; gave_up the number of a call whose kernel stopped waiting.
+constexpr uint32_t kFeedParts = 32;
+constexpr uint32_t kFeedGroups = 64;
+struct HostFeed {
+    struct alignas(64) Part {
+        uint64_t staged;
+    } part[kFeedParts];
+    alignas(64) uint64_t gave_up;
+};
+// Pseudo-formats: both 8-byte formats / both 16-byte formats, the second into
+// dst2.
+constexpr int kFeedDual = 1 << 16, kFeedDualAlpha = (1 << 16) + 1;
+// part_blocks: blocks per part (at most kFeedParts parts); call: a number that
+// no word holds yet; patience: how long a wait may last, in 10 ns ticks.
+hipError_t launch_fed(int fmt, const void* src, size_t pitch, void* dst, void* dst2, uint32_t bw, uint32_t nblocks,
+                      HostFeed* feed, uint64_t call, uint32_t part_blocks, uint64_t patience, hipStream_t stream);
 // alpha: the work-list holds DXT5 / ETC2 RGBA8 textures too (the kernel
 // instance with all four formats; without, DXT1 / ETC1S only).
 hipError_t launch_batch(const LaunchCfg& cfg, const TexDesc* d_descs, uint32_t ntex, uint32_t ntiles, int num_cus,

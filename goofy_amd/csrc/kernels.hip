@@ -181,46 +181,109 @@ __global__ __launch_bounds__(512) void k_encode_plain(const uint8_t* __restrict_
     encode_tile<FMT, BPL, NT>(src, pitch, dst, bw, magic, nblocks, wave * 64u * BPL, threadIdx.x & 63u);
 }
 
-// One image into both formats: each block is loaded and classified once
-// (bounding box, luma, range, thresholds, per-pixel masks) and packed as DXT1
-// and as ETC1S.  72 -> 80 bytes per block instead of 2 x 72 for two plain
-// launches.  One block per lane, streaming loads and stores.
-__global__ __launch_bounds__(512) void k_encode_dual(const uint8_t* __restrict__ src, uint64_t pitch,
-                                                     uint8_t* __restrict__ dst_dxt1, uint8_t* __restrict__ dst_etc1,
-                                                     uint32_t bw, uint32_t nblocks, uint64_t magic, uint32_t order)
+// A tile of 64 blocks into both formats: each block is loaded and classified
+// once (bounding box, luma, range, thresholds, per-pixel masks) and packed as
+// DXT1 and as ETC1S, 72 -> 80 bytes per block instead of 2 x 72 for two plain
+// launches.  With ALPHA into DXT5 and ETC2 RGBA8: the colour classification
+// and the alpha rows are computed once for both, 64 + 16 + 16 = 96 bytes per
+// block instead of 2 x 80.  Streaming loads and stores.
+template <bool ALPHA>
+__device__ __forceinline__ void encode_pair_tile(const uint8_t* __restrict__ src, uint64_t pitch,
+                                                 uint8_t* __restrict__ dst_a, uint8_t* __restrict__ dst_b, uint32_t bw,
+                                                 uint32_t nblocks, uint64_t magic, uint32_t first, uint32_t lane)
 {
-    const uint32_t first = wave_index(order) * 64u, lane = threadIdx.x & 63u;
     u32x4 v[1][4];
     load_tile<1, true>(src, pitch, bw, magic, nblocks, first, lane, v);
     if (first + lane >= nblocks) return;
     uint32_t p[16];
     block_words(v[0], p);
-    const BlockClass c = classify(p);
-    store8_at<true>(raw_rsrc(dst_dxt1 + (uint64_t)first * 8u), lane * 8u, pack_dxt1(c));
-    store8_at<true>(raw_rsrc(dst_etc1 + (uint64_t)first * 8u), lane * 8u, pack_etc1(p, c));
+    if constexpr (ALPHA) {
+        uint32_t amn, amx;
+        const BlockClass c = classify(p, goofy_dev::block_stats_alpha(p, amn, amx));
+        const AlphaRows a = alpha_rows(p, amn, amx);
+        const uint2 d = pack_dxt1(c), ba = bc3_alpha(a);
+        store16_at<true>(raw_rsrc(dst_a + (uint64_t)first * 16u), lane * 16u, make_uint4(ba.x, ba.y, d.x, d.y));
+        const uint2 e = pack_etc1(p, c), ea = eac_alpha(a);
+        store16_at<true>(raw_rsrc(dst_b + (uint64_t)first * 16u), lane * 16u, make_uint4(ea.x, ea.y, e.x, e.y));
+    } else {
+        const BlockClass c = classify(p);
+        store8_at<true>(raw_rsrc(dst_a + (uint64_t)first * 8u), lane * 8u, pack_dxt1(c));
+        store8_at<true>(raw_rsrc(dst_b + (uint64_t)first * 8u), lane * 8u, pack_etc1(p, c));
+    }
 }
 
-// One image into DXT5 and ETC2 RGBA8: each block is loaded once, and the
-// colour classification and the alpha rows are computed once for both.
-// 64 + 16 + 16 = 96 bytes per block instead of 2 x 80 for two plain launches.
+// One image into both 8-byte formats, one block per lane.
+__global__ __launch_bounds__(512) void k_encode_dual(const uint8_t* __restrict__ src, uint64_t pitch,
+                                                     uint8_t* __restrict__ dst_dxt1, uint8_t* __restrict__ dst_etc1,
+                                                     uint32_t bw, uint32_t nblocks, uint64_t magic, uint32_t order)
+{
+    encode_pair_tile<false>(src, pitch, dst_dxt1, dst_etc1, bw, nblocks, magic, wave_index(order) * 64u,
+                            threadIdx.x & 63u);
+}
+
+// One image into both 16-byte formats.
 __global__ __launch_bounds__(512) void k_encode_dual_alpha(const uint8_t* __restrict__ src, uint64_t pitch,
                                                            uint8_t* __restrict__ dst_dxt5,
                                                            uint8_t* __restrict__ dst_etc2, uint32_t bw,
                                                            uint32_t nblocks, uint64_t magic)
 {
-    const uint32_t first = wave_index(0u) * 64u, lane = threadIdx.x & 63u;
-    u32x4 v[1][4];
-    load_tile<1, true>(src, pitch, bw, magic, nblocks, first, lane, v);
-    if (first + lane >= nblocks) return;
-    uint32_t p[16];
-    block_words(v[0], p);
-    uint32_t amn, amx;
-    const BlockClass c = classify(p, goofy_dev::block_stats_alpha(p, amn, amx));
-    const AlphaRows a = alpha_rows(p, amn, amx);
-    const uint2 d = pack_dxt1(c), ba = bc3_alpha(a);
-    store16_at<true>(raw_rsrc(dst_dxt5 + (uint64_t)first * 16u), lane * 16u, make_uint4(ba.x, ba.y, d.x, d.y));
-    const uint2 e = pack_etc1(p, c), ea = eac_alpha(a);
-    store16_at<true>(raw_rsrc(dst_etc2 + (uint64_t)first * 16u), lane * 16u, make_uint4(ea.x, ea.y, e.x, e.y));
+    encode_pair_tile<true>(src, pitch, dst_dxt5, dst_etc2, bw, nblocks, magic, wave_index(0u) * 64u,
+                           threadIdx.x & 63u);
+}
+
+// Waits until part p of the image is staged (HostFeed): one lane reads the
+// part's word in host memory, about every 2 us.  The host stages every part of
+// a kernel it has launched without any call in between that could wait for
+// the device, so the wait ends; should the host thread not run for `patience`
+// ticks of the 100 MHz clock, the wait ends all the same, and says so.
+__device__ __forceinline__ bool await_part(HostFeed* feed, uint32_t p, uint64_t call, uint64_t patience)
+{
+    const uint64_t t0 = wall_clock64();
+    while (__hip_atomic_load(&feed->part[p].staged, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != call) {
+        if (wall_clock64() - t0 > patience) {
+            __hip_atomic_store(&feed->gave_up, call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            return false;
+        }
+        __builtin_amdgcn_s_sleep(8);
+    }
+    return true;
+}
+
+// One image (or chunk of one) in pinned host memory, encoded over PCIe while
+// the host is still staging it: launched first, it takes each group of 512
+// blocks as soon as the parts it lies in are staged.  FMT: a format, or
+// kFeedDual / kFeedDualAlpha into dst and dst2.  part_blocks: blocks per part.
+// A grid of at most kFeedGroups workgroups steps through the groups in order:
+// PCIe needs few loads in flight, and every waiting workgroup polls over the
+// same link.
+template <int FMT>
+__global__ __launch_bounds__(512) void k_encode_fed(const uint8_t* src, uint64_t pitch, uint8_t* dst, uint8_t* dst2,
+                                                    uint32_t bw, uint32_t nblocks, uint64_t magic, HostFeed* feed,
+                                                    uint64_t call, uint32_t part_blocks, uint64_t patience)
+{
+    __shared__ uint32_t staged;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (uint32_t group = blockIdx.x; (uint64_t)group * 512u < nblocks; group += gridDim.x) {
+        const uint32_t first = group * 512u;
+        if (threadIdx.x == 0) {
+            const uint32_t end = (min(first + 511u, nblocks - 1u)) / part_blocks;
+            bool ok = true;
+            for (uint32_t p = first / part_blocks; ok && p <= end; ++p) ok = await_part(feed, p, call, patience);
+            staged = ok ? 1u : 0u;
+        }
+        __syncthreads();
+        const bool ok = staged != 0u;
+        __syncthreads();  // the word is free for the next group
+        if (!ok) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");  // the rows, after the words (system scope)
+        const uint32_t tile = first + wave * 64u;
+        if (tile >= nblocks) continue;
+        if constexpr (FMT == kFeedDual) encode_pair_tile<false>(src, pitch, dst, dst2, bw, nblocks, magic, tile, lane);
+        else if constexpr (FMT == kFeedDualAlpha)
+            encode_pair_tile<true>(src, pitch, dst, dst2, bw, nblocks, magic, tile, lane);
+        else encode_tile<FMT, 1, true>(src, pitch, dst, bw, magic, nblocks, tile, lane);
+    }
 }
 
 // Many textures.  tile_begin[0..ntex] is the prefix sum of the textures'
@@ -352,6 +415,26 @@ hipError_t launch_plain(int fmt, const LaunchCfg& c, const void* src, size_t pit
     case GOOFY_FORMAT_DXT5: return plain_bpl<2>(c, grid, block, src, pitch, dst, bw, nblocks, magic, stream, start, stop);
     default: return plain_bpl<3>(c, grid, block, src, pitch, dst, bw, nblocks, magic, stream, start, stop);
     }
+}
+
+hipError_t launch_fed(int fmt, const void* src, size_t pitch, void* dst, void* dst2, uint32_t bw, uint32_t nblocks,
+                      HostFeed* feed, uint64_t call, uint32_t part_blocks, uint64_t patience, hipStream_t stream)
+{
+    if (nblocks == 0 || part_blocks == 0 || (nblocks - 1u) / part_blocks >= kFeedParts) return hipErrorInvalidValue;
+    const dim3 grid(std::min((nblocks + 511u) / 512u, kFeedGroups)), block(512);
+    const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, (const uint8_t*)src, (uint64_t)pitch, (uint8_t*)dst,
+                           (uint8_t*)dst2, bw, nblocks, div_magic(bw), feed, call, part_blocks, patience);
+    };
+    switch (fmt) {
+    case GOOFY_FORMAT_DXT1: go(k_encode_fed<0>); break;
+    case GOOFY_FORMAT_ETC1: go(k_encode_fed<1>); break;
+    case GOOFY_FORMAT_DXT5: go(k_encode_fed<2>); break;
+    case GOOFY_FORMAT_ETC2: go(k_encode_fed<3>); break;
+    case kFeedDual: go(k_encode_fed<kFeedDual>); break;
+    default: go(k_encode_fed<kFeedDualAlpha>);
+    }
+    return hipGetLastError();
 }
 
 hipError_t launch_dual(const LaunchCfg& c, const void* src, size_t pitch, void* dst_dxt1, void* dst_etc1, uint32_t bw,

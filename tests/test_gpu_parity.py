@@ -760,6 +760,35 @@ def test_dropin_zero_copy_parts_match_device(gpu, w, h, extra):
         assert np.array_equal(got, to_host(dev)[: nb * 16])
 
 
+@pytest.mark.parametrize("fmt", [W.DXT1, W.ETC1, W.DXT5, W.ETC2])
+@pytest.mark.parametrize("w,h,extra", [(16, 4, 0), (128, 252, 64), (128, 256, 0), (144, 260, 16), (2048, 32, 0),
+                                       (4096, 8, 0), (32768, 8, 0), (16, 8192, 4), (1456, 1436, 0)])
+def test_dropin_fed_kernel_sizes(gpu, w, h, extra, fmt):
+    """One-chunk host images on both sides of the size from which the kernel
+    is launched before the rows are staged, with uneven last parts, parts of
+    one block row, and a group of blocks in several parts, == the device entry
+    point; and again with a kernel that gives up its wait at once, whose image
+    is encoded again."""
+    import ctypes
+    stride = w * 4 + extra
+    img = gpu.synth_host(2, 51, fmt, 12, w, h, stride, fill=0xA5)
+    n = (w // 4) * (h // 4) * gpu.block_bytes(fmt)
+    src, out = upload(img.reshape(h, stride)[:, :w * 4]), dev_buffer(n)
+    gpu.compress_device(fmt, out, src, w, h, w * 4)
+    want = to_host(out)
+    say(f"drop-in fed kernel {w}x{h} stride {stride} fmt {fmt}")
+    late = gpu._lib.goofy_impl_compress_with_patience
+    late.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint, ctypes.c_uint, ctypes.c_uint,
+                     ctypes.c_uint64]
+    for call in range(6):
+        got = np.full(n + 64, 0xCD, np.uint8)
+        if call % 2:
+            assert late(fmt, got.ctypes.data, img.ctypes.data, w, h, stride, 0) == 0
+        else:
+            assert gpu._lib.goofy_hip_compress(fmt, gpu._u8(got), gpu._u8(img), w, h, stride) == 0
+        assert np.array_equal(got[:n], want) and (got[n:] == 0xCD).all(), call
+
+
 def test_dropin_from_threads(gpu):
     """The drop-in on four host threads at once, each with its own images of
     one to several staging chunks: every call bit-identical to the same call
