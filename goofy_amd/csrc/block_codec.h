@@ -89,22 +89,21 @@ __device__ __forceinline__ uint32_t max3_b16(uint32_t a, uint32_t b, uint32_t c)
     return __builtin_bit_cast(uint32_t, r);
 }
 
-// Luma of the colour in byte lanes 0..2 of c (result in byte 0, other bytes
-// are don't-care).
-__device__ __forceinline__ uint32_t luma_b0(uint32_t c)
+// Luma of the colour in bytes 0..2 of c (byte 3 ignored), in byte 1 of the
+// result; bytes 2 and 3 are zero, byte 0 is don't-care.  The two nested
+// rounding averages come to (R + 2G + B + 3) >> 2, a dot product: with the
+// weights and the 3 times 64 the shift by 2 ends on a byte boundary (64 x 1023
+// < 2^16).  One v_dot4_u32_u8 per pixel.
+__device__ __forceinline__ uint32_t luma_b1(uint32_t c)
 {
-    const uint32_t rb = avg4(c, c >> 16);  // byte0 = avg(R,B)
-    return avg4(rb, c >> 8) & 0xFFu;       // byte0 = avg(avg(R,B),G)
+    return __builtin_amdgcn_udot4(c, 0x00408040u, 192u, false);
 }
 
-// Luma of four pixels, packed: byte i = Y(p_i).
+// Luma of four pixels, packed: byte i = Y(p_i).  Seven instructions (nine with
+// byte averages).
 __device__ __forceinline__ uint32_t luma4(uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3)
 {
-    // [R0 R1 G0 G1] and [B0 B1 G0 G1] -> avg -> [avg(R,B)0, avg(R,B)1, G0, G1]
-    const uint32_t q01 = avg4(perm(p1, p0, 0x05010400u), perm(p1, p0, 0x05010602u));
-    const uint32_t q23 = avg4(perm(p3, p2, 0x05010400u), perm(p3, p2, 0x05010602u));
-    // [rb0 rb1 rb2 rb3] and [G0 G1 G2 G3]
-    return avg4(perm(q23, q01, 0x05040100u), perm(q23, q01, 0x07060302u));
+    return perm(luma_b1(p1), luma_b1(p0), 0x0c0c0501u) | perm(luma_b1(p3), luma_b1(p2), 0x05010c0cu);
 }
 
 // Byte 0 of x copied into all four bytes (v_perm_b32 broadcast; avoids the
@@ -116,26 +115,20 @@ __device__ __forceinline__ uint32_t q5(uint32_t c) { return (c - (c != 0u ? 1u :
 
 struct BlockStats {
     uint32_t range, mid, qt;
-    uint32_t mnrb, mxrb;  // R, B of the bounding-box corners in 16-bit lanes
-    uint32_t mng, mxg;    // G of the corners
+    uint32_t mn, mx;  // corners of the bounding box: bytes R, G, B, 0
 };
 
-// The rest of the statistics from the bounding-box corners: R, B in the
-// 16-bit lanes of mnrb / mxrb, G in mng / mxg.  Both corners' lumas come
-// out of one pass of byte averages (bytes 0 and 1 of y2), and the roundings
-// (x + 1) >> 1 of mid and qt are byte averages too (range <= 255).
-__device__ __forceinline__ BlockStats corner_stats(uint32_t mnrb, uint32_t mxrb, uint32_t mng, uint32_t mxg)
+// The rest of the statistics from the bounding-box corners.  The roundings
+// (x + 1) >> 1 of mid and qt are byte averages (range <= 255).
+__device__ __forceinline__ BlockStats corner_stats(uint32_t mn, uint32_t mx)
 {
     BlockStats s;
-    s.mnrb = mnrb;
-    s.mxrb = mxrb;
-    s.mng = mng;
-    s.mxg = mxg;
-    const uint32_t rb = perm(mxrb, mnrb, 0x06020400u);             // [R_mn R_mx B_mn B_mx]
-    const uint32_t y2 = avg4(avg4(rb, rb >> 16), mng | (mxg << 8));  // [Y(mn) Y(mx) . .]
-    const uint32_t d = ((y2 >> 8) & 0xFFu) - (y2 & 0xFFu);          // >= 0: luma is monotone per channel
+    s.mn = mn;
+    s.mx = mx;
+    const uint32_t ymn = luma_b1(mn), ymx = luma_b1(mx);
+    const uint32_t d = (ymx >> 8) - (ymn >> 8);  // >= 0: luma is monotone per channel
     s.range = d > 8u ? d : 8u;
-    s.mid = avg4(y2, y2 >> 8) & 0xFFu;
+    s.mid = (avg4(ymn, ymx) >> 8) & 0xFFu;
     const uint32_t half = avg4(s.range, 0u);
     const uint32_t quarter = avg4(half, 0u);
     const uint32_t eighth = avg4(quarter, 0u);
@@ -178,9 +171,9 @@ __device__ __forceinline__ BlockStats block_stats(const uint32_t (&p)[16])
     mxg = max3_b16(mxg, g[5], g[6]);
     mng = pk_min16(mng, g[7]);
     mxg = pk_max16(mxg, g[7]);
-    mng = pk_min16(mng, mng >> 16) & 0xFFu;
-    mxg = pk_max16(mxg, mxg >> 16) & 0xFFu;
-    return corner_stats(mnrb, mxrb, mng, mxg);
+    mng = pk_min16(mng, mng >> 16);
+    mxg = pk_max16(mxg, mxg >> 16);
+    return corner_stats(perm(mng, mnrb, 0x0c020400u), perm(mxg, mxrb, 0x0c020400u));
 }
 
 // The same for a block whose alpha range is needed too: v_pk_min_u16 /
@@ -200,12 +193,12 @@ __device__ __forceinline__ BlockStats block_stats_alpha(const uint32_t (&p)[16],
     }
     amn = lo >> 24;
     amx = hi >> 24;
-    return corner_stats(mnrb, mxrb, (lo >> 8) & 0xFFu, (hi >> 8) & 0xFFu);
+    return corner_stats(perm(lo, mnrb, 0x0c020500u), perm(hi, mxrb, 0x0c020500u));
 }
 
 // Per-byte comparison masks for four packed lumas y4 against the block's mid
-// and threshold: bit 7 of each byte of *gez = (y >= mid), of *near =
-// (|y - mid| < qt) = (lo <= y <= hi).  Uses avg(~a, b) >= 128  <=>  b >= a
+// and threshold: bit 7 of each byte of *gez = (y >= mid), other bits
+// don't-care; of *near = (|y - mid| < qt) = (lo <= y <= hi), other bits zero.  Uses avg(~a, b) >= 128  <=>  b >= a
 // for bytes a, b, and for the upper bound the floor average:
 // (~hi + y) >> 1 >= 128  <=>  y > hi, which also holds for hi = 255 (never).
 // nhi4 = ~hi in all four bytes.
@@ -213,7 +206,8 @@ __device__ __forceinline__ void compare4(uint32_t y4, uint32_t nmid4, uint32_t n
                                          uint32_t* near)
 {
     *gez = avg4(nmid4, y4);
-    *near = avg4(nlo4, y4) & ~__builtin_amdgcn_lerp(nhi4, y4, 0u);
+    // a & ~b & c (truth table 0x20)
+    *near = __builtin_amdgcn_bitop3_b32(avg4(nlo4, y4), __builtin_amdgcn_lerp(nhi4, y4, 0u), 0x80808080u, 0x20u);
 }
 
 // q5 of the two 16-bit lanes of x: subsat(c, 1) >> 3 per lane.
@@ -225,34 +219,29 @@ __device__ __forceinline__ uint32_t q5x2(uint32_t x)
 
 // The DXT1 endpoint word c0 | c1 << 16: c0 = RGB565 of the box maximum with
 // the green LSB forced to 1 (so c0 > c1, 4-colour mode), c1 = RGB565 of the
-// minimum.  All six channels go through q5 in 16-bit lanes: [R, B] of the
-// maximum, [R, B] of the minimum and [G max, G min]; two v_perm_b32 pair the
-// reds and the blues of both endpoints.
+// minimum.  A v_perm_b32 per channel pairs it of both corners, maximum in the
+// low 16-bit lane, and all six channels go through q5 in 16-bit lanes.
 __device__ __forceinline__ uint32_t dxt1_endpoints(const BlockStats& s)
 {
-    const uint32_t x = q5x2(s.mxrb), n = q5x2(s.mnrb), g = q5x2(s.mxg | (s.mng << 16));
-    const uint32_t r = perm(n, x, 0x0c040c00u);  // [R max, R min] in the two lanes
-    const uint32_t b = perm(n, x, 0x0c060c02u);  // [B max, B min]
+    const uint32_t r = q5x2(perm(s.mn, s.mx, 0x0c040c00u));
+    const uint32_t g = q5x2(perm(s.mn, s.mx, 0x0c050c01u));
+    const uint32_t b = q5x2(perm(s.mn, s.mx, 0x0c060c02u));
     return (r << 11) | (g << 6) | b | 0x20u;
 }
 
 // The DXT1 index word from the per-row compare masks (bit 7 of byte c of
 // gez[r] / near[r] for pixel (r, c)): pixel (r, c)'s 2-bit code, bit 0 =
-// y < mid and bit 1 = near, at bits 8r + 2c.  Per row, bit selects put both
-// flags in bits 6, 7 of each byte, the byte pairs' codes side by side in bits
-// 6..9 and 22..25, and all four in bits 6..13.
+// y < mid and bit 1 = near, at bits 8r + 2c.  A row's flags, 0 or 128 each,
+// weighted by 4^c and 2 x 4^c, are 128 times the row's index byte: two dot
+// products a row.  Rows are joined in pairs below 2^23 before the 128 goes.
 __device__ __forceinline__ uint32_t dxt1_index_word(const uint32_t (&gez)[4], const uint32_t (&near)[4])
 {
-    uint32_t idx = 0;
+    uint32_t row[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        // near in bit 7, ~gez in bit 6 (truth table 0xC5: sel ? near : ~gez)
-        const uint32_t z = __builtin_amdgcn_bitop3_b32(0x80808080u, near[r], gez[r] >> 1, 0xC5u);
-        const uint32_t y = bsel(0x00C000C0u, z, z >> 6);
-        const uint32_t g = bsel(0x000003C0u, y, y >> 12);
-        idx |= ((g >> 6) & 0xFFu) << (8 * r);
-    }
-    return idx;
+    for (int r = 0; r < 4; ++r)
+        row[r] = __builtin_amdgcn_udot4(
+            near[r], 0x80200802u, __builtin_amdgcn_udot4(~gez[r] & 0x80808080u, 0x40100401u, 0u, false), false);
+    return ((row[0] + (row[1] << 8)) >> 7) | ((row[2] + (row[3] << 8)) << 9);
 }
 
 // The ETC1S selector word (goofy_tc.h:1375-1395: word bit j <-> column
@@ -300,7 +289,7 @@ typedef short i16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ uint32_t etc1_base_bytes(uint32_t avgc, uint32_t mid)
 {
-    const int32_t ya = (int32_t)luma_b0(avgc);
+    const int32_t ya = (int32_t)(luma_b1(avgc) >> 8);
     const int32_t t = (int32_t)mid - ya - 1;
     const int32_t sd = t < -128 ? -128 : (t > 126 ? 126 : t);  // the correction minus one
     const uint32_t sd2 = perm(0u, (uint32_t)sd, 0x01000100u);   // in both lanes
@@ -435,19 +424,21 @@ __device__ __forceinline__ uint2 encode_block(const uint32_t (&p)[16])
 // max - 9m (highest level on the maximum).
 
 struct AlphaRows {
-    uint32_t w[4];  // word r: byte c = alpha of pixel (row r, column c)
+    uint32_t pair[8];  // the alphas of pixels 2i and 2i + 1 in the 16-bit lanes
+    uint32_t w[4];     // word r: byte c = alpha of pixel (row r, column c)
     uint32_t mn, mx;
 };
 
-// Alpha rows of a block whose alpha range [amn, amx] is known.
+// Alphas of a block whose alpha range [amn, amx] is known.
 __device__ __forceinline__ AlphaRows alpha_rows(const uint32_t (&p)[16], uint32_t amn, uint32_t amx)
 {
     AlphaRows a;
     a.mn = amn;
     a.mx = amx;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)  // [A0 A1 0 0] | [0 0 A2 A3]
-        a.w[r] = perm(p[4 * r + 1], p[4 * r], 0x0c0c0703u) | perm(p[4 * r + 3], p[4 * r + 2], 0x07030c0cu);
+    for (int i = 0; i < 8; ++i) a.pair[i] = perm(p[2 * i + 1], p[2 * i], 0x0c070c03u);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) a.w[r] = perm(a.pair[2 * r + 1], a.pair[2 * r], 0x06040200u);
     return a;
 }
 
@@ -478,47 +469,109 @@ __device__ __forceinline__ uint32_t sel3(uint32_t s2, uint32_t s1, uint32_t s0)
     return bsel(0x80808080u, s2, bsel(0x40404040u, s1 >> 1, s0 >> 2));
 }
 
-// BC3 alpha block as two little-endian words, from the block's alpha rows.
+// The BC3 ranks of a block by one multiply-add per pixel.  With d = alpha - min
+// and range R = max - min, the rank of a pixel among the 8 levels (as above:
+// the number of midpoints ceil((lv[k-1] + lv[k]) / 2), lv[k] = floor(k R / 7),
+// that d reaches) is the top three bits of the 16-bit number d * mul + add for
+// a suitable mul and add of each R: the midpoints lie close enough to a line.
+// One entry per R, from the midpoints themselves: for each of them d * mul +
+// add has to reach k * 8192 there and not one step before, and 2^16 nowhere.
+// lut: the selector of each rank (0 -> 1 (min), 7 -> 0 (max), 8 - t between).
+//   R = 2 and R = 4 have other ranks: their few values of d take ranks of
+// their own, and the entry's lut has the selectors.  R = 254 misses by little
+// (bc3_alpha).
+struct Bc3Entry {
+    uint32_t mul, add, lut_lo, lut_hi;
+};
+struct Bc3Table {
+    Bc3Entry e[256];
+};
+
+constexpr Bc3Table make_bc3_table()
+{
+    Bc3Table t{};
+    for (int range = 0; range < 256; ++range) {
+        Bc3Entry& e = t.e[range];
+        e.lut_lo = 0x05060701u;
+        e.lut_hi = 0x00020304u;
+        if (range == 0) {  // one value, the maximum's selector
+            e.add = 7u * 8192u;
+            continue;
+        }
+        if (range == 2) {  // ranks 3, 6, 7, the last taken as 9 mod 8
+            e.mul = e.add = 3u * 8192u;
+            e.lut_lo = 0x05060001u;
+            continue;
+        }
+        if (range == 4) {  // ranks 1, 3, 5, 6, 7, taken as 1 .. 5
+            e.mul = e.add = 8192u;
+            e.lut_lo = 0x03050701u;
+            e.lut_hi = 0x00020002u;
+            continue;
+        }
+        int mid[8] = {};
+        for (int k = 1; k < 8; ++k) mid[k] = ((k - 1) * range / 7 + k * range / 7 + 1) / 2;
+        for (int mul = range < 7 ? 8192 : 57344 / range - 24; mul < 57344 / range + 24 && !e.mul; ++mul) {
+            int lo = 0, hi = 65535 - range * mul;
+            for (int k = 1; k < 8; ++k) {
+                if (k * 8192 - mid[k] * mul > lo) lo = k * 8192 - mid[k] * mul;
+                if (mid[k] > 0 && k * 8192 - 1 - (mid[k] - 1) * mul < hi) hi = k * 8192 - 1 - (mid[k] - 1) * mul;
+            }
+            if (lo <= hi) {
+                e.mul = (uint32_t)mul;
+                e.add = (uint32_t)lo;
+            }
+        }
+        if (range == 254) {  // right but for d = 235, 2 above the last step's 57344
+            e.mul = 226u;
+            e.add = 4236u;
+        }
+    }
+    return t;
+}
+static __device__ const Bc3Table bc3_table = make_bc3_table();
+
+// BC3 alpha block as two little-endian words, from the block's alphas.  Nine
+// instructions a row where seven threshold compares and the selector logic
+// take twenty, and one 16-byte table entry instead of eight levels.  The alpha
+// encoders are bound by their instructions as much as by memory (84-90% of
+// their cycles issued one): with this, the lumas and the index word by dot
+// products and EAC's packing in bytes, DXT5 at 8192^2 went from 53.7 to 52.3 us
+// (4100x3076: 13.1 to 12.2), ETC2 RGBA8 54.5 to 53.5, both from one read 70.0
+// to 65.8.
 __device__ __forceinline__ uint2 bc3_alpha(const AlphaRows& a)
 {
-    // level k = mn + floor(k*range/7); (x * 9363) >> 16 == x / 7 for x <= 1785.
-    // Inverted: 255 - level = nmn - floor(k*r9 / 2^16) = the high half of
-    // (nmn << 16 | 0xffff) - k*r9 (the low half only absorbs the borrow), so
-    // one multiply-add and one v_perm_b32 of byte 2 give the replicated level.
-    const uint32_t range = a.mx - a.mn, r9 = range * 9363u, nmn = 255u - a.mn;
-    const uint32_t c = (nmn << 16) | 0xFFFFu;
-    uint32_t nlv4[8];
-    nlv4[0] = rep4(nmn);
+    const uint32_t range = a.mx - a.mn;
+    const Bc3Entry e = bc3_table.e[range];
+    const unsigned short mul = (unsigned short)e.mul, add = (unsigned short)(e.add - a.mn * e.mul);
+    const u16x2 mul2 = {mul, mul}, add2 = {add, add};
+    uint32_t pair[8];
 #pragma unroll
-    for (int k = 1; k < 7; ++k) nlv4[k] = perm(0u, c - (uint32_t)k * r9, 0x02020202u);
-    nlv4[7] = rep4(255u - a.mx);
-    uint32_t nthr4[7];
-    rep_midpoints(nlv4, nthr4);
-    uint32_t g[4];
+    for (int i = 0; i < 8; ++i) pair[i] = a.pair[i];
+    if (__builtin_expect(range == 254u, 0)) {
+        // d = 235 ranks one too high: take it as 234, which has its rank
+        const unsigned short at = (unsigned short)(a.mn + 235u);
+        const u16x2 at2 = {at, at}, one = {1, 1};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const u16x2 v = __builtin_bit_cast(u16x2, pair[i]);
+            pair[i] = __builtin_bit_cast(uint32_t, v - one + __builtin_elementwise_min(v ^ at2, one));
+        }
+    }
+    uint32_t row[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        uint32_t m[7];
-        rank_flags(a.w[r], nthr4, m);
-        // rank t -> selector: 0 -> 1 (a1), 7 -> 0 (a0), 8 - t in between:
-        //   t    0 1 2 3 4 5 6 7
-        //   s2   0 1 1 1 1 0 0 0   = f1 & ~f5
-        //   s1   0 1 1 0 0 1 1 0   = f1 ^ f3 ^ f5 ^ f7
-        //   s0   1 1 0 1 0 1 0 0   = (f1 ^ ... ^ f6) | ~f1
-        const uint32_t x = xor3(m[0], m[2], m[4]);
-        const uint32_t s2 = m[0] & ~m[4], s1 = x ^ m[6];
-        const uint32_t s0 = (x ^ xor3(m[1], m[3], m[5])) | ~m[0];
-        const uint32_t z = sel3(s2, s1, s0);
-        // columns 0, 1 -> bits 5..10 and 2, 3 -> bits 21..26, then all four
-        // -> bits 5..16, column c at 5 + 3c (other bits don't-care)
-        const uint32_t y = bsel(0x00E000E0u, z, z >> 5);
-        g[r] = bsel(0x000007E0u, y, y >> 10);
+        const u16x2 t0 = __builtin_bit_cast(u16x2, pair[2 * r]) * mul2 + add2;
+        const u16x2 t1 = __builtin_bit_cast(u16x2, pair[2 * r + 1]) * mul2 + add2;
+        // the four ranks in bits 5..7 of the bytes, then bits 0..2: the lookup's selectors
+        const uint32_t t = perm(__builtin_bit_cast(uint32_t, t1), __builtin_bit_cast(uint32_t, t0), 0x07050301u);
+        const uint32_t s = perm(e.lut_hi, e.lut_lo, (t >> 5) & 0x07070707u);
+        // column c at bits 3c
+        row[r] = ((s >> 24) << 9) | __builtin_amdgcn_udot4(s, 0x00400801u, 0u, false);
     }
-    // row r at bits 12r..12r+11 of the 48 index bits after a0, a1: word 0
-    // takes row 0 and the low 4 bits of row 1, word 1 the rest
-    const uint32_t head = a.mx | (a.mn << 8);
-    const uint32_t w0 = bsel(0xFFFFu, head, bsel(0x0FFF0000u, g[0] << 11, g[1] << 23));
-    const uint32_t w1 = bsel(0xFFu, g[1] >> 9, bsel(0xFFF00u, g[2] << 3, g[3] << 15));
-    return make_uint2(w0, w1);
+    // row r at bits 12r..12r+11 of the 48 index bits after a0, a1
+    const uint32_t lo = row[0] | (row[1] << 12), hi = row[2] | (row[3] << 12);
+    return make_uint2((a.mx | (a.mn << 8)) | (lo << 16), perm(hi, lo, 0x06050402u));
 }
 
 // EAC (ETC2 RGBA8 alpha) block as two little-endian words, from the block's
@@ -549,29 +602,29 @@ __device__ __forceinline__ uint2 eac_alpha(const AlphaRows& a)
     for (int k = 0; k < 8; ++k) nlv4[k] = perm(0u, w[k >> 1], (k & 1) ? 0x02020202u : 0u);
     uint32_t nthr4[7];
     rep_midpoints(nlv4, nthr4);
-    // Selector column groups: even columns (0, 2) and odd ones (1, 3) in the
-    // two 16-bit halves, 12 bits each, row 0 in the top three.
-    uint32_t ge = 0, go = 0;
+    uint32_t z[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        uint32_t m[7];
-        rank_flags(a.w[r], nthr4, m);
+        uint32_t f[7];
+        rank_flags(a.w[r], nthr4, f);
         // rank t -> selector: 0..3 -> 3..0 (negative modifiers), 4..7
         // unchanged: s2 = f4, s1 = ~(f2 ^ f6), s0 = ~(f1 ^ f2 ^ f3 ^ f5 ^ f6 ^ f7)
-        const uint32_t s1 = ~(m[1] ^ m[5]);
-        const uint32_t s0 = ~(xor3(m[0], m[1], m[2]) ^ xor3(m[4], m[5], m[6]));
-        const uint32_t z = sel3(m[3], s1, s0);
-        // column 0 / 2 selector at bits 5..7 / 21..23 -> 9-3r / 25-3r;
-        // column 1 / 3 at bits 13..15 / 29..31 -> 9-3r / 25-3r
-        const uint32_t dst = 0x0E000E00u >> (3 * r);
-        ge = bsel(dst, r < 2 ? z << (4 - 3 * r) : z >> (3 * r - 4), ge);
-        go = bsel(dst, z >> (4 + 3 * r), go);
+        const uint32_t s1 = ~(f[1] ^ f[5]);
+        const uint32_t s0 = ~(xor3(f[0], f[1], f[2]) ^ xor3(f[4], f[5], f[6]));
+        z[r] = sel3(f[3], s1, s0);
     }
-    // 48 bits, big-endian: column 0 (x = 0) first, 12 bits per column
-    const uint32_t hi = ((ge & 0xFFFu) << 12) | (go & 0xFFFu);  // columns 0, 1
-    const uint32_t lo = ((ge >> 16) << 12) | (go >> 16);        // columns 2, 3
+    // 48 bits, big-endian: column 0 (x = 0) first, 12 bits per column, row 0
+    // in its top three.  Rows 0, 1 and 2, 3 of every column in bits 2..7 of a
+    // byte; the two bytes of a column in a 16-bit lane, moved together to bits
+    // 4..15; and the lanes of two columns together to bits 8..31.
+    const uint32_t r01 = bsel(0xE0E0E0E0u, z[0], z[1] >> 3), r23 = bsel(0xE0E0E0E0u, z[2], z[3] >> 3);
+    auto columns = [](uint32_t c) {  // c: bytes r23, r01 of the second column, then of the first
+        const uint32_t q = bsel(0xFC00FC00u, c, c << 2);
+        return bsel(0xFFF00000u, q, q << 4);
+    };
+    const uint32_t hi = columns(perm(r01, r23, 0x04000501u)), lo = columns(perm(r01, r23, 0x06020703u));
     const uint32_t head = (uint32_t)b | (((m << 4) | 9u) << 8);
-    return make_uint2(perm(hi, head, 0x05060100u), perm(lo, hi, 0x04050600u));
+    return make_uint2(perm(hi, head, 0x06070100u), perm(lo, hi, 0x05060701u));
 }
 
 // DXT5 / ETC2 RGBA8 block: {alpha words, colour words}.  One pass over the

@@ -70,7 +70,15 @@ inline uint32_t goofy_host_alignbit(uint32_t a, uint32_t b, uint32_t s)
     return (uint32_t)((((uint64_t)a << 32) | b) >> (s & 31u));
 }
 
+// V_DOT4_U32_U8: c plus the sum of the products of a's and b's bytes.
+inline uint32_t goofy_host_udot4(uint32_t a, uint32_t b, uint32_t c, bool)
+{
+    for (int i = 0; i < 4; ++i) c += ((a >> (8 * i)) & 0xFFu) * ((b >> (8 * i)) & 0xFFu);
+    return c;
+}
+
 #define __builtin_amdgcn_perm goofy_host_perm
 #define __builtin_amdgcn_alignbit goofy_host_alignbit
 #define __builtin_amdgcn_lerp goofy_host_lerp
 #define __builtin_amdgcn_bitop3_b32 goofy_host_bitop3
+#define __builtin_amdgcn_udot4 goofy_host_udot4

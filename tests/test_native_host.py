@@ -69,6 +69,33 @@ def test_device_block_codec_on_host_matches_oracle(tmp_path, oracle, codec_host,
         assert bad.size == 0, f"format {fmt}: {bad.size} blocks differ, first {bad[:5]}"
 
 
+def test_device_alpha_codec_on_host_exhaustive(tmp_path, oracle, codec_host):
+    """Every alpha range (min, max) with every alpha in between, and the two
+    ends, in every block: the multiply-add that ranks BC3 alphas has an entry
+    for each range, and EAC packs its selectors column by column."""
+    import numpy as np
+    alphas = []
+    for mn in range(256):
+        for mx in range(mn, 256):
+            v = np.arange(mn, mx + 1)
+            n = -(-v.size // 14)
+            v = np.concatenate([v, np.full(n * 14 - v.size, mx)]).reshape(n, 14)
+            ends = np.tile([mx, mn], (n, 1))
+            alphas.append(np.concatenate([v[:, :5], ends[:, :1], v[:, 5:], ends[:, 1:]], 1))
+    alphas = np.concatenate(alphas).astype(np.uint8)
+    blocks = np.random.default_rng(5).integers(0, 256, (alphas.shape[0], 16, 4), dtype=np.uint8)
+    blocks[:, :, 3] = alphas
+    blocks = np.ascontiguousarray(blocks.reshape(-1, 64))
+    n = blocks.shape[0]
+    (tmp_path / "in.bin").write_bytes(blocks.tobytes())
+    subprocess.run([str(codec_host), "encode", str(tmp_path / "in.bin"), str(tmp_path / "out.bin")], check=True,
+                   timeout=120)
+    out = np.frombuffer((tmp_path / "out.bin").read_bytes(), np.uint8)[16 * n:].reshape(2, n, 16)
+    for fmt in (2, 3):
+        bad = np.nonzero((out[fmt - 2] != oracle.encode_blocks(fmt, blocks).reshape(n, 16)).any(1))[0]
+        assert bad.size == 0, f"format {fmt}: {bad.size} of {n} blocks differ, first alphas {alphas[bad[:3]]}"
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 2, 3])
 def test_device_block_decoders_on_host_match_oracle(tmp_path, oracle, harness, codec_host, fmt):
     """The kernels' decoders against the oracle's and the harness's on random
