@@ -20,22 +20,39 @@
 
 namespace goofy_dev {
 
-// The decoders below hand out one pixel row at a time: emit(y, row) gets the
-// four RGBA8 words of row y (y = 0..3, in order), so a caller that consumes
-// rows as they come (a store, a comparison) keeps 4 pixels live, not 16.
+// The decoders below hand out one pixel row at a time, as four channel planes:
+// emit(y, plane) gets row y (y = 0..3, in order), byte x of plane[c] being
+// byte c of pixel (x, y).  A caller that consumes rows as they come (a
+// comparison) keeps 4 pixels live, not 16, and one that works on planes is
+// spared their interleaving into pixel words (interleave_row).
+// OPAQUE: plane[3] is all ones, known at compile time.
 
-// Replace byte 3 (alpha) of a row's four pixels with the bytes of a4.
-__device__ __forceinline__ void put_alpha(uint32_t (&row)[4], uint32_t a4)
+// The four RGBA8 words of a row.
+template <bool OPAQUE>
+__device__ __forceinline__ void interleave_row(const uint32_t (&plane)[4], uint32_t (&row)[4])
 {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) row[c] = __builtin_amdgcn_perm(a4, row[c], 0x04020100u + (c << 24));
+    const uint32_t rg01 = __builtin_amdgcn_perm(plane[1], plane[0], 0x05010400u);  // R0 G0 R1 G1
+    const uint32_t rg23 = __builtin_amdgcn_perm(plane[1], plane[0], 0x07030602u);  // R2 G2 R3 G3
+    if constexpr (OPAQUE) {
+        // pixel x = R_x G_x from rg, B_x, alpha 255 (selector 0x0d)
+        row[0] = __builtin_amdgcn_perm(plane[2], rg01, 0x0d040100u);
+        row[1] = __builtin_amdgcn_perm(plane[2], rg01, 0x0d050302u);
+        row[2] = __builtin_amdgcn_perm(plane[2], rg23, 0x0d060100u);
+        row[3] = __builtin_amdgcn_perm(plane[2], rg23, 0x0d070302u);
+    } else {
+        const uint32_t ba01 = __builtin_amdgcn_perm(plane[3], plane[2], 0x05010400u);  // B0 A0 B1 A1
+        const uint32_t ba23 = __builtin_amdgcn_perm(plane[3], plane[2], 0x07030602u);  // B2 A2 B3 A3
+        row[0] = __builtin_amdgcn_perm(ba01, rg01, 0x05040100u);
+        row[1] = __builtin_amdgcn_perm(ba01, rg01, 0x07060302u);
+        row[2] = __builtin_amdgcn_perm(ba23, rg23, 0x05040100u);
+        row[3] = __builtin_amdgcn_perm(ba23, rg23, 0x07060302u);
+    }
 }
 
 // BC1 block rows; FOUR: the colour block of BC3, always in 4-colour mode,
 // its alpha bytes from alpha_row(y).  Per channel the 4 palette bytes sit in
 // one word (byte k = entry k); a row's pixels come from one v_perm_b32 per
-// channel whose selector bytes are the pixels' 2-bit indices, and six more
-// interleave the channel rows and the alpha row into RGBA words.
+// channel whose selector bytes are the pixels' 2-bit indices.
 template <bool FOUR, class Alpha, class Emit>
 __device__ __forceinline__ void bc1_rows(uint32_t w0, uint32_t w1, Alpha&& alpha_row, Emit&& emit)
 {
@@ -58,19 +75,10 @@ __device__ __forceinline__ void bc1_rows(uint32_t w0, uint32_t w1, Alpha&& alpha
         const uint32_t x = (w1 >> (8 * y)) & 0xFFu;  // pixel c's index at bits 2c
         const uint32_t t = (x & 0x0Fu) | ((x & 0xF0u) << 12);
         const uint32_t sel = (t & 0x00030003u) | ((t & 0x000C000Cu) << 6);  // pixel c's index in byte c
-        const uint32_t r = __builtin_amdgcn_perm(0u, plane[0], sel);
-        const uint32_t g = __builtin_amdgcn_perm(0u, plane[1], sel);
-        const uint32_t bl = __builtin_amdgcn_perm(0u, plane[2], sel);
-        const uint32_t rg01 = __builtin_amdgcn_perm(g, r, 0x05010400u);   // R0 G0 R1 G1
-        const uint32_t rg23 = __builtin_amdgcn_perm(g, r, 0x07030602u);   // R2 G2 R3 G3
         // alpha: the BC3 alpha block's row, or BC1's own (3-colour mode)
-        const uint32_t a = FOUR ? alpha_row(y) : __builtin_amdgcn_perm(0u, alpha, sel);
-        const uint32_t ba01 = __builtin_amdgcn_perm(a, bl, 0x05010400u);  // B0 A0 B1 A1
-        const uint32_t ba23 = __builtin_amdgcn_perm(a, bl, 0x07030602u);  // B2 A2 B3 A3
-        uint32_t row[4] = {__builtin_amdgcn_perm(ba01, rg01, 0x05040100u),
-                           __builtin_amdgcn_perm(ba01, rg01, 0x07060302u),
-                           __builtin_amdgcn_perm(ba23, rg23, 0x05040100u),
-                           __builtin_amdgcn_perm(ba23, rg23, 0x07060302u)};
+        const uint32_t row[4] = {__builtin_amdgcn_perm(0u, plane[0], sel), __builtin_amdgcn_perm(0u, plane[1], sel),
+                                 __builtin_amdgcn_perm(0u, plane[2], sel),
+                                 FOUR ? alpha_row(y) : __builtin_amdgcn_perm(0u, alpha, sel)};
         emit(y, row);
     }
 }
@@ -125,15 +133,15 @@ __device__ __forceinline__ void etc2_th_planes(uint32_t hi, bool tmode, uint32_t
 // alpha 255.  O: red = bits 30-25 of hi, green 24 then 22-17, blue 16 then
 // 12-11 then 9-7; H: red 6-2 then 0, green = bits 31-25 of lo, blue 24-19;
 // V: red 18-13, green 12-6, blue 5-0.  6- and 7-bit values are widened by
-// replicating their top bits.  Writes the four pixels of row y.
-__device__ __forceinline__ void etc2_planar_row(uint32_t hi, uint32_t lo, int y, uint32_t (&row)[4])
+// replicating their top bits.  Writes the planes of row y.
+__device__ __forceinline__ void etc2_planar_row(uint32_t hi, uint32_t lo, int y, uint32_t (&plane)[4])
 {
     const uint32_t o6[3] = {(hi >> 25) & 63u, (((hi >> 24) & 1u) << 6) | ((hi >> 17) & 63u),
                             (((hi >> 16) & 1u) << 5) | (((hi >> 11) & 3u) << 3) | ((hi >> 7) & 7u)};
     const uint32_t h6[3] = {(((hi >> 2) & 31u) << 1) | (hi & 1u), lo >> 25, (lo >> 19) & 63u};
     const uint32_t v6[3] = {(lo >> 13) & 63u, (lo >> 6) & 127u, lo & 63u};
-#pragma unroll
-    for (int x = 0; x < 4; ++x) row[x] = 0xFF000000u;
+    plane[0] = plane[1] = plane[2] = 0u;
+    plane[3] = 0xFFFFFFFFu;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const int up = c == 1 ? 1 : 2, down = c == 1 ? 6 : 4;  // 7-bit green, 6-bit red and blue
@@ -146,7 +154,7 @@ __device__ __forceinline__ void etc2_planar_row(uint32_t hi, uint32_t lo, int y,
         // whose upper result bits the compiler assumes zero and gfx950 does
         // not clear
 #pragma unroll
-        for (int x = 0; x < 4; ++x, t += dh) row[x] |= ((uint32_t)min(max(t, 0), 1023) >> 2) << (8 * c);
+        for (int x = 0; x < 4; ++x, t += dh) plane[c] |= ((uint32_t)min(max(t, 0), 1023) >> 2) << (8 * x);
     }
 }
 
@@ -156,10 +164,9 @@ __device__ __forceinline__ void etc2_planar_row(uint32_t hi, uint32_t lo, int y,
 // Per channel, the 8 clamped palette bytes of both sub-blocks sit in two
 // words (sub-block 0 in the low word, entry = selector value).  A row's four
 // pixels then come from one v_perm_b32 per channel whose selector bytes are
-// the pixels' 2-bit selectors plus 4 for sub-block 1, and four more
-// v_perm_b32 interleave the channel rows into RGBA words (alpha 255 from
-// selector byte 0x0d).  T and H blocks use the same lookup with their four
-// paint colours in both words; planar blocks replace each row's pixels.
+// the pixels' 2-bit selectors plus 4 for sub-block 1.  T and H blocks use the
+// same lookup with their four paint colours in both words; planar blocks
+// replace each row's pixels.
 template <bool ALPHA, class Alpha, class Emit>
 __device__ __forceinline__ void etc_rows(uint32_t w0, uint32_t w1, Alpha&& alpha_row, Emit&& emit)
 {
@@ -191,7 +198,7 @@ __device__ __forceinline__ void etc_rows(uint32_t w0, uint32_t w1, Alpha&& alpha
         for (int y = 0; y < 4; ++y) {
             uint32_t row[4];
             etc2_planar_row(hi, lo, y, row);
-            if constexpr (ALPHA) put_alpha(row, alpha_row(y));
+            if constexpr (ALPHA) row[3] = alpha_row(y);
             emit(y, row);
         }
         return;
@@ -240,31 +247,13 @@ __device__ __forceinline__ void etc_rows(uint32_t w0, uint32_t w1, Alpha&& alpha
         const uint32_t t = cols >> y;
         uint32_t sel = (t & 0x01010101u) | ((t >> 3) & 0x02020202u);  // pixel x's selector in byte x
         sel |= flip ? (y >= 2 ? 0x04040404u : 0u) : 0x04040000u;
-        const uint32_t r = __builtin_amdgcn_perm(plane[0][1], plane[0][0], sel);
-        const uint32_t g = __builtin_amdgcn_perm(plane[1][1], plane[1][0], sel);
-        const uint32_t bl = __builtin_amdgcn_perm(plane[2][1], plane[2][0], sel);
-        const uint32_t rg01 = __builtin_amdgcn_perm(g, r, 0x05010400u);   // R0 G0 R1 G1
-        const uint32_t rg23 = __builtin_amdgcn_perm(g, r, 0x07030602u);   // R2 G2 R3 G3
-        if constexpr (ALPHA) {
-            const uint32_t a = alpha_row(y);
-            const uint32_t ba01 = __builtin_amdgcn_perm(a, bl, 0x05010400u);  // B0 A0 B1 A1
-            const uint32_t ba23 = __builtin_amdgcn_perm(a, bl, 0x07030602u);  // B2 A2 B3 A3
-            uint32_t row[4] = {__builtin_amdgcn_perm(ba01, rg01, 0x05040100u),
-                               __builtin_amdgcn_perm(ba01, rg01, 0x07060302u),
-                               __builtin_amdgcn_perm(ba23, rg23, 0x05040100u),
-                               __builtin_amdgcn_perm(ba23, rg23, 0x07060302u)};
-            emit(y, row);
-        } else {
-            // pixel x = R_x G_x from rg, B_x from bl, alpha 255 (selector 0x0d)
-            uint32_t row[4] = {__builtin_amdgcn_perm(bl, rg01, 0x0d040100u),
-                               __builtin_amdgcn_perm(bl, rg01, 0x0d050302u),
-                               __builtin_amdgcn_perm(bl, rg23, 0x0d060100u),
-                               __builtin_amdgcn_perm(bl, rg23, 0x0d070302u)};
-            emit(y, row);
-        }
+        const uint32_t row[4] = {__builtin_amdgcn_perm(plane[0][1], plane[0][0], sel),
+                                 __builtin_amdgcn_perm(plane[1][1], plane[1][0], sel),
+                                 __builtin_amdgcn_perm(plane[2][1], plane[2][0], sel),
+                                 ALPHA ? alpha_row(y) : 0xFFFFFFFFu};
+        emit(y, row);
     }
 }
-
 
 // An alpha palette of 8 levels held as the bytes of {hi:lo}, and the block's
 // 48 code bits; row r's four alphas are one v_perm_b32 with the row's 3-bit
@@ -377,11 +366,17 @@ __device__ __forceinline__ void decode_block_rows(uint4 b, Emit&& emit)
     }
 }
 
+// Formats whose decoded alpha is always 255 (BC1 has transparent black).
+template <int FMT>
+constexpr bool kOpaque = FMT == 1;
+
 // The 16 pixels of a block, row-major.
 template <int FMT>
 __device__ __forceinline__ void decode_block(uint4 b, uint32_t (&px)[16])
 {
-    decode_block_rows<FMT>(b, [&](int y, const uint32_t (&row)[4]) {
+    decode_block_rows<FMT>(b, [&](int y, const uint32_t (&plane)[4]) {
+        uint32_t row[4];
+        interleave_row<kOpaque<FMT>>(plane, row);
 #pragma unroll
         for (int c = 0; c < 4; ++c) px[4 * y + c] = row[c];
     });

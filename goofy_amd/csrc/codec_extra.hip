@@ -111,91 +111,80 @@ __global__ __launch_bounds__(256) void k_decode(const uint8_t* __restrict__ bloc
     }
 }
 
-// Squared errors of pixel pairs, summed exactly in integers.  e[0..3] sum
-// the per-byte squares.  The harness's luma weights are 0.21 / 0.72 / 0.07 on
-// bytes 2 / 1 / 0, so 100 x the luma difference is the integer
-// 21 dr + 72 dg + 7 db, whose square is
+// Squared errors, summed exactly in integers.  The harness's luma weights are
+// 0.21 / 0.72 / 0.07 on bytes 2 / 1 / 0, so 100 x the luma difference is the
+// integer 21 dr + 72 dg + 7 db, whose square is
 //   441 dr^2 + 5184 dg^2 + 49 db^2 + 3024 dr dg + 294 dr db + 1008 dg db.
-// Beyond the channel squares the luma sum needs only the three cross products
-// x[0] = sum dr dg, x[1] = sum dr db, x[2] = sum dg db (three 24-bit
-// multiply-adds a pixel, against a weighted sum and a 32-bit square);
+// Beyond the channel squares the luma sum needs only the three cross products.
 // lane_totals() forms the weighted total once per lane.  The host divides it by
 // 10^4 once: the exact value of the harness's sum, which its own double
 // arithmetic rounds per pixel (relative differences of order 1e-15 per term).
-// A lane's sums over at most kQualityLaneUnits blocks (or 4-pixel quads):
-// |x|, e <= 2048 * 16 * 255^2 < 2^31, so the loop adds in 32 bits and widens
-// once, at the end.
+//   The differences themselves are never formed.  With a row of each image as
+// channel planes, four pixels' bytes to a word, products of bytes sum by
+// v_dot4_u32_u8, and
+//   (a - d)^2         = (a a + d d) - 2 a d
+//   (ai - di)(aj - dj) = (ai aj + di dj) - (ai dj + di aj),
+// each bracket and product a sum of its own, subtracted once per lane.  24 dot
+// products a row of four pixels and 8 v_perm_b32 to split the source's words
+// into planes, where forming 16-bit differences and 7 products of them took 38
+// instructions and the decoders 6 to 8 more to interleave their planes.  Whole
+// calls went from 27.7 to 26.9 us at 4100x3076 and 65.6 to 65.4 at 8192^2
+// (ETC1; ETC2 RGBA8 30.6 to 30.1 and 73.3 to 71.8): the kernel then moves 6.0
+// TB/s.
+//   A lane sums over at most kQualityLaneUnits blocks (or 4-pixel quads): each
+// sum is at most 2048 * 16 * 2 * 255^2 = 4,261,478,400 < 2^32.
 struct ErrSums {
-    uint32_t e[4];
-    int32_t x[3];
+    uint32_t sq[4], ad[4];       // per byte: a a + d d, and a d
+    uint32_t same[3], mixed[3];  // per pair of bytes (2, 1), (2, 0), (1, 0)
 };
-// c + a * b on the low 24 bits of a and b, as one full-rate v_mad_i32_i24.
-// The compiler would split each into a 24-bit multiply and a shared
-// three-input add (1.5 instructions); the operands here are byte differences.
-__device__ __forceinline__ int32_t mad24(int32_t a, int32_t b, int32_t c)
+
+__device__ __forceinline__ uint32_t dot4(uint32_t a, uint32_t b, uint32_t c)
 {
-    int32_t r;
-    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
+    return __builtin_amdgcn_udot4(a, b, c, false);
 }
-__device__ __forceinline__ void accum_pixel(uint32_t a, uint32_t d, ErrSums& s)
+
+// The four pixels of a row as channel planes.
+__device__ __forceinline__ void split_row(u32x4 v, uint32_t (&plane)[4])
 {
-    int32_t diff[4];
+    const uint32_t rg01 = __builtin_amdgcn_perm(v.y, v.x, 0x05010400u), ba01 = __builtin_amdgcn_perm(v.y, v.x, 0x07030602u);
+    const uint32_t rg23 = __builtin_amdgcn_perm(v.w, v.z, 0x05010400u), ba23 = __builtin_amdgcn_perm(v.w, v.z, 0x07030602u);
+    plane[0] = __builtin_amdgcn_perm(rg23, rg01, 0x05040100u);
+    plane[1] = __builtin_amdgcn_perm(rg23, rg01, 0x07060302u);
+    plane[2] = __builtin_amdgcn_perm(ba23, ba01, 0x05040100u);
+    plane[3] = __builtin_amdgcn_perm(ba23, ba01, 0x07060302u);
+}
+
+// Four pixels: source words against decoded planes.  OPAQUE: decoded alpha is
+// 255 everywhere, and its error the square of the source's complement.
+template <bool OPAQUE>
+__device__ __forceinline__ void accum_row(u32x4 src, const uint32_t (&d)[4], ErrSums& s)
+{
+    uint32_t a[4];
+    split_row(src, a);
 #pragma unroll
-    for (int ch = 0; ch < 4; ++ch) {
-        diff[ch] = (int32_t)((a >> (8 * ch)) & 0xFFu) - (int32_t)((d >> (8 * ch)) & 0xFFu);
-        s.e[ch] = (uint32_t)mad24(diff[ch], diff[ch], (int32_t)s.e[ch]);
+    for (int c = 0; c < (OPAQUE ? 3 : 4); ++c) {
+        s.sq[c] = dot4(a[c], a[c], dot4(d[c], d[c], s.sq[c]));
+        s.ad[c] = dot4(a[c], d[c], s.ad[c]);
     }
-    s.x[0] = mad24(diff[2], diff[1], s.x[0]);
-    s.x[1] = mad24(diff[2], diff[0], s.x[1]);
-    s.x[2] = mad24(diff[1], diff[0], s.x[2]);
-}
-// The same sums two pixels at a time: one v_perm_b32 per channel and image
-// puts byte c of both pixels into the two 16-bit lanes of a word, one 16-bit
-// subtract gives both signed differences, and each of the seven sums takes
-// one v_dot2_i32_i16 (both lanes' products added): 19 instructions per pair
-// where the per-pixel form takes 22.  The ETC round trips use it (quality
-// calls 1-2% faster); in the BC1 / BC3 ones it raised the registers past the
-// grid's 6 waves per SIMD and gained nothing.
-typedef short i16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void accum_pair(uint32_t a0, uint32_t a1, uint32_t d0, uint32_t d1, ErrSums& s)
-{
-    i16x2 dc[4];
+    if constexpr (OPAQUE) s.sq[3] = dot4(~a[3], ~a[3], s.sq[3]);
+    constexpr int first[3] = {2, 2, 1}, second[3] = {1, 0, 0};
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const uint32_t sel = 0x0c040c00u + 0x00010001u * (uint32_t)c;  // [byte c of p0, 0, byte c of p1, 0]
-        dc[c] = __builtin_bit_cast(i16x2, __builtin_amdgcn_perm(a1, a0, sel)) -
-                __builtin_bit_cast(i16x2, __builtin_amdgcn_perm(d1, d0, sel));
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-        s.e[c] = (uint32_t)__builtin_amdgcn_sdot2(dc[c], dc[c], (int32_t)s.e[c], false);
-    s.x[0] = __builtin_amdgcn_sdot2(dc[2], dc[1], s.x[0], false);
-    s.x[1] = __builtin_amdgcn_sdot2(dc[2], dc[0], s.x[1], false);
-    s.x[2] = __builtin_amdgcn_sdot2(dc[1], dc[0], s.x[2], false);
-}
-// Four pixels: source words a against decoded words d.
-template <bool PAIRS>
-__device__ __forceinline__ void accum_quad(u32x4 a, const uint32_t (&d)[4], ErrSums& s)
-{
-    if constexpr (PAIRS) {
-        accum_pair(a.x, a.y, d[0], d[1], s);
-        accum_pair(a.z, a.w, d[2], d[3], s);
-    } else {
-        accum_pixel(a.x, d[0], s);
-        accum_pixel(a.y, d[1], s);
-        accum_pixel(a.z, d[2], s);
-        accum_pixel(a.w, d[3], s);
+    for (int k = 0; k < 3; ++k) {
+        const int i = first[k], j = second[k];
+        s.same[k] = dot4(a[i], a[j], dot4(d[i], d[j], s.same[k]));
+        s.mixed[k] = dot4(a[i], d[j], dot4(d[i], a[j], s.mixed[k]));
     }
 }
 // The lane's channel sums and its sum of squared luma differences (x 10^4),
 // in 64 bits; the luma total is exact and non-negative.
 __device__ __forceinline__ void lane_totals(const ErrSums& s, unsigned long long (&e)[4], unsigned long long& ey)
 {
+    long long x[3];
 #pragma unroll
-    for (int ch = 0; ch < 4; ++ch) e[ch] = s.e[ch];
-    ey = (unsigned long long)(441ll * s.e[2] + 5184ll * s.e[1] + 49ll * s.e[0] + 3024ll * s.x[0] + 294ll * s.x[1] +
-                              1008ll * s.x[2]);
+    for (int ch = 0; ch < 4; ++ch) e[ch] = s.sq[ch] - 2ull * s.ad[ch];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) x[k] = (long long)s.same[k] - (long long)s.mixed[k];
+    ey = 441ull * e[2] + 5184ull * e[1] + 49ull * e[0] + (unsigned long long)(3024ll * x[0] + 294ll * x[1] + 1008ll * x[2]);
 }
 
 // Sums of one workgroup (256 lanes = 4 waves): wave reduction by lane
@@ -309,20 +298,17 @@ template <int FMT>
 __device__ __forceinline__ void sqerr_tile(const QTile& t, bool valid, ErrSums& acc)
 {
     if (valid)
-        decode_block_rows<FMT>(t.b, [&](int y, const uint32_t (&row)[4]) {
-            accum_quad<FMT == 1 || FMT == 3>(t.v[y], row, acc);
+        decode_block_rows<FMT>(t.b, [&](int y, const uint32_t (&plane)[4]) {
+            accum_row<goofy_dev::kOpaque<FMT>>(t.v[y], plane, acc);
         });
 }
 
-// A wave's tiles first, first + step, ... in a grid-stride loop.
-// PIPELINE (BC1, ETC1, BC3): two register sets in turn, the next tile's
-// loads issued before the current tile is compared; every path into a
-// comparison has the same loads outstanding after it, so its wait leaves the
-// other set's loads in flight (65 / 75 / 73 VGPRs, within the grid's 6 waves
-// per SIMD; quality calls 2-3% faster).  ETC2 RGBA8 compares one tile at a
-// time (60 VGPRs): its two-set form needs 85, 5 waves per SIMD, and its
-// quality call took 8% longer.
-template <int FMT, bool NEAR, bool PIPELINE>
+// A wave's tiles first, first + step, ... in a grid-stride loop, one tile at a
+// time (48-65 VGPRs, so that all of the grid's 6 waves per SIMD fit).  Loading
+// the next tile into a second register set before comparing this one needs
+// 89-100 VGPRs with the plane sums and was no faster (whole calls at 8192^2,
+// two sets / one: BC1 65.7 / 64.8 us, ETC1 65.4 / 65.4, BC3 71.6 / 70.5).
+template <int FMT, bool NEAR>
 __device__ __forceinline__ void sqerr_loop(const uint8_t* __restrict__ blocks, const uint8_t* __restrict__ src,
                                            uint64_t pitch, uint32_t bw, uint32_t nblocks, uint64_t magic,
                                            ErrSums& acc)
@@ -330,31 +316,10 @@ __device__ __forceinline__ void sqerr_loop(const uint8_t* __restrict__ blocks, c
     const uint32_t step = gridDim.x * 256u;  // nblocks <= kQualityMaxLaunchUnits < 2^30: no overflow below
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t t = __builtin_amdgcn_readfirstlane(blockIdx.x * 256u + (threadIdx.x & ~63u));
-    if (t >= nblocks) return;
-    QTile a, b;
-    if constexpr (PIPELINE) {
-        uint32_t n = (nblocks - 1u - t) / step + 1u;  // tiles of this wave; all but the last are whole
+    for (; t < nblocks; t += step) {
+        QTile a;
         load_qtile<FMT, NEAR>(blocks, src, pitch, bw, nblocks, magic, t, lane, a);
-        while (n >= 3u) {
-            load_qtile<FMT, NEAR>(blocks, src, pitch, bw, nblocks, magic, t + step, lane, b);
-            sqerr_tile<FMT>(a, true, acc);
-            load_qtile<FMT, NEAR>(blocks, src, pitch, bw, nblocks, magic, t + 2u * step, lane, a);
-            sqerr_tile<FMT>(b, true, acc);
-            t += 2u * step;
-            n -= 2u;
-        }
-        if (n == 2u) {
-            load_qtile<FMT, NEAR>(blocks, src, pitch, bw, nblocks, magic, t + step, lane, b);
-            sqerr_tile<FMT>(a, true, acc);
-            sqerr_tile<FMT>(b, t + step + lane < nblocks, acc);
-        } else {
-            sqerr_tile<FMT>(a, t + lane < nblocks, acc);
-        }
-    } else {
-        for (; t < nblocks; t += step) {
-            load_qtile<FMT, NEAR>(blocks, src, pitch, bw, nblocks, magic, t, lane, a);
-            sqerr_tile<FMT>(a, t + lane < nblocks, acc);
-        }
+        sqerr_tile<FMT>(a, t + lane < nblocks, acc);
     }
 }
 
@@ -370,10 +335,9 @@ __global__ __launch_bounds__(256) void k_sqerr(const uint8_t* __restrict__ block
                                                uint64_t pitch, uint32_t bw, uint32_t nblocks, uint64_t magic,
                                                const QualityDest dest)
 {
-    constexpr bool kPipeline = FMT != 3;
     ErrSums acc = {};
-    if (tile_near(bw, 64u, pitch)) sqerr_loop<FMT, true, kPipeline>(blocks, src, pitch, bw, nblocks, magic, acc);
-    else sqerr_loop<FMT, false, kPipeline>(blocks, src, pitch, bw, nblocks, magic, acc);
+    if (tile_near(bw, 64u, pitch)) sqerr_loop<FMT, true>(blocks, src, pitch, bw, nblocks, magic, acc);
+    else sqerr_loop<FMT, false>(blocks, src, pitch, bw, nblocks, magic, acc);
     unsigned long long e[4], ey;
     lane_totals(acc, e, ey);
     finish_sums(e, ey, dest);
@@ -392,10 +356,9 @@ __global__ __launch_bounds__(256) void k_sqerr_images(const uint8_t* __restrict_
             __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a + (uint64_t)y * pitch_a + (uint64_t)x * 16u));
         const u32x4 vb =
             __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(b + (uint64_t)y * pitch_b + (uint64_t)x * 16u));
-        accum_pixel(va.x, vb.x, acc);
-        accum_pixel(va.y, vb.y, acc);
-        accum_pixel(va.z, vb.z, acc);
-        accum_pixel(va.w, vb.w, acc);
+        uint32_t d[4];
+        split_row(vb, d);
+        accum_row<false>(va, d, acc);
     }
     unsigned long long e[4], ey;
     lane_totals(acc, e, ey);

@@ -360,6 +360,34 @@ def test_quality_sums_past_one_launch_closed_form(gpu):
                                                                   abs=1e-9)
 
 
+@pytest.mark.parametrize("fmt", [W.DXT1, W.DXT5])
+def test_quality_sums_past_one_launch_of_white_blocks(gpu, fmt):
+    """The same 819,200,000 blocks, white and decoded white or nearly: the
+    sums of squares of both images, from which twice the sum of products is
+    taken, reach 2048 x 16 x 2 x 65025 = 4,261,478,400 in a lane, just under
+    2^32.  Every block errs as those of a small white image do."""
+    from goofy_amd import hip
+    w, h = 4096, 3_200_000
+    print(f"white quality past one launch: fmt={fmt} {w}x{h}", flush=True)
+    src = hip.DeviceBuffer(w * 4 * h, fill=0xFF)
+    blocks = hip.DeviceBuffer((w // 4) * (h // 4) * gpu.block_bytes(fmt))
+    dec = hip.DeviceBuffer(4 * 4 * 4)
+    try:
+        gpu.compress_device(fmt, blocks, src, w, h, w * 4)
+        gpu.decode_device(fmt, dec, blocks, 4, 4)
+        q = gpu.quality_device(fmt, blocks, src, w, h, w * 4)
+        px = dec.download().reshape(16, 4).astype(np.int64)
+    finally:
+        src.free()
+        blocks.free()
+    err = 255 - px
+    assert err.max() <= 8 and (px[:, 3] == 255).all()
+    n = (w // 4) * (h // 4)
+    assert q["sse_byte"] == [int(v) * n for v in (err ** 2).sum(0)]
+    y = int(((21 * err[:, 2] + 72 * err[:, 1] + 7 * err[:, 0]) ** 2).sum()) * n
+    assert q["sse_luma"] == pytest.approx(y / 1e4, rel=1e-15)
+
+
 @pytest.mark.parametrize("fmt", [W.ETC1, W.ETC2])
 def test_quality_sums_past_one_launch_etc_closed_form(gpu, oracle, fmt):
     """The same 819,200,000 blocks for the ETC round trips, which add two
