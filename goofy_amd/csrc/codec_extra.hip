@@ -80,12 +80,17 @@ __device__ __forceinline__ uint4 load_block_fmt(const uint8_t* blocks, uint64_t 
     }
 }
 
-template <int FMT>
+// Cache policies of the decoders' stores: streaming, streaming written through
+// (sc0 sc1 nt), and cached.
+constexpr int kStream = 2, kStreamThrough = 19, kCached = 0;
+
+template <int FMT, int STORE>
 __global__ __launch_bounds__(256) void k_decode(const uint8_t* __restrict__ blocks, uint8_t* __restrict__ dst,
-                                                uint64_t pitch, uint32_t bw, uint32_t nblocks, uint64_t magic)
+                                                uint64_t pitch, uint32_t bw, uint32_t nblocks, uint64_t magic,
+                                                uint32_t order)
 {
     // a wave's 64 consecutive blocks start at `first` (wave-uniform)
-    const uint32_t first = __builtin_amdgcn_readfirstlane(blockIdx.x * blockDim.x + (threadIdx.x & ~63u));
+    const uint32_t first = __builtin_amdgcn_readfirstlane(xcd_workgroup(order) * 256u + (threadIdx.x & ~63u));
     const uint32_t lane = threadIdx.x & 63u, i = first + lane;
     if (i >= nblocks) return;
     // the four rows are stored together after the block is decoded: storing
@@ -98,7 +103,7 @@ __global__ __launch_bounds__(256) void k_decode(const uint8_t* __restrict__ bloc
 #pragma unroll
         for (int y = 0; y < 4; ++y) {
             const u32x4 v = {px[4 * y], px[4 * y + 1], px[4 * y + 2], px[4 * y + 3]};
-            __builtin_amdgcn_raw_buffer_store_b128(v, t.rows, off, (uint32_t)pitch * y, kBufAux<true>);
+            __builtin_amdgcn_raw_buffer_store_b128(v, t.rows, off, (uint32_t)pitch * y, STORE);
         }
     } else {
         const uint32_t by = (uint32_t)(((uint64_t)i * magic) >> 40), bx = i - by * bw;
@@ -303,6 +308,11 @@ __device__ __forceinline__ void sqerr_tile(const QTile& t, bool valid, ErrSums& 
         });
 }
 
+// Runs of 32 workgroups per XCD (xcd_workgroup), as the grid-stride loops of
+// the quality kernels walk the image: BC1 at 8192^2 64.7 -> 63.9 us, ETC2 RGBA8
+// 72.3 -> 70.9, at 12004x9000 106.5 -> 103.4, image sums 94.5 -> 93.5.
+constexpr uint32_t kQualityOrder = 6;
+
 // A wave's tiles first, first + step, ... in a grid-stride loop, one tile at a
 // time (48-65 VGPRs, so that all of the grid's 6 waves per SIMD fit).  Loading
 // the next tile into a second register set before comparing this one needs
@@ -315,7 +325,7 @@ __device__ __forceinline__ void sqerr_loop(const uint8_t* __restrict__ blocks, c
 {
     const uint32_t step = gridDim.x * 256u;  // nblocks <= kQualityMaxLaunchUnits < 2^30: no overflow below
     const uint32_t lane = threadIdx.x & 63u;
-    uint32_t t = __builtin_amdgcn_readfirstlane(blockIdx.x * 256u + (threadIdx.x & ~63u));
+    uint32_t t = __builtin_amdgcn_readfirstlane(xcd_workgroup(kQualityOrder) * 256u + (threadIdx.x & ~63u));
     for (; t < nblocks; t += step) {
         QTile a;
         load_qtile<FMT, NEAR>(blocks, src, pitch, bw, nblocks, magic, t, lane, a);
@@ -350,7 +360,7 @@ __global__ __launch_bounds__(256) void k_sqerr_images(const uint8_t* __restrict_
                                                       uint32_t nquads, uint64_t magic, const QualityDest dest)
 {
     ErrSums acc = {};
-    for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < nquads; i += (uint64_t)gridDim.x * 256u) {
+    for (uint64_t i = (uint64_t)xcd_workgroup(kQualityOrder) * 256u + threadIdx.x; i < nquads; i += (uint64_t)gridDim.x * 256u) {
         const uint32_t y = (uint32_t)((i * magic) >> 40), x = (uint32_t)i - y * qw;
         const u32x4 va =
             __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a + (uint64_t)y * pitch_a + (uint64_t)x * 16u));
@@ -417,9 +427,9 @@ __device__ __forceinline__ uint32_t rgb565_cell(uint32_t p, uint32_t q, uint32_t
 // One lane per 4 pixels x 2 rows (two cells): 32 bytes in, 32 bytes out.
 __global__ __launch_bounds__(256) void k_rgb565_baseline(const uint8_t* __restrict__ src, uint64_t src_pitch,
                                                          uint8_t* __restrict__ dst, uint64_t dst_pitch, uint32_t qw,
-                                                         uint32_t nunits, uint64_t magic)
+                                                         uint32_t nunits, uint64_t magic, uint32_t order)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_workgroup(order) * 256u + threadIdx.x;
     if (i >= nunits) return;
     const uint32_t ry = (uint32_t)(((uint64_t)i * magic) >> 40), x = i - ry * qw;
     const uint8_t* s0 = src + (uint64_t)(2u * ry) * src_pitch + (uint64_t)x * 16u;
@@ -435,20 +445,54 @@ __global__ __launch_bounds__(256) void k_rgb565_baseline(const uint8_t* __restri
 
 }  // namespace
 
+template <int FMT>
+static void decode_go(int store, dim3 grid, hipStream_t stream, const uint8_t* blocks, uint8_t* dst, uint64_t pitch,
+                      uint32_t bw, uint32_t nblocks, uint64_t magic)
+{
+    const auto go = [&](auto kernel) {  // runs of 64 workgroups per XCD
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, blocks, dst, pitch, bw, nblocks, magic, 7u);
+    };
+    if (store == kStreamThrough) go(k_decode<FMT, kStreamThrough>);
+    else if (store == kCached) go(k_decode<FMT, kCached>);
+    else go(k_decode<FMT, kStream>);
+}
+
+// How a decode stores depends on how its rows lie on the 64-byte sectors.
+//   Rows on sectors: every store fills whole sectors, and writing them through
+// is fastest.  Other rows: neighbouring waves share a sector at their ends,
+// which their XCD's L2 has to bring together, so runs of workgroups per XCD and
+// no writing through; cached stores keep more of them together, but only
+// images too large to lie in the last-level cache gain by that.  Measured in us
+// (BC1 / ETC2 RGBA8), streaming in linear order -> as chosen here: 2048^2
+// 5.2 / 5.7 -> 4.2 / 4.5, 4096^2 13.8 / 15.7 -> 12.2 / 14.9, 8192^2 47.2 / 53.9
+// -> 45.8 / 52.9, with a pitch of 32896 55.3 / 59.7 -> 46.6 / 53.2; rows off the
+// sectors 3076^2 10.3 / 11.3 -> 9.8 / 10.9, 6004^2 36.9 / 35.9 -> 31.9 / 34.4,
+// 8196x8192 64.9 / 62.2 -> 54.4 / 57.8.  Cached against streaming there, both in
+// runs: 3076^2 10.1 / 11.7 and 9.8 / 10.9, 4100^2 14.6 / 17.2 and 15.3 / 17.1,
+// 6004^2 31.9 / 34.6 and 34.6 / 34.4, 7004^2 42.5 / 43.9 and 47.7 / 45.5; written
+// through at 8196x8192 61.4 / 67.6.
+static int decode_store(int fmt, const void* dst, size_t pitch, uint32_t height)
+{
+    if (pitch % 64 == 0 && (uintptr_t)dst % 64 == 0) return kStreamThrough;
+    const size_t large = fmt < 2 ? (size_t)64 << 20 : (size_t)160 << 20;
+    return pitch * height >= large ? kCached : kStream;
+}
+
 hipError_t launch_decode(int fmt, const void* blocks, void* dst, uint32_t width, uint32_t height, size_t pitch,
                          hipStream_t stream)
 {
     const uint32_t bw = width / 4, nblocks = bw * (height / 4);
     if (nblocks == 0) return hipSuccess;
-    const dim3 grid((nblocks + 255u) / 256u), block(256);
+    const dim3 grid((nblocks + 255u) / 256u);
     const uint64_t magic = div_magic(bw);
     const uint8_t* b = static_cast<const uint8_t*>(blocks);
     uint8_t* d = static_cast<uint8_t*>(dst);
+    const int store = decode_store(fmt, dst, pitch, height);
     switch (fmt) {
-    case 0: hipLaunchKernelGGL(k_decode<0>, grid, block, 0, stream, b, d, (uint64_t)pitch, bw, nblocks, magic); break;
-    case 1: hipLaunchKernelGGL(k_decode<1>, grid, block, 0, stream, b, d, (uint64_t)pitch, bw, nblocks, magic); break;
-    case 2: hipLaunchKernelGGL(k_decode<2>, grid, block, 0, stream, b, d, (uint64_t)pitch, bw, nblocks, magic); break;
-    default: hipLaunchKernelGGL(k_decode<3>, grid, block, 0, stream, b, d, (uint64_t)pitch, bw, nblocks, magic);
+    case 0: decode_go<0>(store, grid, stream, b, d, pitch, bw, nblocks, magic); break;
+    case 1: decode_go<1>(store, grid, stream, b, d, pitch, bw, nblocks, magic); break;
+    case 2: decode_go<2>(store, grid, stream, b, d, pitch, bw, nblocks, magic); break;
+    default: decode_go<3>(store, grid, stream, b, d, pitch, bw, nblocks, magic);
     }
     return hipGetLastError();
 }
@@ -497,12 +541,16 @@ hipError_t launch_rgb565_baseline(const void* src, size_t src_pitch, void* dst, 
     const uint32_t qw = width / 4, n = qw * (height / 2);
     if (n == 0) return hipSuccess;
     const dim3 grid((n + 255u) / 256u), block(256);
+    // Rows off the 128-byte lines in runs of 32 workgroups per XCD: 4100x3076
+    // 19.0 -> 18.5 us, 8196x8192 88.9 -> 88.2; rows on them were up to 2% slower so
+    // (8192^2 81.4 -> 83.3).
+    const uint32_t order = src_pitch % 128 != 0 || dst_pitch % 128 != 0 ? 6u : 0u;
     if (start || stop)
         hipExtLaunchKernelGGL(k_rgb565_baseline, grid, block, 0, stream, start, stop, 0, (const uint8_t*)src,
-                              (uint64_t)src_pitch, (uint8_t*)dst, (uint64_t)dst_pitch, qw, n, div_magic(qw));
+                              (uint64_t)src_pitch, (uint8_t*)dst, (uint64_t)dst_pitch, qw, n, div_magic(qw), order);
     else
         hipLaunchKernelGGL(k_rgb565_baseline, grid, block, 0, stream, (const uint8_t*)src, (uint64_t)src_pitch,
-                           (uint8_t*)dst, (uint64_t)dst_pitch, qw, n, div_magic(qw));
+                           (uint8_t*)dst, (uint64_t)dst_pitch, qw, n, div_magic(qw), order);
     return hipGetLastError();
 }
 

@@ -173,6 +173,38 @@ def test_decode_and_quality_address_paths(gpu, oracle, w, h, pitch):
         dst.free()
 
 
+@pytest.mark.parametrize("fmt", [W.DXT1, W.ETC1, W.DXT5, W.ETC2])
+@pytest.mark.parametrize("w,h,pad,offset", [(1024, 272, 0, 0), (1040, 272, 0, 0), (1028, 272, 0, 0), (1024, 272, 48, 0),
+                                            (1024, 272, 0, 16), (256, 1028, 64, 32), (4100, 4100, 0, 0),
+                                            (6500, 6500, 0, 16)])
+def test_decode_stores_by_row_alignment(gpu, w, h, pad, offset, fmt):
+    """The decoders' stores follow the rows' alignment (pitch and base on 64
+    bytes or not) and, off it, the image's size; workgroups go to the XCDs in
+    runs, with a last run that is incomplete.  Each against decodes of strips
+    of 64 block rows into a tight image of its own, and nothing written
+    between or after the rows."""
+    from goofy_amd import hip
+    pitch, bb = w * 4 + pad, gpu.block_bytes(fmt)
+    print(f"decode stores {w}x{h} pitch {pitch} offset {offset} fmt {fmt}", flush=True)
+    rng = np.random.default_rng(w + fmt)
+    row = (w // 4) * bb
+    enc = rng.integers(0, 256, row * (h // 4), dtype=np.uint8)
+    blocks = hip.DeviceBuffer.from_array(enc)
+    dst = hip.DeviceBuffer(pitch * h + 4096, fill=0xA5)
+    gpu.decode_device(fmt, dst.view(offset, pitch * h), blocks, w, h, pitch)
+    hip.synchronize()
+    got = dst.download()
+    assert (got[:offset] == 0xA5).all() and (got[offset + pitch * h:] == 0xA5).all()
+    rows = got[offset:offset + pitch * h].reshape(h, pitch)
+    assert (rows[:, w * 4:] == 0xA5).all()
+    strip = hip.DeviceBuffer(w * 4 * 256)
+    for y in range(0, h, 256) if h <= 1028 else (0, h // 8 * 4, (h - 256) // 4 * 4):
+        n = min(256, h - y)
+        gpu.decode_device(fmt, strip, blocks.view(y // 4 * row, n // 4 * row), w, n)
+        hip.synchronize()
+        assert np.array_equal(rows[y:y + n, :w * 4].reshape(-1), strip.download(w * 4 * n)), y
+
+
 def integer_sums(src, dec):
     """The round-trip sums in integers: squared error of bytes 0..3, and
     10^4 x the harness's luma error sum (its weights 0.21 / 0.72 / 0.07 on
