@@ -24,6 +24,11 @@ HIPCC_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "-shared", f"--offload-arch={ARCH}",
     # packed FP32 instructions stay off in all device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # the first 14 words of a kernel's arguments are in scalar registers when a
+    # wave starts (14: what 16 user registers hold beside the arguments'
+    # address), instead of scalar loads at the head of every wave:
+    # 0.4 us of a 5 us kernel, 1% of a decode at 8192^2
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-Wall", "-Wno-unused-result", "-Wno-unused-command-line-argument",
     "-fvisibility=hidden", "-pthread",
 ]

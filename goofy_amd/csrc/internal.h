@@ -50,6 +50,9 @@ inline uint32_t order_arg(const LaunchCfg& c)
     return c.tile_order ? 1u + (uint32_t)__builtin_ctz(kXcdRunTiles / (uint32_t)c.wg_waves) : 0u;
 }
 
+// The one-image kernels' shape argument: that, and the waves per workgroup from bit 8 up.
+inline uint32_t shape_arg(const LaunchCfg& c) { return order_arg(c) | (uint32_t)c.wg_waves << 8; }
+
 inline LaunchCfg to_cfg(const goofy_launch_config& u)
 {
     return LaunchCfg{u.blocks_per_lane, u.wg_waves, u.waves_per_cu, u.nontemporal, u.tile_order};

@@ -156,28 +156,28 @@ __device__ __forceinline__ void encode_tile(const uint8_t* __restrict__ src, uin
 }
 
 // Index of this wave in the launch, with the workgroups renumbered by `order`
-// (xcd_workgroup in tile_io.h).
-// wpg = waves per workgroup.  The batch kernels take it as an argument; the
-// others read blockDim.x, a 16-bit field of the dispatch packet, which this
-// target reads with a vector load at the head of every wave.  Measured both
-// ways: on the DXT1 / ETC1S kernels at 8192^2 (HBM-bound) the read is 2%
-// faster than the argument, and no different on the alpha ones; on the
-// 4096-texture batch, whose waves first search the work-list, the argument is
-// 2-3% faster.
+// (xcd_workgroup in tile_io.h).  wpg = waves per workgroup, an argument and
+// not blockDim.x: that is a 16-bit field in memory, which this target reads
+// with a vector load at the head of every wave, while the arguments are in
+// scalar registers when the wave starts (build.py asks for them).  Both ways,
+// with arguments so preloaded: ETC1S 3000x2052 5.8 -> 5.2 us per call, DXT1
+// 8192^2 46.2 -> 45.9; preloading without this, or this without preloading,
+// 5.8 and 5.4 us on the first, 5.6 with neither.
 __device__ __forceinline__ uint32_t wave_index(uint32_t order, uint32_t wpg)
 {
     return __builtin_amdgcn_readfirstlane(xcd_workgroup(order) * wpg + (threadIdx.x >> 6));
 }
 
-__device__ __forceinline__ uint32_t wave_index(uint32_t order) { return wave_index(order, blockDim.x >> 6); }
+// The same from the one argument of shape_arg().
+__device__ __forceinline__ uint32_t wave_index(uint32_t shape) { return wave_index(shape & 0xFFu, shape >> 8); }
 
 // One image; wave w encodes tile w.
 template <int FMT, int BPL, bool NT>
 __global__ __launch_bounds__(512) void k_encode_plain(const uint8_t* __restrict__ src, uint64_t pitch,
                                                       uint8_t* __restrict__ dst, uint32_t bw, uint32_t nblocks,
-                                                      uint64_t magic, uint32_t order)
+                                                      uint64_t magic, uint32_t shape)
 {
-    const uint32_t wave = wave_index(order);
+    const uint32_t wave = wave_index(shape);
     encode_tile<FMT, BPL, NT>(src, pitch, dst, bw, magic, nblocks, wave * 64u * BPL, threadIdx.x & 63u);
 }
 
@@ -215,9 +215,9 @@ __device__ __forceinline__ void encode_pair_tile(const uint8_t* __restrict__ src
 // One image into both 8-byte formats, one block per lane.
 __global__ __launch_bounds__(512) void k_encode_dual(const uint8_t* __restrict__ src, uint64_t pitch,
                                                      uint8_t* __restrict__ dst_dxt1, uint8_t* __restrict__ dst_etc1,
-                                                     uint32_t bw, uint32_t nblocks, uint64_t magic, uint32_t order)
+                                                     uint32_t bw, uint32_t nblocks, uint64_t magic, uint32_t shape)
 {
-    encode_pair_tile<false>(src, pitch, dst_dxt1, dst_etc1, bw, nblocks, magic, wave_index(order) * 64u,
+    encode_pair_tile<false>(src, pitch, dst_dxt1, dst_etc1, bw, nblocks, magic, wave_index(shape) * 64u,
                             threadIdx.x & 63u);
 }
 
@@ -225,9 +225,9 @@ __global__ __launch_bounds__(512) void k_encode_dual(const uint8_t* __restrict__
 __global__ __launch_bounds__(512) void k_encode_dual_alpha(const uint8_t* __restrict__ src, uint64_t pitch,
                                                            uint8_t* __restrict__ dst_dxt5,
                                                            uint8_t* __restrict__ dst_etc2, uint32_t bw,
-                                                           uint32_t nblocks, uint64_t magic)
+                                                           uint32_t nblocks, uint64_t magic, uint32_t shape)
 {
-    encode_pair_tile<true>(src, pitch, dst_dxt5, dst_etc2, bw, nblocks, magic, wave_index(0u) * 64u,
+    encode_pair_tile<true>(src, pitch, dst_dxt5, dst_etc2, bw, nblocks, magic, wave_index(shape) * 64u,
                            threadIdx.x & 63u);
 }
 
@@ -368,15 +368,15 @@ __global__ __launch_bounds__(256) void k_synth(goofy_synth::Params P, uint8_t* _
 // the kernel's execution, without marker packets around it.
 template <int FMT, int BPL, bool NT>
 static hipError_t plain_go(dim3 grid, dim3 block, const void* src, size_t pitch, void* dst, uint32_t bw,
-                           uint32_t nblocks, uint64_t magic, uint32_t order, hipStream_t s, hipEvent_t e0,
+                           uint32_t nblocks, uint64_t magic, uint32_t shape, hipStream_t s, hipEvent_t e0,
                            hipEvent_t e1)
 {
     if (e0 || e1)
         hipExtLaunchKernelGGL((k_encode_plain<FMT, BPL, NT>), grid, block, 0, s, e0, e1, 0, (const uint8_t*)src,
-                              (uint64_t)pitch, (uint8_t*)dst, bw, nblocks, magic, order);
+                              (uint64_t)pitch, (uint8_t*)dst, bw, nblocks, magic, shape);
     else
         hipLaunchKernelGGL((k_encode_plain<FMT, BPL, NT>), grid, block, 0, s, (const uint8_t*)src, (uint64_t)pitch,
-                           (uint8_t*)dst, bw, nblocks, magic, order);
+                           (uint8_t*)dst, bw, nblocks, magic, shape);
     return hipGetLastError();
 }
 
@@ -386,7 +386,7 @@ static hipError_t plain_bpl(const LaunchCfg& c, dim3 grid, dim3 block, const voi
                             hipEvent_t e1)
 {
     const bool nt = c.nontemporal != 0;
-    const uint32_t o = order_arg(c);
+    const uint32_t o = shape_arg(c);
     switch (c.blocks_per_lane) {
     case 1:
         return nt ? plain_go<FMT, 1, true>(grid, block, src, pitch, dst, bw, nblocks, magic, o, s, e0, e1)
@@ -441,15 +441,15 @@ hipError_t launch_dual(const LaunchCfg& c, const void* src, size_t pitch, void* 
                        uint32_t nblocks, hipStream_t stream, hipEvent_t start, hipEvent_t stop)
 {
     if (nblocks == 0) return hipSuccess;
-    const uint32_t ntiles = (nblocks + 63u) / 64u, wg = (uint32_t)c.wg_waves, order = order_arg(c);
+    const uint32_t ntiles = (nblocks + 63u) / 64u, wg = (uint32_t)c.wg_waves, shape = shape_arg(c);
     const dim3 grid((ntiles + wg - 1u) / wg), block(64u * wg);
     const uint64_t magic = div_magic(bw);
     if (start || stop)
         hipExtLaunchKernelGGL(k_encode_dual, grid, block, 0, stream, start, stop, 0, (const uint8_t*)src,
-                              (uint64_t)pitch, (uint8_t*)dst_dxt1, (uint8_t*)dst_etc1, bw, nblocks, magic, order);
+                              (uint64_t)pitch, (uint8_t*)dst_dxt1, (uint8_t*)dst_etc1, bw, nblocks, magic, shape);
     else
         hipLaunchKernelGGL(k_encode_dual, grid, block, 0, stream, (const uint8_t*)src, (uint64_t)pitch,
-                           (uint8_t*)dst_dxt1, (uint8_t*)dst_etc1, bw, nblocks, magic, order);
+                           (uint8_t*)dst_dxt1, (uint8_t*)dst_etc1, bw, nblocks, magic, shape);
     return hipGetLastError();
 }
 
@@ -457,15 +457,15 @@ hipError_t launch_dual_alpha(uint32_t wg_waves, const void* src, size_t pitch, v
                              uint32_t bw, uint32_t nblocks, hipStream_t stream, hipEvent_t start, hipEvent_t stop)
 {
     if (nblocks == 0) return hipSuccess;
-    const uint32_t ntiles = (nblocks + 63u) / 64u;
+    const uint32_t ntiles = (nblocks + 63u) / 64u, shape = wg_waves << 8;
     const dim3 grid((ntiles + wg_waves - 1u) / wg_waves), block(64u * wg_waves);
     const uint64_t magic = div_magic(bw);
     if (start || stop)
         hipExtLaunchKernelGGL(k_encode_dual_alpha, grid, block, 0, stream, start, stop, 0, (const uint8_t*)src,
-                              (uint64_t)pitch, (uint8_t*)dst_dxt5, (uint8_t*)dst_etc2, bw, nblocks, magic);
+                              (uint64_t)pitch, (uint8_t*)dst_dxt5, (uint8_t*)dst_etc2, bw, nblocks, magic, shape);
     else
         hipLaunchKernelGGL(k_encode_dual_alpha, grid, block, 0, stream, (const uint8_t*)src, (uint64_t)pitch,
-                           (uint8_t*)dst_dxt5, (uint8_t*)dst_etc2, bw, nblocks, magic);
+                           (uint8_t*)dst_dxt5, (uint8_t*)dst_etc2, bw, nblocks, magic, shape);
     return hipGetLastError();
 }
 
