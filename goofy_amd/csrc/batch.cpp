@@ -278,7 +278,7 @@ int goofy_batch_launch_per_texture(goofy_batch* b, void* stream)
         for (uint32_t y0 = 0; y0 < bh;) {
             const uint32_t rows = std::min(max_rows, bh - y0);
             const uint32_t nb = rows * bw;
-            const LaunchCfg c = plain_cfg(t.format, nb, b->num_cus);
+            const LaunchCfg c = wide_cfg(nb, b->num_cus);
             hipError_t e = launch_plain(t.format, c, static_cast<const uint8_t*>(t.src) + (size_t)y0 * 4 * t.pitch,
                                         t.pitch, static_cast<uint8_t*>(t.dst) + (size_t)y0 * bw * block_bytes(t.format),
                                         bw, nb, (hipStream_t)stream);

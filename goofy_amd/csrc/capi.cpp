@@ -75,16 +75,13 @@ int device_info(DeviceInfo* out)
     return GOOFY_OK;
 }
 
-// Measured on MI355X (8192^2, both formats): one block per lane with
-// streaming (non-temporal) loads and stores is fastest; 1-4 wave workgroups
-// are within noise of each other, 4 blocks per lane loses ~10%.  Large launches
-// into the 8-byte formats and batches start from this in wide_cfg.
-// One block per lane, streaming, linear tile order, and the largest
-// workgroup (8, 4, 2 or 1 waves) that still leaves two workgroups per CU.
-// 8-wave workgroups are the fastest shape on large images (on the 8192^2
-// image within 1% of the other one-block-per-lane shapes, on 16384^2 images
-// with a 65792-byte pitch 20-25% faster than 2-wave ones); a texture of a
-// few hundred tiles needs smaller workgroups to reach every CU.
+// The shape of small and middling launches, and what wide_cfg starts from for
+// large ones: one block per lane (4 lose ~10% at 8192^2), streaming loads and
+// stores, linear tile order, and the largest workgroup (8, 4, 2 or 1 waves)
+// that still leaves two workgroups per CU: up to 8192 tiles 8-wave workgroups
+// are the fastest linear shape (3000x2052 DXT1 5.7 us, 5.8 / 5.9 / 6.0 in 4- /
+// 2- / 1-wave ones), while a texture of a few hundred tiles needs smaller ones
+// to reach every CU.
 LaunchCfg auto_cfg(uint64_t blocks, int num_cus)
 {
     const uint64_t tiles = (blocks + 63u) / 64u;
@@ -266,7 +263,7 @@ static hipError_t launch_any(int fmt, const LaunchCfg& cfg, const void* in, size
                              uint32_t bw, uint32_t nblocks, hipStream_t stream)
 {
     return fmt == kFeedDualAlpha
-               ? launch_dual_alpha((uint32_t)cfg.wg_waves, in, row_bytes, out, out2, bw, nblocks, stream)
+               ? launch_dual_alpha(cfg, in, row_bytes, out, out2, bw, nblocks, stream)
            : fmt == kFeedDual ? launch_dual(cfg, in, row_bytes, out, out2, bw, nblocks, stream)
                               : launch_plain(fmt, cfg, in, row_bytes, out, bw, nblocks, stream);
 }
@@ -457,7 +454,7 @@ static int compress_device(int fmt, void* d_result, const void* d_input, unsigne
     for (uint32_t y0 = 0; y0 < bh;) {
         const uint32_t rows = std::min(max_rows, bh - y0);
         const uint32_t nb = rows * bw;  // <= 0xFFFFFFFF by max_stripe_brows
-        const LaunchCfg c = ucfg ? cfg : plain_cfg(fmt, nb, num_cus);
+        const LaunchCfg c = ucfg ? cfg : wide_cfg(nb, num_cus);
         hipError_t e = launch_plain(fmt, c, static_cast<const uint8_t*>(d_input) + (size_t)y0 * 4 * pitch, pitch,
                                     static_cast<uint8_t*>(d_result) + (size_t)y0 * bw * bb, bw, nb,
                                     (hipStream_t)stream, y0 == 0 ? (hipEvent_t)ev_start : nullptr,
@@ -600,10 +597,9 @@ static int compress_device_pair(bool alpha, void* d_a, void* d_b, const void* d_
         uint8_t* b = static_cast<uint8_t*>(d_b) + out_off;
         hipEvent_t e0 = y0 == 0 ? (hipEvent_t)start_event : nullptr;
         hipEvent_t e1 = y0 + rows == bh ? (hipEvent_t)stop_event : nullptr;
-        hipError_t e = alpha ? launch_dual_alpha((uint32_t)auto_cfg(nb, di.num_cus).wg_waves, in, pitch, a, b, bw, nb,
-                                                 (hipStream_t)stream, e0, e1)
-                             : launch_dual(wide_cfg(nb, di.num_cus), in, pitch, a, b, bw, nb, (hipStream_t)stream, e0,
-                                           e1);
+        const LaunchCfg c = wide_cfg(nb, di.num_cus);
+        hipError_t e = alpha ? launch_dual_alpha(c, in, pitch, a, b, bw, nb, (hipStream_t)stream, e0, e1)
+                             : launch_dual(c, in, pitch, a, b, bw, nb, (hipStream_t)stream, e0, e1);
         if (e != hipSuccess) return fail_hip(e, "dual encode kernel launch");
         y0 += rows;
     }

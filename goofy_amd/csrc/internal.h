@@ -110,7 +110,7 @@ hipError_t launch_plain(int fmt, const LaunchCfg& cfg, const void* src, size_t p
 // cfg: workgroup size and tile order (one block per lane, streaming).
 hipError_t launch_dual(const LaunchCfg& cfg, const void* src, size_t pitch, void* dst_dxt1, void* dst_etc1, uint32_t bw,
                        uint32_t nblocks, hipStream_t stream, hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
-hipError_t launch_dual_alpha(uint32_t wg_waves, const void* src, size_t pitch, void* dst_dxt5, void* dst_etc2,
+hipError_t launch_dual_alpha(const LaunchCfg& cfg, const void* src, size_t pitch, void* dst_dxt5, void* dst_etc2,
                              uint32_t bw, uint32_t nblocks, hipStream_t stream, hipEvent_t start = nullptr,
                              hipEvent_t stop = nullptr);
 // The drop-in's kernel, which encodes an image in pinned host memory while
@@ -239,33 +239,30 @@ inline int tile_blocks(const LaunchCfg& c) { return 64 * c.blocks_per_lane; }
 // Default launch shape for a launch of `blocks` 4x4 blocks on a device with
 // num_cus compute units (used wherever the caller gives no shape).
 LaunchCfg auto_cfg(uint64_t blocks, int num_cus);
-// The default for a launch that reads large amounts of pixels and is bound by
-// that: batches, and images into the 8-byte formats.  Above 64 MiB of pixels
-// (16384 tiles) tiles go to the XCDs in runs, in workgroups of 4 waves, or 8
-// from 1 GiB on; smaller launches keep auto_cfg's shape.  Measured in us per
-// launch, linear order in 8-wave workgroups -> this: batches of 128 / 1024 /
-// 4096 textures 34.6 -> 32.6, 282 -> 262, 1090 -> 1006; DXT1 6000x4000
-// 18.9 -> 18.8, 8192^2 47.9 -> 46.9, 16384^2 189.5 -> 178.5 (its 65792-byte
-// pitch 195.9 -> 187.2), DXT1 + ETC1S 8192^2 54.7 -> 52.7; but 4096^2
-// 13.4 -> 13.8 and 2048^2 5.0 -> 5.4.  A 2048-texture batch of 660k tiles took
-// 478 us in 8-wave workgroups and 490 in 4-wave ones, an 8192^2 image 47.1 and
-// 46.9.
+// The default of every encode launch on device memory.  Above 32 MiB of
+// pixels (8192 tiles), where loads bound the kernel, tiles go to the XCDs in
+// runs, in workgroups of 4 waves, or 8 from 1 GiB on; smaller launches keep
+// auto_cfg's shape.  Measured in us per launch, linear order in 8-wave
+// workgroups -> runs in 4-wave ones, per format (DXT1, ETC1S, DXT5, ETC2) and
+// pair (DXT1 + ETC1S, DXT5 + ETC2):
+//   3400^2        9.4   9.5  10.7  11.5  10.3  15.0 ->   8.8   8.8  10.3  11.2  10.1  14.3
+//   4096^2       12.9  13.1  14.2  15.0  14.8  19.1 ->  12.3  12.4  14.1  14.9  14.2  18.9
+//   8192^2       48.9  49.1  53.4  54.2  54.7  65.8 ->  46.0  46.0  51.5  54.1  52.3  65.5
+//   12004x9000   80.0  80.3  86.4  90.2   -   108.2 ->  75.5  74.8  82.6  87.5  85.4 105.2
+//   16384^2     192.3 192.2 209.8 209.4   -   246.1 -> 187.2 184.9 206.5 212.2 208.0 245.9
+// and batches: 16 textures of 8.7k tiles 9.8 -> 8.9, 256 of 11.5k 10.8 -> 10.2,
+// 1024 282 -> 262, 4096 1090 -> 1006.  Below, 3000x2052 (6011 tiles) loses 2%.
+// From 262144 tiles 4 and 8 waves are alike on images; a 2048-texture batch of
+// 660k tiles took 478 us in 8-wave workgroups and 490 in 4-wave ones.
 inline LaunchCfg wide_cfg(uint64_t blocks, int num_cus)
 {
     LaunchCfg c = auto_cfg(blocks, num_cus);
     const uint64_t tiles = (blocks + 63u) / 64u;
-    if (tiles > 16384u) {
+    if (tiles > 8192u) {
         c.wg_waves = tiles < 262144u ? 4 : 8;
         c.tile_order = 1;
     }
     return c;
-}
-// The default for one image of a format.  The 16-byte formats, half bound by
-// their arithmetic, gained up to 3% from runs at some sizes and lost 2% at
-// others: they stay linear.
-inline LaunchCfg plain_cfg(int format, uint64_t blocks, int num_cus)
-{
-    return format >= GOOFY_FORMAT_DXT5 ? auto_cfg(blocks, num_cus) : wide_cfg(blocks, num_cus);
 }
 bool cfg_valid(const LaunchCfg& c);
 

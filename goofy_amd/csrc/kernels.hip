@@ -453,12 +453,12 @@ hipError_t launch_dual(const LaunchCfg& c, const void* src, size_t pitch, void* 
     return hipGetLastError();
 }
 
-hipError_t launch_dual_alpha(uint32_t wg_waves, const void* src, size_t pitch, void* dst_dxt5, void* dst_etc2,
+hipError_t launch_dual_alpha(const LaunchCfg& c, const void* src, size_t pitch, void* dst_dxt5, void* dst_etc2,
                              uint32_t bw, uint32_t nblocks, hipStream_t stream, hipEvent_t start, hipEvent_t stop)
 {
     if (nblocks == 0) return hipSuccess;
-    const uint32_t ntiles = (nblocks + 63u) / 64u, shape = wg_waves << 8;
-    const dim3 grid((ntiles + wg_waves - 1u) / wg_waves), block(64u * wg_waves);
+    const uint32_t ntiles = (nblocks + 63u) / 64u, wg = (uint32_t)c.wg_waves, shape = shape_arg(c);
+    const dim3 grid((ntiles + wg - 1u) / wg), block(64u * wg);
     const uint64_t magic = div_magic(bw);
     if (start || stop)
         hipExtLaunchKernelGGL(k_encode_dual_alpha, grid, block, 0, stream, start, stop, 0, (const uint8_t*)src,

@@ -269,7 +269,7 @@ bool goofy_server::launch_group(Slot& s, std::vector<Req>& group)
     } else {
         for (Req& q : group) {
             const uint32_t bw = q.r.width / 4, nb = bw * (q.r.height / 4);
-            e = launch_plain(q.r.format, auto_shape ? plain_cfg(q.r.format, nb, num_cus) : launch, q.r.src, q.r.pitch,
+            e = launch_plain(q.r.format, auto_shape ? wide_cfg(nb, num_cus) : launch, q.r.src, q.r.pitch,
                              arena.base() + q.arena_off, bw, nb, s.stream);
             if (e != hipSuccess) break;
         }

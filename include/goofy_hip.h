@@ -130,8 +130,8 @@ typedef struct goofy_launch_config {
 /* As goofy_hip_compress_device with an explicit launch shape.  NULL = the
  * default shape, sized to the launch: one block per lane, streaming loads and
  * stores, linear tile order, and the largest workgroup of 8, 4, 2 or 1 waves
- * that still gives at least two workgroups per CU; for DXT1 and ETC1S above 64
- * MiB of pixels tile order 1, in workgroups of 4 waves, or 8 from 1 GiB on. */
+ * that still gives at least two workgroups per CU; above 32 MiB of pixels tile
+ * order 1, in workgroups of 4 waves, or 8 from 1 GiB on. */
 GOOFY_HIP_API int goofy_hip_compress_device_cfg(int format, void* d_result, const void* d_input, unsigned int width,
                                                 unsigned int height, size_t pitch, void* stream,
                                                 const goofy_launch_config* cfg);

@@ -375,6 +375,32 @@ def test_runs_per_xcd_match_linear_order(gpu, w, h):
         assert np.array_equal(a.download(), want[0]) and np.array_equal(b.download(), want[1]), cfg
 
 
+@pytest.mark.parametrize("w,h", [(2048, 4096), (2052, 4096), (2900, 2996)])
+def test_runs_per_xcd_16_byte_formats(gpu, w, h):
+    """Above 8192 tiles of 64 blocks runs per XCD are the default shape of
+    every format and pair: the last size below, one above with an incomplete
+    span, and a ragged one, against the linear order."""
+    say(f"runs per XCD, 16-byte formats {w}x{h}: {(w // 4) * (h // 4) / 64:.1f} tiles")
+    from goofy_amd import hip
+    src = dev_buffer(w * h * 4)
+    gpu.synth_device(2, 78, 0, 12, src, w, h)
+    a, b = dev_buffer((w // 4) * (h // 4) * 16), dev_buffer((w // 4) * (h // 4) * 16)
+    want = []
+    for fmt in (W.DXT5, W.ETC2):
+        for cfg in [dict(blocks_per_lane=1, wg_waves=8, waves_per_cu=0, nontemporal=1, tile_order=0), None]:
+            a.fill(0xCD)
+            gpu.compress_device(fmt, a, src, w, h, w * 4, config=cfg)
+            hip.synchronize()
+            if cfg:
+                want.append(a.download())
+            assert np.array_equal(a.download(), want[-1]), (fmt, cfg)
+    a.fill(0xCD)
+    b.fill(0xCD)
+    gpu.compress_device_dual_alpha(a, b, src, w, h, w * 4)
+    hip.synchronize()
+    assert np.array_equal(a.download(), want[0]) and np.array_equal(b.download(), want[1])
+
+
 def test_tune_device_picks_a_valid_shape(gpu, oracle):
     w, h, pitch = 2048, 1024, 2048 * 4 + 256
     img = gpu.synth_host(0, 99, 0, 12, w, h, pitch, fill=0)
