@@ -219,21 +219,22 @@ __device__ __forceinline__ unsigned long long block_sums(unsigned long long (&e)
 // End of a quality kernel.  With a host result (d.host) the launch finishes
 // the sums itself, one lane per word (QualityAccum): a lane adds its word and a
 // count of one with a device-scope atomic, and the lane whose returned count
-// completes the word has its total and writes it to pinned host memory.  The
-// words need no order among each other, nothing is read twice and there is no
-// fence (one per workgroup is a write-back of the whole L2: the BC1 round trip
-// of an 8192^2 image took 124 us instead of 51 with it).  The completing lane
-// leaves the word at zero for the next launch.
+// completes the word takes its total in exchange for the zero that the next
+// launch starts from, and writes it to pinned host memory, where the host waits
+// for it.  The total depends on the exchange's return, so the zero is in place
+// before the host can see the word and give the work area to another stream.
+// The words need no order among each other and there is no fence (one per
+// workgroup is a write-back of the whole L2: the BC1 round trip of an 8192^2
+// image took 124 us instead of 51 with it).
 //   Atomics on one line run one after another, about 8 ns each: 1536
 // workgroups counting on one word took 12 us.  Grids of more workgroups than
 // slots therefore add into one of 64 slots first, and the completed slots into
 // the total: 24 + 64 at most on a line.
 //   A second launch that adds the workgroups' partials (4 us and the gap before
-// it) was slower: whole calls from Python, second launch -> this, 512x512 DXT1
-// 21.0 -> 18.9 us, 8192^2 ETC1 69.1 -> 66.7, floor and image-against-image
-// figures of 4100x3076 57.5 -> 54.7; what remains of a small call is the host's
-// launch and stream synchronisation.  Integer sums: the order of the adds does
-// not show.
+// it) was slower: whole calls from Python, second launch -> this, both with a
+// stream synchronisation behind, 512x512 DXT1 21.0 -> 18.9 us, 8192^2 ETC1 69.1
+// -> 66.7, floor and image-against-image figures of 4100x3076 57.5 -> 54.7.
+// Integer sums: the order of the adds does not show.
 // Without d.host the workgroup leaves its partial for k_sums_final.
 __device__ __forceinline__ void finish_sums(unsigned long long (&e)[4], unsigned long long ey, const QualityDest& d)
 {
@@ -255,15 +256,14 @@ __device__ __forceinline__ void finish_sums(unsigned long long (&e)[4], unsigned
         unsigned long long* w = &d.accum->slot[s].word[lane];
         const unsigned long long before = __hip_atomic_fetch_add(w, v + one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if ((before >> kQualityCountBit) != in_slot - 1u) return;
-        __hip_atomic_store(w, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        v += before & (one - 1u);
+        v = __hip_atomic_exchange(w, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & (one - 1u);
         parts = kQualitySlots;
     }
     unsigned long long* w = &d.accum->total.word[lane];
     const unsigned long long before = __hip_atomic_fetch_add(w, v + one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if ((before >> kQualityCountBit) != parts - 1u) return;
-    __hip_atomic_store(w, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    d.host->word[lane] = v + (before & (one - 1u));
+    v = __hip_atomic_exchange(w, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & (one - 1u);
+    __hip_atomic_store(&d.host->word[lane], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // One wave's tile of the round trip: 64 consecutive blocks from `first`,

@@ -167,8 +167,10 @@ struct QualityAccum {
 };
 // Pinned host memory: the words of one launch, without counts.
 struct QualityHost {
-    unsigned long long word[kQualityWords];
+    uint64_t word[kQualityWords];
 };
+// A word that no launch has written yet (counts and sums stay below it).
+constexpr uint64_t kQualityNone = ~0ull;
 // A pooled call waits after this many stripes, each with a QualityHost.
 constexpr uint32_t kQualityStripes = 16;
 // Where a quality launch leaves its sums.  Pooled: the zeroed accum on the way

@@ -484,6 +484,36 @@ def test_quality_sums_finished_by_the_last_workgroup(gpu):
             assert q["sse_byte"] == sse and q["sse_luma"] == y100 / 1e4, h
 
 
+def test_quality_calls_return_when_their_words_are_written(gpu):
+    """A call waits for the sums themselves: calls in turn on two streams and
+    the default one, which hand the same work area on to each other, grids
+    below and above the number of slots; and calls behind a millisecond and
+    more of other work on their stream, for which they wait to the end."""
+    from goofy_amd import hip
+    w = 1024
+    rng = np.random.default_rng(19)
+    a, b = (rng.integers(0, 256, w * 4 * 300, dtype=np.uint8) for _ in range(2))
+    da, db = hip.DeviceBuffer.from_array(a), hip.DeviceBuffer.from_array(b)
+    want = {h: integer_sums(a[:w * 4 * h], b[:w * 4 * h])[0] for h in (1, 64, 65, 300)}
+    streams = [hip.Stream(), hip.Stream(), None]
+    for i in range(120):
+        h = (300, 65, 64, 1)[i % 4]
+        assert gpu.quality_images_device(da, db, w, h, stream=streams[i % 3])["sse_byte"] == want[h], i
+    n = 4096
+    big = hip.DeviceBuffer(n * n * 4, fill=0x55)
+    out = hip.DeviceBuffer(n * n // 2)
+    small = hip.DeviceBuffer(w * 4 * 300, fill=0x33)
+    plain = integer_sums(a, np.full(w * 4 * 300, 0x33, np.uint8))[0]
+    for s in streams:
+        print("quality behind other work", flush=True)
+        for _ in range(200):  # 12 us each
+            gpu.compress_device(0, out, big, n, n, n * 4, stream=s)
+        assert gpu.quality_images_device(da, small, w, 300, stream=s)["sse_byte"] == plain
+        assert gpu.quality_images_device(da, db, w, 65, stream=s)["sse_byte"] == want[65]
+    for s in streams[:2]:
+        s.destroy()
+
+
 def test_quality_call_refused_under_capture_leaves_no_trace(gpu):
     """A quality call cannot be captured: it reports so, and the calls after
     it, on the same kept work area, are right."""
