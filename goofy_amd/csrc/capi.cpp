@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cfloat>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -99,24 +100,40 @@ bool cfg_valid(const LaunchCfg& c)
            (c.tile_order == 0 || c.tile_order == 1);
 }
 
-// ---- host-memory drop-in: pinned staging, chunked pipeline ---------------------
+// ---- host-memory drop-in: pinned staging, read by the kernels themselves ------
 //
-// goofy::compressDXT1/ETC1 take pageable host buffers.  The image is moved in
+// goofy::compressDXT1/ETC1 take pageable host buffers.  The image goes in
 // chunks of block rows (about 8 MiB of pixels each) through three pinned
-// staging slots.  While the GPU copies chunk k in, host threads copy the rows
-// of chunk k+1 into the next slot, and the host collects the blocks of chunk
-// k-2.  Uploads go on a stream of their own, back to back: the kernel and the
-// download of a chunk wait for its upload on the other stream, and a slot is
-// refilled only after the host has collected its previous chunk, so the
-// upload stream never waits on the device.  (On a single stream each upload
-// is ordered behind the previous chunk's kernel and download; on MI355X the
-// 8192^2 call took 6.6 ms that way and 5.5 ms with the uploads apart, at the
-// link's measured host-to-device ceiling.)  Row copies of large chunks are
-// split over a small persistent thread pool.  An image of one chunk goes
-// through a fed kernel instead (encode_one_chunk).  Contexts (stream, events, device
-// and pinned buffers) come from a process-wide pool: concurrent callers never
-// share one, and nothing is freed at thread exit (the HIP runtime may already
-// be gone then).
+// staging slots.  A chunk's kernel (k_encode_fed) is launched before any of its
+// rows is staged, reads the slot over PCIe part by part as the host marks the
+// parts, writes its blocks to pinned memory over PCIe and marks them group by
+// group, so that the link runs from the first part staged to the last block,
+// and the host copies rows in and blocks out meanwhile.  Chunks alternate
+// between two streams: the next chunk's kernel is waiting when one ends.  DXT1 /
+// ETC2 RGBA8 in us per call; in the middle images up to 8 MiB with a fed kernel
+// and a stream synchronisation before the blocks were copied out, larger ones by
+// copy engines both ways (8 MiB chunks, plain kernels); on the left images up to
+// 8 MiB with a plain kernel per 512 KiB staged:
+//     64x64      18 / 18     ->    17 / 17     ->    14 / 15
+//    512x512     55 / 59     ->    45 / 49     ->    38 / 40
+//   1440x1448   274 / 328    ->   227 / 274    ->   194 / 200
+//   2048x2048   490 / 532    ->   494 / 535    ->   408 / 410
+//   4096x4096  1485 / 1540   ->  1490 / 1545   ->  1385 / 1410
+//   8192x8192  5455 / 5860   ->  5450 / 5820   ->  5140 / 5180
+// The kernels read 52 GB/s over the link.  With the first chunk fed and copy
+// engines for the others the calls were bound by the host (4096x4096 1473 /
+// 1617, 8192x8192 5530 / 6790).
+//   A slot is refilled after its chunk's blocks are collected.  Between a fed
+// launch and the mark of the chunk's last part the host calls nothing that
+// could wait for the device, so the kernel's wait ends whatever other threads
+// and streams do.  Should this thread stand still for `patience` ticks, the
+// kernel ends unfinished, and the chunk, all staged by then, is encoded by a
+// plain launch.  Images below 128 KiB are staged first: a look at a mark over
+// PCIe costs more than it hides there; so is every chunk where a launch returns
+// only after its kernel.
+//   Contexts (streams, events, pinned buffers) come from a process-wide pool:
+// concurrent callers never share one, and nothing is freed at thread exit (the
+// HIP runtime may already be gone then).
 
 constexpr int kSlots = 3;
 constexpr uint64_t kFeedPatience = 2000000;  // 20 ms in 10 ns ticks
@@ -133,17 +150,15 @@ static bool launches_block()
 
 struct StagingCtx {
     int device = -1;
-    hipStream_t stream = nullptr;     // kernels and downloads
-    hipStream_t in_stream = nullptr;  // uploads
-    hipEvent_t h2d_done[kSlots] = {};   // upload of the slot's chunk finished
-    hipEvent_t out_ready[kSlots] = {};  // pinned output slot holds a finished chunk
-    void* d_in[kSlots] = {};
-    void* d_out[kSlots] = {};
-    void* h_in[kSlots] = {};
-    void* h_out[kSlots] = {};
+    hipStream_t stream[2] = {};
+    hipEvent_t ended[2] = {};
+    struct Slot {
+        uint8_t* in = nullptr;     // staged rows
+        uint8_t* out = nullptr;    // blocks, a pair's second format behind the first
+        HostFeed* feed = nullptr;  // the marks of the slot's parts and groups
+    } slot[kSlots];
     size_t in_cap = 0, out_cap = 0;
-    HostFeed* feed = nullptr;     // fed kernels: the marks of the parts,
-    uint64_t call = 0;            // the number of the last launch
+    uint64_t call = 0;  // the number of the last launch
     bool stage_first = launches_block();
 };
 
@@ -182,40 +197,31 @@ static StagingPool& staging_pool()
 static int ensure_ctx(StagingCtx* c, size_t in_bytes, size_t out_bytes)
 {
     hipError_t e;
-    if (!c->stream) {
-        if ((e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess ||
-            (e = hipStreamCreateWithFlags(&c->in_stream, hipStreamNonBlocking)) != hipSuccess)
+    for (int i = 0; i < 2; ++i) {
+        if (!c->stream[i] && (e = hipStreamCreateWithFlags(&c->stream[i], hipStreamNonBlocking)) != hipSuccess)
             return fail_hip(e, "hipStreamCreate");
-        for (int i = 0; i < kSlots; ++i) {
-            if ((e = hipEventCreateWithFlags(&c->h2d_done[i], hipEventDisableTiming)) != hipSuccess ||
-                (e = hipEventCreateWithFlags(&c->out_ready[i], hipEventDisableTiming)) != hipSuccess)
-                return fail_hip(e, "hipEventCreate");
-        }
-    }
-    if (!c->feed) {
-        if ((e = hipHostMalloc((void**)&c->feed, sizeof(HostFeed), hipHostMallocCoherent)) != hipSuccess)
-            return fail_hip(e, "hipHostMalloc(staging)");
-        *c->feed = HostFeed{};
+        if (!c->ended[i] && (e = hipEventCreateWithFlags(&c->ended[i], hipEventDisableTiming)) != hipSuccess)
+            return fail_hip(e, "hipEventCreate");
     }
     if (c->in_cap < in_bytes || c->out_cap < out_bytes) {
-        (void)hipStreamSynchronize(c->in_stream);
-        (void)hipStreamSynchronize(c->stream);
+        for (hipStream_t s : c->stream) (void)hipStreamSynchronize(s);
         const size_t ni = std::max(in_bytes, c->in_cap), no = std::max(out_bytes, c->out_cap);
-        for (int i = 0; i < kSlots; ++i) {
-            if (c->d_in[i]) (void)hipFree(c->d_in[i]);
-            if (c->d_out[i]) (void)hipFree(c->d_out[i]);
-            if (c->h_in[i]) (void)hipHostFree(c->h_in[i]);
-            if (c->h_out[i]) (void)hipHostFree(c->h_out[i]);
-            c->d_in[i] = c->d_out[i] = c->h_in[i] = c->h_out[i] = nullptr;
+        for (StagingCtx::Slot& s : c->slot) {
+            if (s.in) (void)hipHostFree(s.in);
+            if (s.out) (void)hipHostFree(s.out);
+            s.in = s.out = nullptr;
         }
         c->in_cap = c->out_cap = 0;
-        for (int i = 0; i < kSlots; ++i) {
-            if ((e = hipMalloc(&c->d_in[i], ni)) != hipSuccess || (e = hipMalloc(&c->d_out[i], no)) != hipSuccess)
-                return fail_hip(e, "hipMalloc(staging)");
-            // coherent: a fed kernel reads rows that are written while it runs
-            if ((e = hipHostMalloc(&c->h_in[i], ni, hipHostMallocCoherent)) != hipSuccess ||
-                (e = hipHostMalloc(&c->h_out[i], no, hipHostMallocCoherent)) != hipSuccess)
+        for (StagingCtx::Slot& s : c->slot) {
+            // coherent: kernels and host read and write it while both run
+            if ((e = hipHostMalloc((void**)&s.in, ni, hipHostMallocCoherent)) != hipSuccess ||
+                (e = hipHostMalloc((void**)&s.out, no, hipHostMallocCoherent)) != hipSuccess)
                 return fail_hip(e, "hipHostMalloc(staging)");
+            if (!s.feed) {
+                if ((e = hipHostMalloc((void**)&s.feed, sizeof(HostFeed), hipHostMallocCoherent)) != hipSuccess)
+                    return fail_hip(e, "hipHostMalloc(staging)");
+                *s.feed = HostFeed{};
+            }
         }
         c->in_cap = ni;
         c->out_cap = no;
@@ -223,28 +229,15 @@ static int ensure_ctx(StagingCtx* c, size_t in_bytes, size_t out_bytes)
     return GOOFY_OK;
 }
 
-// Copy `rows` rows of `row_bytes` from src (stride) to dst (packed), split
-// over the copy pool when large.
-static void copy_rows(uint8_t* dst, const uint8_t* src, size_t stride, size_t row_bytes, unsigned rows)
+// Copy `rows` rows of `row_bytes` from src (stride) to dst (packed).
+static void copy_rows(uint8_t* dst, const uint8_t* src, size_t stride, size_t row_bytes, size_t rows)
 {
-    const size_t total = row_bytes * rows;
-    CopyPool& pool = CopyPool::get();
-    const int parts = total >= (2u << 20) ? std::min<int>(pool.workers() + 1, (int)std::max<size_t>(1, total >> 20)) : 1;
-    if (stride == row_bytes) {
-        const size_t step = (total + parts - 1) / parts;
-        pool.run(parts, [&](int i) {
-            const size_t a = (size_t)i * step, b = std::min(total, a + step);
-            if (a < b) std::memcpy(dst + a, src + a, b - a);
-        });
-        return;
-    }
-    pool.run(parts, [&](int i) {
-        const unsigned r0 = (unsigned)((uint64_t)rows * i / parts), r1 = (unsigned)((uint64_t)rows * (i + 1) / parts);
-        for (unsigned r = r0; r < r1; ++r) std::memcpy(dst + r * row_bytes, src + (size_t)r * stride, row_bytes);
-    });
+    if (stride == row_bytes) std::memcpy(dst, src, row_bytes * rows);
+    else
+        for (size_t r = 0; r < rows; ++r) std::memcpy(dst + r * row_bytes, src + r * stride, row_bytes);
 }
 
-// Marks every part of a launched image on the way out: all are marked already
+// Marks every part of a launched chunk on the way out: all are marked already
 // unless the staging was left by an exception.
 struct FeedGuard {
     HostFeed* feed;
@@ -268,55 +261,119 @@ static hipError_t launch_any(int fmt, const LaunchCfg& cfg, const void* in, size
                               : launch_plain(fmt, cfg, in, row_bytes, out, bw, nblocks, stream);
 }
 
-// Encodes an image of one chunk (up to about 8 MiB) into ctx->h_out[0].  The
-// kernel reads the pinned staging copy over PCIe and writes its blocks to
-// pinned memory over PCIe: the copy engines' set-up and synchronisation weigh
-// more than the copy (512x512: 82 us through them).
-//   From 128 KiB on a fed kernel (k_encode_fed) is launched before anything is
-// staged and reads the parts while the host still writes the next ones, so the
-// launch and the copy are hidden behind the link: 512x512 43.7 us, 1024x1024
-// 116 us, against 55 and 146 us with one launch per 512 KiB staged.  Below
-// that the kernel's look at the mark, over PCIe, costs more than it hides
-// (64x64: 19.4 against 17.0 us): staged first, one plain launch.  Images of
-// more chunks keep the DMA pipeline, which reaches 52-56 GB/s on their chunks,
-// kernels 49.
-//   Between the fed launch and the mark of the last part the host calls
-// nothing that could wait for the device, so the kernel's wait ends whatever
-// other threads and streams do.  Should this thread stand still for `patience`
-// ticks the kernel ends unfinished, and the image, by then all staged, is
-// encoded by a plain launch.  Where a launch returns only after its kernel the
-// image is staged first, too.
-static hipError_t encode_one_chunk(StagingCtx* ctx, int fmt, const LaunchCfg& cfg, const uint8_t* input,
-                                   unsigned stride, uint32_t bw, uint32_t bh, size_t out_bytes, uint64_t patience)
+// What the chunks of one image share.
+struct HostImage {
+    StagingCtx* ctx;
+    int fmt;
+    LaunchCfg cfg;  // of a plain launch
+    unsigned char* result;
+    unsigned char* result2;  // a pair's second format, or null
+    const unsigned char* input;
+    size_t stride, row_bytes, block_bytes;
+    uint32_t bw;
+    size_t part_bytes;  // about what a part of a chunk holds
+    uint64_t patience;
+};
+
+// The k-th chunk: `rows` block rows from the y0-th on, launched as number
+// `call`; of its groups of kFeedBlocks blocks the first `got` are in the
+// caller's memory.
+struct HostChunk {
+    uint32_t k = 0, y0 = 0, rows = 0;
+    uint64_t call = 0;
+    uint32_t got = 0;
+};
+
+static const StagingCtx::Slot& slot_of(const HostImage& im, const HostChunk& c) { return im.ctx->slot[c.k % kSlots]; }
+static hipStream_t stream_of(const HostImage& im, const HostChunk& c) { return im.ctx->stream[c.k & 1u]; }
+
+// Copies blocks [first, last) of a chunk from its slot to the caller, large
+// ranges split over the copy pool.
+static void collect(const HostImage& im, const HostChunk& c, uint32_t first, uint32_t last)
 {
-    const size_t row_bytes = (size_t)bw * 16, bytes = row_bytes * 4 * bh;
-    uint8_t* const in = static_cast<uint8_t*>(ctx->h_in[0]);
-    uint8_t* const out = static_cast<uint8_t*>(ctx->h_out[0]);
-    const auto plain = [&]() -> hipError_t {
-        const hipError_t e = launch_any(fmt, cfg, in, row_bytes, out, out + out_bytes, bw, bw * bh, ctx->stream);
-        return e == hipSuccess ? hipStreamSynchronize(ctx->stream) : e;
+    const uint8_t* const out = slot_of(im, c).out;
+    const size_t bb = im.block_bytes;
+    const auto copy = [&](uint32_t a, uint32_t b) {
+        const size_t to = ((size_t)c.y0 * im.bw + a) * bb, n = (size_t)(b - a) * bb;
+        std::memcpy(im.result + to, out + a * bb, n);
+        if (im.result2) std::memcpy(im.result2 + to, out + ((size_t)im.bw * c.rows + a) * bb, n);
     };
-    if (bytes < (128u << 10) || ctx->stage_first) {
-        copy_rows(in, input, stride, row_bytes, bh * 4);
-        return plain();
+    constexpr uint32_t kPiece = 8192;  // blocks
+    if (last - first < 4u * kPiece) return copy(first, last);
+    CopyPool::get().run((int)((last - first + kPiece - 1) / kPiece), [&](int i) {
+        const uint32_t a = first + (uint32_t)i * kPiece;
+        copy(a, last - a < kPiece ? last : a + kPiece);
+    });
+}
+
+// Launches a chunk's kernel and stages its rows.
+static hipError_t start_chunk(const HostImage& im, HostChunk& c)
+{
+    const StagingCtx::Slot& slot = slot_of(im, c);
+    const uint32_t nblocks = im.bw * c.rows;
+    const size_t bytes = im.row_bytes * 4 * c.rows;
+    const uint8_t* const rows = im.input + (size_t)c.y0 * 4 * im.stride;
+    const bool fed = bytes >= (128u << 10) && !im.ctx->stage_first;
+    // parts of whole block rows
+    const uint32_t want = (uint32_t)std::max<size_t>(1, std::min<size_t>(kFeedParts, bytes / im.part_bytes));
+    const uint32_t prows = (c.rows + want - 1) / want, parts = (c.rows + prows - 1) / prows;
+    const auto stage = [&](uint32_t p) {
+        const size_t r0 = (size_t)p * prows * 4, n = std::min((size_t)prows * 4, (size_t)c.rows * 4 - r0);
+        copy_rows(slot.in + r0 * im.row_bytes, rows + r0 * im.stride, im.stride, im.row_bytes, n);
+    };
+    // one thread copies an image of 1 MiB at the link's rate, and waking others
+    // takes longer (512x512: 38 us with one, 43 with them)
+    const auto each_part = [&](auto&& f) {
+        if (bytes >= (2u << 20)) CopyPool::get().run((int)parts, [&](int p) { f((uint32_t)p); });
+        else
+            for (uint32_t p = 0; p < parts; ++p) f(p);
+    };
+    if (!fed) each_part(stage);
+    c.call = ++im.ctx->call;
+    const hipError_t e =
+        launch_fed(im.fmt, slot.in, im.row_bytes, slot.out, slot.out + nblocks * im.block_bytes, im.bw, nblocks,
+                   slot.feed, c.call, fed ? im.bw * prows : 0u, im.patience, stream_of(im, c));
+    if (e != hipSuccess || !fed) return e;
+    const FeedGuard guard{slot.feed, c.call, parts};
+    each_part([&](uint32_t p) {
+        stage(p);
+        guard.mark(p);
+    });
+    return hipSuccess;
+}
+
+// Collects the groups of a chunk that are marked, in order.
+static bool collect_marked(const HostImage& im, HostChunk& c)
+{
+    const uint32_t nblocks = im.bw * c.rows, groups = feed_groups(nblocks);
+    const HostFeed* const feed = slot_of(im, c).feed;
+    uint32_t to = c.got;
+    while (to < std::min(groups, kFeedMarks) && __atomic_load_n(&feed->done[to], __ATOMIC_ACQUIRE) == c.call) ++to;
+    if (to != c.got) collect(im, c, c.got * kFeedBlocks, std::min(to * kFeedBlocks, nblocks));
+    c.got = to;
+    return c.got == groups;
+}
+
+// Waits for a chunk and collects it: by its marks, or, where they don't come
+// within 2 ms or don't reach, by its stream.
+static hipError_t finish_chunk(const HostImage& im, HostChunk& c)
+{
+    const auto end = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    for (uint32_t look = 1; !collect_marked(im, c); ++look) {
+        if (c.got == kFeedMarks || (look % 64 == 0 && std::chrono::steady_clock::now() > end)) break;
     }
-    // parts of whole block rows, about 64 KiB or a thirty-second of the image
-    const unsigned want = (unsigned)std::min<size_t>(kFeedParts, bytes >> 16);
-    const unsigned prows = (bh + want - 1) / want, parts = (bh + prows - 1) / prows;
-    const uint64_t call = ++ctx->call;
-    hipError_t e = launch_fed(fmt, in, row_bytes, out, out + out_bytes, bw, bw * bh, ctx->feed, call, bw * prows,
-                              patience, ctx->stream);
-    if (e != hipSuccess) return e;
-    {
-        const FeedGuard guard{ctx->feed, call, parts};
-        for (unsigned p = 0; p < parts; ++p) {
-            const size_t r0 = (size_t)p * prows, rows = std::min<size_t>(prows, bh - r0);
-            copy_rows(in + r0 * 4 * row_bytes, input + r0 * 4 * stride, stride, row_bytes, (unsigned)rows * 4);
-            guard.mark(p);
-        }
+    if (c.got == feed_groups(im.bw * c.rows)) return hipSuccess;
+    const StagingCtx::Slot& slot = slot_of(im, c);
+    const hipStream_t stream = stream_of(im, c);
+    const uint32_t nblocks = im.bw * c.rows;
+    hipError_t e = hipStreamSynchronize(stream);
+    if (e == hipSuccess && __atomic_load_n(&slot.feed->gave_up, __ATOMIC_ACQUIRE) == c.call) {
+        e = launch_any(im.fmt, im.cfg, slot.in, im.row_bytes, slot.out, slot.out + nblocks * im.block_bytes, im.bw,
+                       nblocks, stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(stream);
     }
-    if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return e;
-    return ctx->feed->gave_up == call ? plain() : hipSuccess;
+    if (e == hipSuccess) collect(im, c, c.got * kFeedBlocks, nblocks);
+    return e;
 }
 
 // fmt: one format into `result`, or kFeedDual: DXT1 into `result` and ETC1S
@@ -344,9 +401,15 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
     int rc = device_info(&di);
     if (rc != GOOFY_OK) return rc;
     StagingCtx* ctx = staging_pool().acquire(di.device);
-    struct Release {
+    struct Release {  // on every path, the kernels are through with the context first
         StagingCtx* c;
-        ~Release() { staging_pool().release(c); }
+        bool done = false;
+        ~Release()
+        {
+            for (hipStream_t s : c->stream)
+                if (s && !done) (void)hipStreamSynchronize(s);
+            staging_pool().release(c);
+        }
     } rel{ctx};
 
     const size_t row_bytes = (size_t)width * 4;
@@ -357,65 +420,30 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
     const size_t outs = dual ? 2 : 1;
     const size_t bb = dual_alpha ? 16 : (dual ? 8 : block_bytes(fmt));
     if ((rc = ensure_ctx(ctx, row_bytes * 4 * cb, outs * bw * cb * bb)) != GOOFY_OK) return rc;
-    const unsigned nchunks = (bh + cb - 1) / cb;
-    const LaunchCfg cfg = auto_cfg((uint64_t)bw * cb, di.num_cus);
+    // Parts of an image of one chunk: 64 KiB, or a thirty-second of it, so that
+    // the kernel can start early.  Of larger ones: 1 MiB, copied as streams by
+    // the threads; pieces of 256 KiB take 2 to 3 times as long from an image
+    // that others have just written (first call on a new 4096x4096 image 2.1-3.4
+    // ms, in 1 MiB pieces 1.5) and are 1-2% faster on one that lies in the
+    // caches.
+    const size_t part_bytes = cb < bh ? (size_t)1 << 20 : (size_t)1 << 16;
+    const HostImage im{ctx,    fmt,       auto_cfg((uint64_t)bw * cb, di.num_cus), result, dual ? result2 : nullptr, input,
+                       stride, row_bytes, bb, bw, part_bytes, patience};
+    HostChunk ring[kSlots];  // chunks [oldest, k) are launched and not yet collected
     hipError_t e = hipSuccess;
-
-    // Copies chunk k's blocks from its slot to the caller.
-    auto collect = [&](unsigned k) {
-        const int s = (int)(k % kSlots);
-        const size_t n = (size_t)std::min(cb, bh - k * cb) * bw * bb;
-        std::memcpy(result + (size_t)k * cb * bw * bb, ctx->h_out[s], n);
-        if (dual) std::memcpy(result2 + (size_t)k * cb * bw * bb, static_cast<uint8_t*>(ctx->h_out[s]) + n, n);
-    };
-    if (nchunks == 1) {
-        if ((e = encode_one_chunk(ctx, fmt, cfg, input, stride, bw, bh, (size_t)bw * bh * bb, patience)) != hipSuccess) {
-            (void)hipStreamSynchronize(ctx->stream);
-            return fail_hip(e, "drop-in one-chunk launch");
-        }
-        collect(0);
-        return GOOFY_OK;
+    uint32_t k = 0, oldest = 0;
+    for (uint64_t y0 = 0; y0 < bh && e == hipSuccess; y0 += cb, ++k) {
+        if (k - oldest == kSlots && (e = finish_chunk(im, ring[oldest++ % kSlots])) != hipSuccess) break;
+        ring[k % kSlots] = HostChunk{k, (uint32_t)y0, std::min<uint32_t>(cb, bh - (uint32_t)y0)};
+        e = start_chunk(im, ring[k % kSlots]);
+        if (oldest < k) collect_marked(im, ring[oldest % kSlots]);
     }
-    auto finish_chunk = [&](unsigned k) -> hipError_t {
-        hipError_t r = hipEventSynchronize(ctx->out_ready[k % kSlots]);
-        if (r == hipSuccess) collect(k);
-        return r;
-    };
-
-    // Chunk k uses slot k % kSlots.  Chunk k-kSlots, the slot's previous user,
-    // was collected by finish_chunk in an earlier iteration, so its upload,
-    // kernel and download are complete and the slot is free on both sides.
-    const hipStream_t up = ctx->in_stream;
-    unsigned collected = 0;  // chunks [0, collected) are in `result`
-    for (unsigned k = 0; k < nchunks && e == hipSuccess; ++k) {
-        const int s = (int)(k % kSlots);
-        const unsigned rows = std::min(cb, bh - k * cb);  // block rows in this chunk
-        copy_rows(static_cast<uint8_t*>(ctx->h_in[s]), input + (size_t)k * cb * 4 * stride, stride, row_bytes,
-                  rows * 4);
-        void* const kin = ctx->d_in[s];
-        void* const kout = ctx->d_out[s];
-        if ((e = hipMemcpyAsync(ctx->d_in[s], ctx->h_in[s], row_bytes * 4 * rows, hipMemcpyHostToDevice, up)) !=
-            hipSuccess)
-            break;
-        if ((e = hipEventRecord(ctx->h2d_done[s], up)) != hipSuccess) break;
-        if ((e = hipStreamWaitEvent(ctx->stream, ctx->h2d_done[s], 0)) != hipSuccess) break;
-        const size_t n = (size_t)bw * rows * bb;
-        uint8_t* second = static_cast<uint8_t*>(kout) + n;
-        e = launch_any(fmt, cfg, kin, row_bytes, kout, second, bw, bw * rows, ctx->stream);
-        if (e != hipSuccess) break;
-        if ((e = hipMemcpyAsync(ctx->h_out[s], ctx->d_out[s], outs * n, hipMemcpyDeviceToHost, ctx->stream)) !=
-            hipSuccess)
-            break;
-        if ((e = hipEventRecord(ctx->out_ready[s], ctx->stream)) != hipSuccess) break;
-        // collect what is kSlots - 1 chunks behind, freeing the slot chunk k+1 uses
-        while (e == hipSuccess && collected + (kSlots - 1) <= k) e = finish_chunk(collected++);
-    }
-    while (e == hipSuccess && collected < nchunks) e = finish_chunk(collected++);
-    if (e != hipSuccess) {
-        (void)hipStreamSynchronize(ctx->in_stream);
-        (void)hipStreamSynchronize(ctx->stream);
-        return fail_hip(e, "drop-in staging pipeline");
-    }
+    // a marker behind the kernels while they run, for a caller that goes on to
+    // wait for the device
+    for (uint32_t i = 0; i < std::min(k, 2u); ++i) (void)hipEventRecord(ctx->ended[i], ctx->stream[i]);
+    while (e == hipSuccess && oldest < k) e = finish_chunk(im, ring[oldest++ % kSlots]);
+    if (e != hipSuccess) return fail_hip(e, "drop-in staging");
+    rel.done = true;
     return GOOFY_OK;
 }
 

@@ -116,19 +116,26 @@ hipError_t launch_dual_alpha(const LaunchCfg& cfg, const void* src, size_t pitch
 // The drop-in's kernel, which encodes an image in pinned host memory while
 // the host is still staging it there.  HostFeed (pinned, coherent): the word
 // of a part holds the number of the call whose rows are staged in it, written
-// after them; gave_up the number of a call whose kernel stopped waiting.
+// after them; gave_up the number of a call whose kernel stopped waiting; done,
+// of each group of kFeedBlocks blocks up to kFeedMarks (8 MiB of pixels), the
+// number of the last call whose blocks of it are in host memory.
 constexpr uint32_t kFeedParts = 32;
-constexpr uint32_t kFeedGroups = 64;
+constexpr uint32_t kFeedGroups = 24;
+constexpr uint32_t kFeedBlocks = 512;
+constexpr uint32_t kFeedMarks = 256;
+inline uint32_t feed_groups(uint32_t nblocks) { return nblocks / kFeedBlocks + (nblocks % kFeedBlocks != 0); }
 struct HostFeed {
     struct alignas(64) Part {
         uint64_t staged;
     } part[kFeedParts];
     alignas(64) uint64_t gave_up;
+    alignas(64) uint64_t done[kFeedMarks];
 };
 // Pseudo-formats: both 8-byte formats / both 16-byte formats, the second into
 // dst2.
 constexpr int kFeedDual = 1 << 16, kFeedDualAlpha = (1 << 16) + 1;
-// part_blocks: blocks per part (at most kFeedParts parts); call: a number that
+// part_blocks: blocks per part (at most kFeedParts parts), or 0 where all rows
+// are staged before the launch; call: a number that
 // no word holds yet; patience: how long a wait may last, in 10 ns ticks.
 hipError_t launch_fed(int fmt, const void* src, size_t pitch, void* dst, void* dst2, uint32_t bw, uint32_t nblocks,
                       HostFeed* feed, uint64_t call, uint32_t part_blocks, uint64_t patience, hipStream_t stream);

@@ -231,6 +231,9 @@ __global__ __launch_bounds__(512) void k_encode_dual_alpha(const uint8_t* __rest
                            threadIdx.x & 63u);
 }
 
+// s_waitcnt's operand for vmcnt(0), the other counters at their highest.
+constexpr int kWaitStores = 0x0F70;
+
 // Waits until part p of the image is staged (HostFeed): one lane reads the
 // part's word in host memory, about every 2 us.  The host stages every part of
 // a kernel it has launched without any call in between that could wait for
@@ -251,11 +254,16 @@ __device__ __forceinline__ bool await_part(HostFeed* feed, uint32_t p, uint64_t 
 
 // One image (or chunk of one) in pinned host memory, encoded over PCIe while
 // the host is still staging it: launched first, it takes each group of 512
-// blocks as soon as the parts it lies in are staged.  FMT: a format, or
-// kFeedDual / kFeedDualAlpha into dst and dst2.  part_blocks: blocks per part.
-// A grid of at most kFeedGroups workgroups steps through the groups in order:
-// PCIe needs few loads in flight, and every waiting workgroup polls over the
-// same link.
+// blocks as soon as the parts it lies in are staged (part_blocks blocks each;
+// 0: the whole image is), and marks the group once its blocks are in host
+// memory, so that the host takes them on while later groups are on the link.
+// FMT: a format, or kFeedDual / kFeedDualAlpha into dst and dst2.
+//   A grid of at most kFeedGroups workgroups steps through the groups in order:
+// the link needs few loads in flight, and every waiting workgroup polls over it
+// (8192x8192 DXT1 with 16, 24, 32, 64 workgroups: 5.23, 5.14, 5.22, 5.46 ms per
+// call).  Every wave waits for its own stores before the barrier; behind
+// it one lane writes back what its L2 may hold of them (the release), then the
+// mark.
 template <int FMT>
 __global__ __launch_bounds__(512) void k_encode_fed(const uint8_t* src, uint64_t pitch, uint8_t* dst, uint8_t* dst2,
                                                     uint32_t bw, uint32_t nblocks, uint64_t magic, HostFeed* feed,
@@ -264,25 +272,37 @@ __global__ __launch_bounds__(512) void k_encode_fed(const uint8_t* src, uint64_t
     __shared__ uint32_t staged;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (uint32_t group = blockIdx.x; (uint64_t)group * 512u < nblocks; group += gridDim.x) {
-        const uint32_t first = group * 512u;
-        if (threadIdx.x == 0) {
-            const uint32_t end = (min(first + 511u, nblocks - 1u)) / part_blocks;
-            bool ok = true;
-            for (uint32_t p = first / part_blocks; ok && p <= end; ++p) ok = await_part(feed, p, call, patience);
-            staged = ok ? 1u : 0u;
+    for (uint32_t group = blockIdx.x; (uint64_t)group * kFeedBlocks < nblocks; group += gridDim.x) {
+        const uint32_t first = group * kFeedBlocks;
+        if (part_blocks) {
+            if (threadIdx.x == 0) {
+                const uint32_t end = (min(first + kFeedBlocks - 1u, nblocks - 1u)) / part_blocks;
+                bool ok = true;
+                for (uint32_t p = first / part_blocks; ok && p <= end; ++p) ok = await_part(feed, p, call, patience);
+                staged = ok ? 1u : 0u;
+            }
+            __syncthreads();
+            if (!staged) return;  // all of the workgroup or none
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");  // the rows, after the words (system scope)
         }
-        __syncthreads();
-        const bool ok = staged != 0u;
-        __syncthreads();  // the word is free for the next group
-        if (!ok) return;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");  // the rows, after the words (system scope)
         const uint32_t tile = first + wave * 64u;
-        if (tile >= nblocks) continue;
-        if constexpr (FMT == kFeedDual) encode_pair_tile<false>(src, pitch, dst, dst2, bw, nblocks, magic, tile, lane);
-        else if constexpr (FMT == kFeedDualAlpha)
-            encode_pair_tile<true>(src, pitch, dst, dst2, bw, nblocks, magic, tile, lane);
-        else encode_tile<FMT, 1, true>(src, pitch, dst, bw, magic, nblocks, tile, lane);
+        if (tile < nblocks) {
+            if constexpr (FMT == kFeedDual)
+                encode_pair_tile<false>(src, pitch, dst, dst2, bw, nblocks, magic, tile, lane);
+            else if constexpr (FMT == kFeedDualAlpha)
+                encode_pair_tile<true>(src, pitch, dst, dst2, bw, nblocks, magic, tile, lane);
+            else encode_tile<FMT, 1, true>(src, pitch, dst, bw, magic, nblocks, tile, lane);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(kWaitStores);
+        __syncthreads();  // also: the word `staged` is free for the next group
+        if (threadIdx.x == 0 && group < kFeedMarks) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+            // the write-back's end: the compiler, having seen the wait above,
+            // leaves out the fence's own
+            __builtin_amdgcn_s_waitcnt(kWaitStores);
+            __hip_atomic_store(&feed->done[group], call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
 }
 
@@ -420,8 +440,8 @@ hipError_t launch_plain(int fmt, const LaunchCfg& c, const void* src, size_t pit
 hipError_t launch_fed(int fmt, const void* src, size_t pitch, void* dst, void* dst2, uint32_t bw, uint32_t nblocks,
                       HostFeed* feed, uint64_t call, uint32_t part_blocks, uint64_t patience, hipStream_t stream)
 {
-    if (nblocks == 0 || part_blocks == 0 || (nblocks - 1u) / part_blocks >= kFeedParts) return hipErrorInvalidValue;
-    const dim3 grid(std::min((nblocks + 511u) / 512u, kFeedGroups)), block(512);
+    if (nblocks == 0 || (part_blocks && (nblocks - 1u) / part_blocks >= kFeedParts)) return hipErrorInvalidValue;
+    const dim3 grid(std::min(feed_groups(nblocks), kFeedGroups)), block(kFeedBlocks);
     const auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, block, 0, stream, (const uint8_t*)src, (uint64_t)pitch, (uint8_t*)dst,
                            (uint8_t*)dst2, bw, nblocks, div_magic(bw), feed, call, part_blocks, patience);

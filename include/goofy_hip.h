@@ -72,8 +72,8 @@ GOOFY_HIP_API int goofy_hip_device_count(void);
  * (width/4)*(height/4) tightly packed blocks (8 bytes each; 16 for DXT5 and
  * ETC2 RGBA8).  -1 if width % 16, then -2 if
  * height % 4; width or height 0 writes nothing and returns 0.  Synchronous:
- * stages through device memory on a per-thread stream and returns when
- * `result` holds the blocks.  Thread-safe. */
+ * kernels read pinned staging memory over PCIe while the rows are copied into
+ * it; returns when `result` holds the blocks.  Thread-safe. */
 GOOFY_HIP_API int goofy_hip_compress(int format, unsigned char* result, const unsigned char* input,
                                      unsigned int width, unsigned int height, unsigned int stride);
 /* The same entry points with the exact CompressFunc_t signature

@@ -815,6 +815,42 @@ def test_dropin_fed_kernel_sizes(gpu, w, h, extra, fmt):
         assert np.array_equal(got[:n], want) and (got[n:] == 0xCD).all(), call
 
 
+@pytest.mark.parametrize("fmt", [W.DXT1, W.ETC1, W.DXT5, W.ETC2])
+@pytest.mark.parametrize("w,h,extra", [(2048, 1028, 0), (2048, 2048, 16), (4096, 2052, 0), (1040, 8196, 64),
+                                       (2097152, 4, 0), (1048592, 8, 0)])
+def test_dropin_fed_chunks(gpu, w, h, extra, fmt):
+    """Host images of two chunks to more than there are staging slots, with a
+    short last chunk, and of chunks with more groups than marks (one block row
+    of 32 MiB and two of 16 MiB) == the device entry point; every other call
+    with kernels that give up their wait at once, whose chunks are encoded
+    again; and a call of one small chunk after each, in the same slots."""
+    import ctypes
+    stride = w * 4 + extra
+    img = gpu.synth_host(2, 52, fmt, 12, w, h, stride, fill=0xA5)
+    n = (w // 4) * (h // 4) * gpu.block_bytes(fmt)
+    src, out = upload(img.reshape(h, stride)[:, :w * 4]), dev_buffer(n)
+    gpu.compress_device(fmt, out, src, w, h, w * 4)
+    want = to_host(out)
+    small = gpu.compress(fmt, img, 64, 4, stride)
+    say(f"drop-in fed chunks {w}x{h} stride {stride} fmt {fmt}")
+    late = gpu._lib.goofy_impl_compress_with_patience
+    late.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint, ctypes.c_uint, ctypes.c_uint,
+                     ctypes.c_uint64]
+    for call in range(4):
+        got = np.full(n + 64, 0xCD, np.uint8)
+        if call % 2:
+            assert late(fmt, got.ctypes.data, img.ctypes.data, w, h, stride, 0) == 0
+        else:
+            assert gpu._lib.goofy_hip_compress(fmt, gpu._u8(got), gpu._u8(img), w, h, stride) == 0
+        assert np.array_equal(got[:n], want) and (got[n:] == 0xCD).all(), call
+        assert np.array_equal(gpu.compress(fmt, img, 64, 4, stride), small)
+    if fmt in (W.DXT1, W.DXT5):
+        pair = gpu.compress_dual(img, w, h, stride) if fmt == W.DXT1 else gpu.compress_dual_alpha(img, w, h, stride)
+        other = dev_buffer(n)
+        gpu.compress_device(W.ETC1 if fmt == W.DXT1 else W.ETC2, other, src, w, h, w * 4)
+        assert np.array_equal(pair[0], want) and np.array_equal(pair[1], to_host(other))
+
+
 def test_dropin_from_threads(gpu):
     """The drop-in on four host threads at once, each with its own images of
     one to several staging chunks: every call bit-identical to the same call
