@@ -156,9 +156,10 @@ static QualityScratchPool& quality_scratch_pool()
 // its inputs and with its work area left at zero, so nothing else need be waited
 // for: the stream's synchronisation returns 5 us later (the marker behind the
 // kernel, its signal).  The marker is put there all the same, while the kernel
-// runs, for a caller that goes on to wait for the stream or the device.  Whole
-// calls from Python in us, waiting for the stream -> for the words -> for the
-// words with the marker; and with a device synchronisation behind each:
+// runs, for a caller that goes on to wait for the stream or the device.  Work
+// queued before the launch has ended by then, too: the kernel started behind it.
+// Whole calls from Python in us, waiting for the stream -> for the words -> for
+// the words with the marker; and with a device synchronisation behind each:
 //   512x512 DXT1          19.0 -> 13.9 -> 14.9,  22.0 -> 25.5 -> 17.7
 //   8192^2 ETC1           66.2 -> 61.2 -> 61.5,  69.4 -> 72.9 -> 65.3
 //   floor and image-against-image figures, 4100x3076

@@ -191,8 +191,13 @@ GOOFY_HIP_API int goofy_hip_decode_device(int format, void* d_rgba, const void* 
  * a pixel is read as a little-endian word, "r" = bits 16..23, "g" = 8..15,
  * "b" = 0..7, "a" = 24..31; luma = 0.21 r + 0.72 g + 0.07 b; PSNR =
  * 10 log10(peak^2 / mse) with peak 255, and 768 for the summed-RGB figure;
- * an MSE below 1e-7 gives DBL_MAX.  Synchronous on `stream`.  Uses a
- * 4 KiB device work area and 768 bytes of pinned host memory, into which the
+ * an MSE below 1e-7 gives DBL_MAX.  Synchronous on `stream`: the call returns
+ * when the work queued there before it and its own kernel's have been done
+ * (the kernel's sums are in host memory).  The stream may report itself busy
+ * for some microseconds more, and what earlier kernels wrote to host memory
+ * that was allocated non-coherent shows after a synchronisation of the
+ * stream, which this call queues but does not wait for.  Uses a 4 KiB device
+ * work area and 768 bytes of pinned host memory, into which the
  * kernel writes the sums, from a per-device pool (allocated on first use,
  * never freed, one pair per concurrent call), so a call never waits on other
  * streams. */
@@ -225,7 +230,7 @@ GOOFY_HIP_API int goofy_hip_quality_device_noalloc(int format, const void* d_blo
 /* getMsePsnr (Src/main.cpp:403-469) between two device RGBA8 images of the
  * same size, e.g. a source and its quality floor below: same figures and
  * labels as goofy_hip_quality_device.  width % 4 == 0; rows 16-byte aligned.
- * Synchronises `stream`. */
+ * Synchronous on `stream` in the same way. */
 GOOFY_HIP_API int goofy_hip_quality_images_device(const void* d_a, size_t pitch_a, const void* d_b, size_t pitch_b,
                                                   unsigned int width, unsigned int height, void* stream,
                                                   goofy_quality* out);
