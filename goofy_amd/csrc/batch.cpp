@@ -31,20 +31,27 @@
 
 using namespace goofy_impl;
 
+// A work-list in device memory: the descriptors and prefix sums of one tile
+// size.  Written once, before the first launch that reads it, and freed with
+// the plan: launches that still run and graphs that captured one keep reading
+// theirs, whatever shape the plan has taken since.
+struct Worklist {
+    TexDesc* d = nullptr;
+    uint32_t ntex = 0, ntiles = 0;
+};
+
 struct goofy_batch {
     int device = -1;
     int num_cus = 0;
     std::string arch;
     std::vector<goofy_texture_desc> textures;  // non-empty textures, caller order
-    std::vector<TexDesc> descs;
-    TexDesc* d_descs = nullptr;
-    size_t d_descs_cap = 0;
-    uint32_t ntiles = 0;
+    Worklist lists[3];              // for 1, 2 and 4 blocks per lane, each made when first needed
+    const Worklist* list = nullptr;  // the one of cfg's tile size
     uint64_t blocks = 0, pixels = 0;
     bool alpha = false;  // holds DXT5 / ETC2 RGBA8 textures
     LaunchCfg cfg{};
-    // Recorded by every launch's own dispatch: the work-list is rewritten or
-    // freed only once the launches that read it have finished.
+    // Recorded by every launch's own dispatch, for the calls that wait for the
+    // plan's launches.
     hipEvent_t launched = nullptr;
     bool launched_pending = false;
 };
@@ -62,13 +69,10 @@ int wait_launched(goofy_batch* b)
     return GOOFY_OK;
 }
 
-// Rebuild the tile prefix sums for the plan's tile size and upload them.
-int build_worklist(goofy_batch* b)
+// Makes the work-list of tiles of `tile` blocks.
+int make_worklist(const goofy_batch* b, uint64_t tile, Worklist* out)
 {
-    int rc = wait_launched(b);
-    if (rc != GOOFY_OK) return rc;
-    const uint64_t tile = (uint64_t)tile_blocks(b->cfg);
-    b->descs.clear();
+    std::vector<TexDesc> descs;
     uint64_t tiles = 0;
     for (const goofy_texture_desc& t : b->textures) {
         // one entry per horizontal stripe of at most max_stripe_brows block
@@ -88,30 +92,45 @@ int build_worklist(goofy_batch* b)
             d.tile_begin = (uint32_t)tiles;
             tiles += (d.nblocks + tile - 1) / tile;
             if (tiles > 0xFFFFFFFFull / tile) return fail(GOOFY_ERR_TOO_LARGE, "batch has too many tiles");
-            b->descs.push_back(d);
+            descs.push_back(d);
             y0 += rows;
         }
     }
-    b->ntiles = (uint32_t)tiles;
-    const size_t ntex = b->descs.size();
+    const size_t ntex = descs.size();
     std::vector<uint8_t> host(worklist_bytes(ntex));
-    if (ntex) std::memcpy(host.data(), b->descs.data(), ntex * sizeof(TexDesc));
+    if (ntex) std::memcpy(host.data(), descs.data(), ntex * sizeof(TexDesc));
     uint32_t* tb = worklist_tile_begin(reinterpret_cast<TexDesc*>(host.data()), ntex);
-    for (size_t i = 0; i < ntex; ++i) tb[i] = b->descs[i].tile_begin;
-    tb[ntex] = b->ntiles;
-    const size_t bytes = host.size();
-    hipError_t e;
-    if (b->d_descs_cap < bytes) {
-        if (b->d_descs) (void)hipFree(b->d_descs);
-        b->d_descs = nullptr;
-        b->d_descs_cap = 0;
-        e = hipMalloc((void**)&b->d_descs, bytes);
-        if (e != hipSuccess) return fail_hip(e, "hipMalloc(descriptors)");
-        b->d_descs_cap = bytes;
+    for (size_t i = 0; i < ntex; ++i) tb[i] = descs[i].tile_begin;
+    tb[ntex] = (uint32_t)tiles;
+    TexDesc* d = nullptr;
+    hipError_t e = hipMalloc((void**)&d, host.size());
+    if (e != hipSuccess) return fail_hip(e, "hipMalloc(descriptors)");
+    e = hipMemcpy(d, host.data(), host.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        (void)hipFree(d);
+        return fail_hip(e, "hipMemcpy(work-list)");
     }
-    e = hipMemcpy(b->d_descs, host.data(), bytes, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return fail_hip(e, "hipMemcpy(work-list)");
+    *out = Worklist{d, (uint32_t)ntex, (uint32_t)tiles};
     return GOOFY_OK;
+}
+
+// Gives the plan the shape c and the work-list of its tile size; on an error
+// the plan keeps the shape it has.
+int set_shape(goofy_batch* b, const LaunchCfg& c)
+{
+    Worklist& l = b->lists[__builtin_ctz((unsigned)c.blocks_per_lane)];
+    if (!l.d) {
+        const int rc = make_worklist(b, (uint64_t)tile_blocks(c), &l);
+        if (rc != GOOFY_OK) return rc;
+    }
+    b->cfg = c;
+    b->list = &l;
+    return GOOFY_OK;
+}
+
+hipError_t launch(const goofy_batch* b, hipStream_t s, hipEvent_t done)
+{
+    return launch_batch(b->cfg, b->list->d, b->list->ntex, b->list->ntiles, b->num_cus, s, b->alpha, done);
 }
 
 // ---- tuning cache ---------------------------------------------------------------
@@ -233,7 +252,7 @@ int goofy_batch_create(const goofy_texture_desc* textures, size_t count, const g
         }
         b->cfg = c;
     }
-    rc = build_worklist(b);
+    rc = set_shape(b, b->cfg);
     if (rc != GOOFY_OK) {
         goofy_batch_destroy(b);
         return rc;
@@ -246,7 +265,7 @@ int goofy_batch_launch(goofy_batch* b, void* stream)
 {
     clear_error();
     if (!b) return fail(GOOFY_ERR_INVALID, "null batch");
-    if (b->ntiles == 0) return GOOFY_OK;
+    if (b->list->ntiles == 0) return GOOFY_OK;
     const hipStream_t s = (hipStream_t)stream;
     hipError_t e;
     if (!b->launched && (e = hipEventCreateWithFlags(&b->launched, hipEventDisableTiming)) != hipSuccess)
@@ -259,8 +278,7 @@ int goofy_batch_launch(goofy_batch* b, void* stream)
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();  // the launch says why
     const bool eager = cap == hipStreamCaptureStatusNone;
-    e = launch_batch(b->cfg, b->d_descs, (uint32_t)b->descs.size(), b->ntiles, b->num_cus, s, b->alpha,
-                     eager ? b->launched : nullptr);
+    e = launch(b, s, eager ? b->launched : nullptr);
     if (e != hipSuccess) return fail_hip(e, "batch kernel launch");
     if (eager) b->launched_pending = true;
     return GOOFY_OK;
@@ -303,15 +321,16 @@ int goofy_batch_set_config(goofy_batch* b, const goofy_launch_config* cfg)
     if (!b || !cfg) return fail(GOOFY_ERR_INVALID, "null argument");
     LaunchCfg c = to_cfg(*cfg);
     if (!cfg_valid(c)) return fail(GOOFY_ERR_INVALID, "invalid launch config");
-    const bool retile = c.blocks_per_lane != b->cfg.blocks_per_lane;
-    b->cfg = c;
-    return retile ? build_worklist(b) : wait_launched(b);
+    const int rc = wait_launched(b);
+    return rc != GOOFY_OK ? rc : set_shape(b, c);
 }
 
 int goofy_batch_autotune(goofy_batch* b, void* stream, int reps, goofy_launch_config* chosen, float* best_ms)
 {
     clear_error();
     if (!b) return fail(GOOFY_ERR_INVALID, "null batch");
+    int rc = wait_launched(b);
+    if (rc != GOOFY_OK) return rc;
     if (reps < 1) reps = 1;
     hipStream_t s = (hipStream_t)stream;
     hipEvent_t e0, e1;
@@ -325,23 +344,20 @@ int goofy_batch_autotune(goofy_batch* b, void* stream, int reps, goofy_launch_co
     const LaunchCfg start = b->cfg;
     LaunchCfg best = b->cfg;
     float best_t = 1e30f;
-    int rc = GOOFY_OK;
     const int bpls[] = {1, 2, 4}, wgs[] = {2, 4, 8}, wpcs[] = {0, 8, 16, 32}, nts[] = {0, 1}, orders[] = {0, 1};
-    for (int bpl : bpls) {
-        b->cfg.blocks_per_lane = bpl;
-        if ((rc = build_worklist(b)) != GOOFY_OK) break;
+    for (int bpl : bpls)
         for (int wg : wgs)
             for (int wpc : wpcs)
                 for (int nt : nts)
                     for (int order : orders) {
-                        b->cfg = LaunchCfg{bpl, wg, wpc, nt, order};
+                        if ((rc = set_shape(b, LaunchCfg{bpl, wg, wpc, nt, order})) != GOOFY_OK) goto done;
                         // one warm-up launch, then the median of `reps` timed ones
-                        e = launch_batch(b->cfg, b->d_descs, (uint32_t)b->descs.size(), b->ntiles, b->num_cus, s, b->alpha);
+                        e = launch(b, s, nullptr);
                         if (e != hipSuccess) { rc = fail_hip(e, "autotune launch"); goto done; }
                         std::vector<float> ts;
                         for (int r = 0; r < reps; ++r) {
                             (void)hipEventRecord(e0, s);
-                            e = launch_batch(b->cfg, b->d_descs, (uint32_t)b->descs.size(), b->ntiles, b->num_cus, s, b->alpha);
+                            e = launch(b, s, nullptr);
                             (void)hipEventRecord(e1, s);
                             if (e != hipSuccess) { rc = fail_hip(e, "autotune launch"); goto done; }
                             e = hipEventSynchronize(e1);
@@ -357,17 +373,11 @@ int goofy_batch_autotune(goofy_batch* b, void* stream, int reps, goofy_launch_co
                             best = b->cfg;
                         }
                     }
-    }
 done:
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    if (rc != GOOFY_OK) {
-        b->cfg = start;
-        (void)build_worklist(b);
-        return rc;
-    }
-    b->cfg = best;
-    if ((rc = build_worklist(b)) != GOOFY_OK) return rc;
+    (void)set_shape(b, rc == GOOFY_OK ? best : start);  // both have their lists
+    if (rc != GOOFY_OK) return rc;
     {
         std::lock_guard<std::mutex> lock(g_tune_mu);
         tune_cache()[shape_key(b)] = best;
@@ -384,7 +394,7 @@ int goofy_batch_info(const goofy_batch* b, uint64_t* textures, uint64_t* blocks,
     if (!b) return fail(GOOFY_ERR_INVALID, "null batch");
     if (textures) *textures = b->textures.size();
     if (blocks) *blocks = b->blocks;
-    if (tiles) *tiles = b->ntiles;
+    if (tiles) *tiles = b->list->ntiles;
     if (pixels) *pixels = b->pixels;
     return GOOFY_OK;
 }
@@ -395,7 +405,8 @@ int goofy_batch_destroy(goofy_batch* b)
     if (!b) return GOOFY_OK;
     (void)wait_launched(b);
     if (b->launched) (void)hipEventDestroy(b->launched);
-    if (b->d_descs) (void)hipFree(b->d_descs);
+    for (const Worklist& l : b->lists)
+        if (l.d) (void)hipFree(l.d);
     delete b;
     return GOOFY_OK;
 }

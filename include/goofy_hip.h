@@ -282,8 +282,11 @@ typedef struct goofy_batch goofy_batch;
  * themselves stay owned by the caller). */
 GOOFY_HIP_API int goofy_batch_create(const goofy_texture_desc* textures, size_t count,
                                      const goofy_launch_config* cfg, goofy_batch** out);
-/* Enqueue the whole batch on `stream`: one kernel launch (a node of the graph
- * when the stream is being captured). */
+/* Enqueue the whole batch on `stream`: one kernel launch.  When the stream is
+ * being captured, the launch becomes a node of the graph, which keeps the shape
+ * and reads the work-list that the plan has now: set_config and autotune do not
+ * change it, but the plan must outlive the graph's last replay, and replays are
+ * the caller's to wait for. */
 GOOFY_HIP_API int goofy_batch_launch(goofy_batch* batch, void* stream);
 /* Same work as individual launches (one plain kernel per texture, or per
  * horizontal stripe for textures beyond one launch's index range), for
@@ -296,8 +299,9 @@ GOOFY_HIP_API int goofy_batch_autotune(goofy_batch* batch, void* stream, int rep
                                        float* best_ms);
 GOOFY_HIP_API int goofy_batch_get_config(const goofy_batch* batch, goofy_launch_config* cfg);
 /* set_config, autotune and destroy first wait for the plan's earlier
- * goofy_batch_launch calls to finish (on whatever stream they were issued),
- * since they rewrite or free the device work-list those launches read. */
+ * goofy_batch_launch calls to finish (on whatever stream they were issued).
+ * A plan has one device work-list per blocks_per_lane that it has been given;
+ * destroy frees them. */
 GOOFY_HIP_API int goofy_batch_set_config(goofy_batch* batch, const goofy_launch_config* cfg);
 /* Totals of the plan: textures, 4x4 blocks, wave tiles, pixels. */
 GOOFY_HIP_API int goofy_batch_info(const goofy_batch* batch, uint64_t* textures, uint64_t* blocks, uint64_t* tiles,

@@ -544,6 +544,53 @@ def test_batch_captured_then_replayed_and_reshaped(gpu, oracle, mode):
     s2.destroy()
 
 
+def test_batch_graph_outlives_reshapes(gpu, oracle):
+    """A graph that captured a batch launch gives the blocks after the plan
+    has taken other tile sizes, and beside launches of the new shapes: it
+    keeps the work-list it was captured with."""
+    import ctypes
+
+    from goofy_amd import hip
+    sizes = [(64, 64), (68, 20), (260, 132), (1028, 4)]
+    items, want = [], []
+    for i, (w, h) in enumerate(sizes):
+        img = gpu.synth_host(0, 60 + i, i, 12, w, h)
+        items.append(dict(src=hip.DeviceBuffer.from_array(img), dst=hip.DeviceBuffer((w // 4) * (h // 4) * 8, fill=0xCD),
+                          width=w, height=h, format=i & 1))
+        want.append(oracle.compress_blocks(i & 1, img, w, h, w * 4))
+    b = gpu.Batch(items)
+
+    def check(tag):
+        hip.synchronize()
+        for it, wv in zip(items, want):
+            assert np.array_equal(it["dst"].download(), wv), tag
+            it["dst"].fill(0xCD)
+        hip.synchronize()
+
+    rt, s = hip._hip, hip.Stream()
+    hip.synchronize()
+    runs = []
+    for bpl in (1, 4, 2):
+        b.config = dict(blocks_per_lane=bpl, wg_waves=4, waves_per_cu=0, nontemporal=1, tile_order=0)
+        graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+        assert rt.hipStreamBeginCapture(ctypes.c_void_p(s.handle), 2) == 0
+        b.launch(s)
+        assert rt.hipStreamEndCapture(ctypes.c_void_p(s.handle), ctypes.byref(graph)) == 0
+        assert rt.hipGraphInstantiate(ctypes.byref(run), graph, None, None, 0) == 0
+        runs.append((graph, run))
+        for r in range(2):
+            for i, (_, x) in enumerate(runs):
+                say(f"batch graph {i} of {len(runs)}, replay {r}, plan at {bpl} blocks per lane")
+                assert rt.hipGraphLaunch(x, ctypes.c_void_p(s.handle)) == 0
+                check(f"graph {i} replay {r}, plan at {bpl}")
+            b.launch(s)
+            check(f"eager {r}, plan at {bpl}")
+    for graph, run in runs:
+        assert rt.hipGraphExecDestroy(run) == 0 and rt.hipGraphDestroy(graph) == 0
+    b.close()
+    s.destroy()
+
+
 def test_batch_full_workload(gpu, oracle):
     """The 4096-texture workload: batch output equals per-texture launches on
     every texture, and the oracle on a sample of textures."""

@@ -158,3 +158,25 @@ def test_device_code_has_no_v_ashr_pk_u8_i32(tmp_path, source):
     text = asm.read_text()
     assert "v_lerp_u8" in text or source != "kernels.hip"  # the dump is the real kernels
     assert "v_ashr_pk_u8_i32" not in text
+
+
+@pytest.fixture(scope="module")
+def batch_lists(tmp_path_factory):
+    """tests/native/batch_lists_test.cpp: the batch planner against a device
+    that runs nothing until it is told to, under AddressSanitizer."""
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    exe = tmp_path_factory.mktemp("batch") / "batch_lists_test"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", f"-I{ROOT / 'include'}", f"-I{ROOT / 'goofy_amd' / 'csrc'}",
+                    str(ROOT / "tests" / "native" / "batch_lists_test.cpp"),
+                    str(ROOT / "goofy_amd" / "csrc" / "batch.cpp"), "-pthread", "-o", str(exe)], check=True)
+    return exe
+
+
+@pytest.mark.parametrize("name", ["captured"])
+def test_batch_worklists_on_host(batch_lists, name):
+    """No launch, and no replay of a captured one, reads a work-list that the
+    plan has rewritten, resized or freed since."""
+    r = subprocess.run([str(batch_lists), name], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "errors=0" in r.stdout, r.stdout + r.stderr
