@@ -50,23 +50,62 @@ struct goofy_batch {
     uint64_t blocks = 0, pixels = 0;
     bool alpha = false;  // holds DXT5 / ETC2 RGBA8 textures
     LaunchCfg cfg{};
-    // Recorded by every launch's own dispatch, for the calls that wait for the
-    // plan's launches.
-    hipEvent_t launched = nullptr;
-    bool launched_pending = false;
+    // The launches that the plan's other calls wait for: of each stream the
+    // last one, by an event that its own dispatch records.
+    struct Launched {
+        hipStream_t stream;
+        hipEvent_t ended;
+        bool pending;
+    };
+    std::vector<Launched> launched;
+    std::mutex launch_mu;  // of `launched`, for launches from several threads
 };
 
 namespace {
 
-// Waits for the plan's last launch (which may be on a caller's
-// non-blocking stream, which a synchronous copy does not wait for).
+// Waits for the plan's launches, on whatever stream.
 int wait_launched(goofy_batch* b)
 {
-    if (!b->launched_pending) return GOOFY_OK;
-    const hipError_t e = hipEventSynchronize(b->launched);
-    if (e != hipSuccess) return fail_hip(e, "hipEventSynchronize(batch launch)");
-    b->launched_pending = false;
+    std::lock_guard<std::mutex> lock(b->launch_mu);
+    for (goofy_batch::Launched& l : b->launched) {
+        if (!l.pending) continue;
+        const hipError_t e = hipEventSynchronize(l.ended);
+        if (e != hipSuccess) return fail_hip(e, "hipEventSynchronize(batch launch)");
+        l.pending = false;
+    }
     return GOOFY_OK;
+}
+
+// The entry for a launch on stream s: the stream's own, whose earlier launches
+// end before this one; else one whose launch has ended; else a new one.  The
+// per-thread default stream's handle names another stream in each thread, so
+// it never has one of its own.  Events are looked at only from the eighth entry
+// on: a plan that is launched on a few streams makes no call for them here.
+hipError_t launch_entry(goofy_batch* b, hipStream_t s, goofy_batch::Launched** out)
+{
+    constexpr size_t kLook = 8;
+    goofy_batch::Launched* found = nullptr;
+    if (s != hipStreamPerThread)
+        for (goofy_batch::Launched& l : b->launched)
+            if (l.stream == s) found = &l;
+    for (size_t i = 0; !found && i < b->launched.size(); ++i)
+        if (!b->launched[i].pending) found = &b->launched[i];
+    for (size_t i = 0; !found && b->launched.size() >= kLook && i < b->launched.size(); ++i) {
+        if (hipEventQuery(b->launched[i].ended) == hipSuccess) found = &b->launched[i];
+        else (void)hipGetLastError();
+    }
+    if (!found) {
+        hipEvent_t ev;
+        const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (e != hipSuccess) return e;
+        b->launched.push_back({s, ev, false});
+        found = &b->launched.back();
+    } else if (found->stream != s || s == hipStreamPerThread) {
+        found->stream = s;
+        found->pending = false;
+    }
+    *out = found;
+    return hipSuccess;
 }
 
 // Makes the work-list of tiles of `tile` blocks.
@@ -267,9 +306,6 @@ int goofy_batch_launch(goofy_batch* b, void* stream)
     if (!b) return fail(GOOFY_ERR_INVALID, "null batch");
     if (b->list->ntiles == 0) return GOOFY_OK;
     const hipStream_t s = (hipStream_t)stream;
-    hipError_t e;
-    if (!b->launched && (e = hipEventCreateWithFlags(&b->launched, hipEventDisableTiming)) != hipSuccess)
-        return fail_hip(e, "hipEventCreate");
     // One kernel: a plain launch.  A hipGraph of this one node cost the host
     // 15-17 us a launch on MI355X (4 ms the first time), the kernel launch
     // 2.8 us, and an event recorded behind it 5 us more than one that the
@@ -277,11 +313,17 @@ int goofy_batch_launch(goofy_batch* b, void* stream)
     // the launch as a node, without the event.
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();  // the launch says why
-    const bool eager = cap == hipStreamCaptureStatusNone;
-    e = launch(b, s, eager ? b->launched : nullptr);
-    if (e != hipSuccess) return fail_hip(e, "batch kernel launch");
-    if (eager) b->launched_pending = true;
-    return GOOFY_OK;
+    hipError_t e;
+    if (cap != hipStreamCaptureStatusNone) {
+        e = launch(b, s, nullptr);
+    } else {
+        std::lock_guard<std::mutex> lock(b->launch_mu);
+        goofy_batch::Launched* l = nullptr;
+        if ((e = launch_entry(b, s, &l)) != hipSuccess) return fail_hip(e, "hipEventCreate");
+        e = launch(b, s, l->ended);
+        if (e == hipSuccess) l->pending = true;
+    }
+    return e == hipSuccess ? GOOFY_OK : fail_hip(e, "batch kernel launch");
 }
 
 int goofy_batch_launch_per_texture(goofy_batch* b, void* stream)
@@ -404,7 +446,7 @@ int goofy_batch_destroy(goofy_batch* b)
     clear_error();
     if (!b) return GOOFY_OK;
     (void)wait_launched(b);
-    if (b->launched) (void)hipEventDestroy(b->launched);
+    for (const goofy_batch::Launched& l : b->launched) (void)hipEventDestroy(l.ended);
     for (const Worklist& l : b->lists)
         if (l.d) (void)hipFree(l.d);
     delete b;

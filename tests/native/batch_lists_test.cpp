@@ -52,6 +52,7 @@ std::map<hipEvent_t, std::pair<uint64_t, uint64_t>> g_event;  // recorded, reach
 std::map<hipEvent_t, hipStream_t> g_event_stream;
 std::set<hipStream_t> g_capturing;
 std::vector<Launch> g_captured;
+hipStream_t g_per_thread = nullptr;  // what hipStreamPerThread names now
 uint64_t g_ticket = 0, g_runs = 0, g_events_made = 0;
 uintptr_t g_next_event = 0x1000;
 std::vector<int> g_hits;  // of each block (by destination address / 8)
@@ -96,6 +97,7 @@ bool reached(hipEvent_t e) { return g_event[e].second >= g_event[e].first; }
 
 hipError_t push(hipStream_t s, bool kernel, const Launch& l, hipEvent_t e)
 {
+    if (s == hipStreamPerThread) s = g_per_thread;
     if (g_capturing.count(s)) {
         if (kernel) g_captured.push_back(l);
         return hipSuccess;
@@ -198,7 +200,7 @@ hipError_t launch_batch(const LaunchCfg& c, const TexDesc* d, uint32_t ntex, uin
 
 namespace {
 
-const hipStream_t kA = (hipStream_t)0x100, kB = (hipStream_t)0x200, kPerThread = hipStreamPerThread;
+const hipStream_t kA = (hipStream_t)0x100, kB = (hipStream_t)0x200;
 
 // 8-byte formats; sizes whose last tiles are ragged at every tile size
 goofy_batch* make_plan()
@@ -263,10 +265,77 @@ void captured()
     finish(b);
 }
 
+uint64_t left(hipStream_t s)
+{
+    uint64_t n = 0;
+    for (const Op& op : g_queue[s]) n += op.kernel;
+    return n;
+}
+
+// set_config, autotune and destroy wait for the launches of every stream.
+void streams()
+{
+    goofy_batch* b = make_plan();
+    const goofy_launch_config same = shape(1), other = shape(4);
+    for (const goofy_launch_config* c : {&same, &other, &same}) {
+        for (hipStream_t s : {kA, kA, kB, (hipStream_t) nullptr})
+            CHECK(goofy_batch_launch(b, s) == GOOFY_OK, "launch");
+        CHECK(left(kA) == 2 && left(kB) == 1 && left(nullptr) == 1, "launches wait for nothing");
+        CHECK(goofy_batch_set_config(b, c) == GOOFY_OK, "set_config");
+        CHECK(left(kA) + left(kB) + left(nullptr) == 0, "launches left after set_config: %d %d %d", (int)left(kA),
+              (int)left(kB), (int)left(nullptr));
+        covered(4, "launches on three streams");
+    }
+    for (hipStream_t s : {kB, kA}) CHECK(goofy_batch_launch(b, s) == GOOFY_OK, "launch");
+    CHECK(goofy_batch_autotune(b, kB, 1, nullptr, nullptr) == GOOFY_OK, "autotune");
+    CHECK(left(kA) == 0, "launches left after autotune");
+    advance(kB, g_ticket);
+    for (hipStream_t s : {kA, kB}) CHECK(goofy_batch_launch(b, s) == GOOFY_OK, "launch");
+    CHECK(goofy_batch_destroy(b) == GOOFY_OK, "destroy");
+    CHECK(left(kA) + left(kB) == 0, "launches left after destroy: %d %d", (int)left(kA), (int)left(kB));
+    CHECK(g_memory.empty() && g_event.empty(), "%zu allocations, %zu events left", g_memory.size(), g_event.size());
+    g_queue.clear();
+}
+
+// The handle of the per-thread default stream names another stream in every
+// thread: here its launches alternate between two.
+void per_thread()
+{
+    goofy_batch* b = make_plan();
+    for (hipStream_t s : {kA, kB}) {
+        g_per_thread = s;
+        CHECK(goofy_batch_launch(b, hipStreamPerThread) == GOOFY_OK, "launch");
+    }
+    const goofy_launch_config c = shape(2);
+    CHECK(goofy_batch_set_config(b, &c) == GOOFY_OK, "set_config");
+    CHECK(left(kA) + left(kB) == 0, "launches left after set_config: %d %d", (int)left(kA), (int)left(kB));
+    covered(2, "launches on two threads' streams");
+    finish(b);
+}
+
+// As many events as streams with unfinished launches, or a few more, not as
+// launches or streams.
+void events()
+{
+    goofy_batch* b = make_plan();
+    for (int i = 0; i < 1000; ++i) {
+        CHECK(goofy_batch_launch(b, kA) == GOOFY_OK, "launch");
+        CHECK(goofy_batch_launch(b, kB) == GOOFY_OK, "launch");
+    }
+    CHECK(g_events_made == 2, "%d events for two streams", (int)g_events_made);
+    for (int i = 0; i < 1000; ++i) {
+        const hipStream_t s = (hipStream_t)(uintptr_t)(0x1000 + 16 * i);
+        CHECK(goofy_batch_launch(b, s) == GOOFY_OK, "launch");
+        advance(s, g_ticket);
+    }
+    CHECK(g_events_made <= 8, "%d events for three streams at a time", (int)g_events_made);
+    finish(b);
+}
+
 const struct {
     const char* name;
     void (*go)();
-} kTests[] = {{"captured", captured}};
+} kTests[] = {{"captured", captured}, {"streams", streams}, {"per_thread", per_thread}, {"events", events}};
 
 }  // namespace
 

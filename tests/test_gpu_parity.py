@@ -591,6 +591,34 @@ def test_batch_graph_outlives_reshapes(gpu, oracle):
     s.destroy()
 
 
+def test_batch_reshape_waits_for_every_stream(gpu):
+    """set_config waits for the plan's launches on all streams: one stands
+    behind milliseconds of other work, the later ones on idle streams."""
+    import ctypes
+
+    from goofy_amd import hip
+    n = 4096
+    big, out = dev_buffer(n * n * 4), dev_buffer(n * n // 2)
+    src, dst = dev_buffer(64 * 64 * 4), dev_buffer(64 * 64 // 2)
+    b = gpu.Batch([dict(src=src, dst=dst, width=64, height=64, format=0)])
+    streams = [hip.Stream() for _ in range(3)]
+    shape = dict(blocks_per_lane=1, wg_waves=4, waves_per_cu=0, nontemporal=1, tile_order=0)
+    hip.synchronize()
+    for bpl in (1, 2):
+        say(f"batch reshape to {bpl} behind three streams")
+        for _ in range(400):  # 12 us each
+            gpu.compress_device(0, out, big, n, n, n * 4, stream=streams[0])
+        behind = hip.Event().record(streams[0])
+        for s in streams:
+            b.launch(s)
+        b.config = dict(shape, blocks_per_lane=bpl)
+        assert hip._hip.hipEventQuery(ctypes.c_void_p(behind.handle)) == 0
+    b.close()
+    hip.synchronize()
+    for s in streams:
+        s.destroy()
+
+
 def test_batch_full_workload(gpu, oracle):
     """The 4096-texture workload: batch output equals per-texture launches on
     every texture, and the oracle on a sample of textures."""

@@ -174,9 +174,10 @@ def batch_lists(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["captured"])
+@pytest.mark.parametrize("name", ["captured", "streams", "per_thread", "events"])
 def test_batch_worklists_on_host(batch_lists, name):
     """No launch, and no replay of a captured one, reads a work-list that the
-    plan has rewritten, resized or freed since."""
+    plan has rewritten, resized or freed since; and the calls that wait for the
+    plan's launches wait for those of every stream."""
     r = subprocess.run([str(batch_lists), name], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and "errors=0" in r.stdout, r.stdout + r.stderr
