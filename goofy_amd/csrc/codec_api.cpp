@@ -186,6 +186,11 @@ static int run_quality(uint64_t pixels, uint32_t height, uint32_t max_rows, hipS
     DeviceInfo di;
     int rc = device_info(&di);
     if (rc != GOOFY_OK) return rc;
+    // The figures are read back here, so the call cannot be captured: a replay
+    // would only add to a work area that other calls use by then.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();  // the launch says why
+    if (cap != hipStreamCaptureStatusNone) return fail(GOOFY_ERR_HIP, "quality call on a stream that is being captured");
     struct Use {  // on every path, the launches are through with the slot before it is reused
         QualitySlot slot;
         hipStream_t s;
@@ -200,9 +205,6 @@ static int run_quality(uint64_t pixels, uint32_t height, uint32_t max_rows, hipS
     } use{quality_scratch_pool().acquire(di.device), stream};
     const QualitySlot& slot = use.slot;
     if (!slot.d) return fail(GOOFY_ERR_OUT_OF_MEMORY, "quality scratch");
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();  // the launch says why
-    const bool eager = cap == hipStreamCaptureStatusNone;
     hipError_t e = hipSuccess;
     if (!slot.clean && (e = hipMemsetAsync(slot.d, 0, sizeof(QualityAccum), stream)) != hipSuccess)
         return fail_hip(e, "quality work area");
@@ -216,8 +218,8 @@ static int run_quality(uint64_t pixels, uint32_t height, uint32_t max_rows, hipS
             if (e != hipSuccess) return fail_hip(e, "quality kernel launch");
             y0 += rows;
         }
-        if (eager && hipEventRecord(slot.ended, stream) != hipSuccess) (void)hipGetLastError();
-        if (!(eager && words_arrive(slot.h, n)) && (e = hipStreamSynchronize(stream)) != hipSuccess)
+        if (hipEventRecord(slot.ended, stream) != hipSuccess) (void)hipGetLastError();
+        if (!words_arrive(slot.h, n) && (e = hipStreamSynchronize(stream)) != hipSuccess)
             return fail_hip(e, "quality readback");
         for (uint32_t i = 0; i < n; ++i) {
             for (int k = 0; k < 5; ++k) sums.sum[k] += slot.h[i].word[k];

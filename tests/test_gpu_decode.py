@@ -538,6 +538,40 @@ def test_quality_call_refused_under_capture_leaves_no_trace(gpu):
         assert gpu.quality_images_device(da, db, w, h)["sse_byte"] == sse
 
 
+def test_quality_call_refused_under_capture_queues_nothing(gpu):
+    """The refused call leaves the capture as it was: it ends well, and holds
+    the one encode that was captured beside it."""
+    import ctypes
+
+    from goofy_amd import hip
+    w, h = 256, 64
+    img = gpu.synth_host(0, 21, 0, 12, w, h)
+    src, out = hip.DeviceBuffer.from_array(img), hip.DeviceBuffer(w * h // 2, fill=0xCD)
+    blocks = hip.DeviceBuffer(w * h // 2)
+    gpu.compress_device(W.DXT1, blocks, src, w, h, w * 4)
+    hip.synchronize()
+    s, rt = hip.Stream(), hip._hip
+    graph, run, n = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_size_t()
+    assert rt.hipStreamBeginCapture(ctypes.c_void_p(s.handle), 2) == 0  # relaxed
+    gpu.compress_device(W.DXT1, out, src, w, h, w * 4, stream=s)
+    for _ in range(2):
+        with pytest.raises(gpu.GoofyError) as e:
+            gpu.quality_device(W.DXT1, blocks, src, w, h, stream=s)
+        assert e.value.status == gpu.ERR_HIP
+    assert rt.hipStreamEndCapture(ctypes.c_void_p(s.handle), ctypes.byref(graph)) == 0
+    assert rt.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0 and n.value == 1
+    assert rt.hipGraphInstantiate(ctypes.byref(run), graph, None, None, 0) == 0
+    for _ in range(3):
+        assert rt.hipGraphLaunch(run, ctypes.c_void_p(s.handle)) == 0
+        s.synchronize()
+        assert np.array_equal(out.download(), blocks.download())
+        out.fill(0xCD)
+        hip.synchronize()
+        gpu.quality_device(W.DXT1, blocks, src, w, h, stream=s)
+    assert rt.hipGraphExecDestroy(run) == 0 and rt.hipGraphDestroy(graph) == 0
+    s.destroy()
+
+
 def test_quality_calls_from_threads_share_the_scratch_pool(gpu):
     """Quality calls on four threads and streams at once (the library keeps a
     pool of scratch buffers): every result equals the same call made alone."""
