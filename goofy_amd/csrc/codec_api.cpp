@@ -222,6 +222,8 @@ static int run_quality(uint64_t pixels, uint32_t height, uint32_t max_rows, hipS
         if (!words_arrive(slot.h, n) && (e = hipStreamSynchronize(stream)) != hipSuccess)
             return fail_hip(e, "quality readback");
         for (uint32_t i = 0; i < n; ++i) {
+            for (uint64_t w : slot.h[i].word)
+                if (w == kQualityNone) return fail(GOOFY_ERR_HIP, "quality kernel ended without its sums");
             for (int k = 0; k < 5; ++k) sums.sum[k] += slot.h[i].word[k];
             sums.sum[4] += slot.h[i].word[5] << 32;
         }

@@ -134,10 +134,27 @@ void capture()
         }
 }
 
+// Words that are still unwritten when the stream has drained are an error, not
+// figures; the next call clears the work area and is right.
+void unwritten()
+{
+    for (auto call : {images, blocks}) {
+        goofy_quality q{};
+        q.pixels = 7;
+        g_writes = false;
+        CHECK(call(&q) == GOOFY_ERR_HIP, "no words");
+        CHECK(q.pixels == 7, "figures from no words");
+        g_writes = true;
+        g_n = {};
+        right(call, "after a call without words");
+        CHECK(g_n.memset == 1, "%d memsets", g_n.memset);
+    }
+}
+
 const struct {
     const char* name;
     void (*go)();
-} kTests[] = {{"capture", capture}};
+} kTests[] = {{"capture", capture}, {"unwritten", unwritten}};
 
 }  // namespace
 

@@ -197,9 +197,10 @@ def quality_host(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["capture"])
+@pytest.mark.parametrize("name", ["capture", "unwritten"])
 def test_quality_calls_on_host(quality_host, name):
-    """capture: a quality call on a capturing stream queues nothing."""
+    """capture: a quality call on a capturing stream queues nothing; unwritten:
+    words that no kernel wrote give an error."""
     import os
     r = subprocess.run([str(quality_host), name], capture_output=True, text=True, timeout=120,
                        env={**os.environ, "ASAN_OPTIONS": "detect_leaks=0"})  # work areas are kept for good
