@@ -194,9 +194,13 @@ GOOFY_HIP_API int goofy_hip_decode_device(int format, void* d_rgba, const void* 
  * an MSE below 1e-7 gives DBL_MAX.  Synchronous on `stream`: the call returns
  * when the work queued there before it and its own kernel's have been done
  * (the kernel's sums are in host memory).  The stream may report itself busy
- * for some microseconds more, and what earlier kernels wrote to host memory
- * that was allocated non-coherent shows after a synchronisation of the
- * stream, which this call queues but does not wait for.  Uses a 4 KiB device
+ * for some microseconds more.  An error of earlier work that keeps the kernel
+ * from running is returned; any other is left to the next call that waits for
+ * the stream.  What earlier kernels wrote to host memory can be read, in
+ * non-coherent allocations too: at its end a kernel's writes are visible to
+ * the whole GPU, whose eight L2s keep none of them back (a partition of one
+ * XCD may, and shows such memory after a synchronisation).  A stream that is being captured is refused
+ * (GOOFY_ERR_HIP) with nothing queued.  Uses a 4 KiB device
  * work area and 768 bytes of pinned host memory, into which the
  * kernel writes the sums, from a per-device pool (allocated on first use,
  * never freed, one pair per concurrent call), so a call never waits on other

@@ -538,6 +538,82 @@ def test_quality_call_refused_under_capture_leaves_no_trace(gpu):
         assert gpu.quality_images_device(da, db, w, h)["sse_byte"] == sse
 
 
+@pytest.mark.parametrize("own_stream", [False, True])
+def test_quality_call_returns_behind_earlier_work(gpu, own_stream):
+    """When a quality call returns, the work queued on its stream before it has
+    been done: the encode that writes the very blocks it measures, behind some
+    milliseconds of others, and an event behind them."""
+    import ctypes
+
+    from goofy_amd import hip
+    n, w = 4096, 512
+    big, out = hip.DeviceBuffer(n * n * 4, fill=0x55), hip.DeviceBuffer(n * n // 2)
+    srcs = [hip.DeviceBuffer.from_array(gpu.synth_host(0, 70 + i, 0, 12, w, w)) for i in range(2)]
+    blocks = hip.DeviceBuffer(w * w // 2)
+    want = []
+    for src in srcs:
+        gpu.compress_device(W.DXT1, blocks, src, w, w, w * 4)
+        hip.synchronize()
+        want.append((blocks.download(), gpu.quality_device(W.DXT1, blocks, src, w, w)))
+    assert want[0][1] != want[1][1]
+    s = hip.Stream() if own_stream else None
+    hip.synchronize()
+    for i in range(6):
+        print(f"quality behind the encode it measures, {i}", flush=True)
+        for _ in range(40 * i):  # 12 us each: words that come at once, and after the time for looking at them
+            gpu.compress_device(W.DXT1, out, big, n, n, n * 4, stream=s)
+        gpu.compress_device(W.DXT1, blocks, srcs[i & 1], w, w, w * 4, stream=s)
+        behind = hip.Event().record(s)
+        assert gpu.quality_device(W.DXT1, blocks, srcs[i & 1], w, w, stream=s) == want[i & 1][1]
+        assert hip._hip.hipEventQuery(ctypes.c_void_p(behind.handle)) == 0
+        assert np.array_equal(blocks.download(), want[i & 1][0])
+    if s:
+        s.destroy()
+
+
+@pytest.mark.parametrize("flags", [0x40000000, 0x80000000])  # coherent, non-coherent
+def test_quality_call_shows_earlier_results_in_host_memory(gpu, flags):
+    """What kernels queued before a quality call wrote to pinned host memory
+    is there when the call returns, in non-coherent memory too: a fill, an
+    encode and a decode with cached or streaming stores."""
+    import ctypes
+
+    from goofy_amd import hip
+    rt = hip._hip
+    w, h, cap = 1028, 252, 1 << 20
+    print(f"earlier results in host memory, flags {flags:#x}", flush=True)
+    ptr = ctypes.c_void_p()
+    assert rt.hipHostMalloc(ctypes.byref(ptr), cap + (w * 4 * h), flags) == 0
+    host = np.ctypeslib.as_array((ctypes.c_uint8 * cap).from_address(ptr.value))
+    imgs, blocks, decoded = [], [], []
+    for i in range(2):
+        imgs.append(hip.DeviceBuffer.from_array(gpu.synth_host(0, 80 + i, 0, 12, w, h)))
+        blocks.append(hip.DeviceBuffer((w // 4) * (h // 4) * 8))
+        gpu.compress_device(W.DXT1, blocks[i], imgs[i], w, h, w * 4)
+        px = hip.DeviceBuffer(w * 4 * h)
+        gpu.decode_device(W.DXT1, px, blocks[i], w, h)
+        hip.synchronize()
+        decoded.append(px.download())
+    encoded = [b.download() for b in blocks]
+    for s in (None, hip.Stream()):
+        handle = ctypes.c_void_p(int(s) if s else None)
+        for it in range(100):
+            i = it & 1
+            assert rt.hipMemsetAsync(ptr, it, cap, handle) == 0
+            gpu.quality_images_device(imgs[0], imgs[1], w, h, stream=s)
+            assert (host == it).all(), it
+            gpu.compress_device(W.DXT1, ptr.value, imgs[i], w, h, w * 4, stream=s)
+            gpu.quality_images_device(imgs[0], imgs[1], w, 4, stream=s)
+            assert np.array_equal(host[:encoded[i].size], encoded[i]), it
+            gpu.decode_device(W.DXT1, ptr.value, blocks[i], w, h, stream=s)
+            gpu.quality_images_device(imgs[0], imgs[1], w, 4, stream=s)
+            assert np.array_equal(host[:min(cap, decoded[i].size)], decoded[i][:cap]), it
+        hip.synchronize()
+        if s:
+            s.destroy()
+    assert rt.hipHostFree(ptr) == 0
+
+
 def test_quality_call_refused_under_capture_queues_nothing(gpu):
     """The refused call leaves the capture as it was: it ends well, and holds
     the one encode that was captured beside it."""
