@@ -137,6 +137,7 @@ bool cfg_valid(const LaunchCfg& c)
 
 constexpr int kSlots = 3;
 constexpr uint64_t kFeedPatience = 2000000;  // 20 ms in 10 ns ticks
+constexpr size_t kWidePart = (size_t)1 << 20;
 
 // Whether a launch returns only when its kernel has ended.
 static bool launches_block()
@@ -229,12 +230,13 @@ static int ensure_ctx(StagingCtx* c, size_t in_bytes, size_t out_bytes)
     return GOOFY_OK;
 }
 
-// Copy `rows` rows of `row_bytes` from src (stride) to dst (packed).
-static void copy_rows(uint8_t* dst, const uint8_t* src, size_t stride, size_t row_bytes, size_t rows)
+// Copy `rows` rows of `bytes` from src to dst, which are `stride` and `pitch`
+// apart.
+static void copy_rows(uint8_t* dst, size_t pitch, const uint8_t* src, size_t stride, size_t bytes, size_t rows)
 {
-    if (stride == row_bytes) std::memcpy(dst, src, row_bytes * rows);
+    if (stride == bytes && pitch == bytes) std::memcpy(dst, src, bytes * rows);
     else
-        for (size_t r = 0; r < rows; ++r) std::memcpy(dst + r * row_bytes, src + r * stride, row_bytes);
+        for (size_t r = 0; r < rows; ++r) std::memcpy(dst + r * pitch, src + r * stride, bytes);
 }
 
 // Marks every part of a launched chunk on the way out: all are marked already
@@ -269,17 +271,18 @@ struct HostImage {
     unsigned char* result;
     unsigned char* result2;  // a pair's second format, or null
     const unsigned char* input;
-    size_t stride, row_bytes, block_bytes;
+    size_t stride, block_bytes;
     uint32_t bw;
     size_t part_bytes;  // about what a part of a chunk holds
     uint64_t patience;
 };
 
-// The k-th chunk: `rows` block rows from the y0-th on, launched as number
+// The k-th chunk: `rows` block rows from the y0-th on, of them the `cols` block
+// columns from the x0-th on (all of them unless rows is 1), launched as number
 // `call`; of its groups of kFeedBlocks blocks the first `got` are in the
 // caller's memory.
 struct HostChunk {
-    uint32_t k = 0, y0 = 0, rows = 0;
+    uint32_t k = 0, y0 = 0, rows = 0, x0 = 0, cols = 0;
     uint64_t call = 0;
     uint32_t got = 0;
 };
@@ -294,9 +297,9 @@ static void collect(const HostImage& im, const HostChunk& c, uint32_t first, uin
     const uint8_t* const out = slot_of(im, c).out;
     const size_t bb = im.block_bytes;
     const auto copy = [&](uint32_t a, uint32_t b) {
-        const size_t to = ((size_t)c.y0 * im.bw + a) * bb, n = (size_t)(b - a) * bb;
+        const size_t to = ((size_t)c.y0 * im.bw + c.x0 + a) * bb, n = (size_t)(b - a) * bb;
         std::memcpy(im.result + to, out + a * bb, n);
-        if (im.result2) std::memcpy(im.result2 + to, out + ((size_t)im.bw * c.rows + a) * bb, n);
+        if (im.result2) std::memcpy(im.result2 + to, out + ((size_t)c.cols * c.rows + a) * bb, n);
     };
     constexpr uint32_t kPiece = 8192;  // blocks
     if (last - first < 4u * kPiece) return copy(first, last);
@@ -310,16 +313,31 @@ static void collect(const HostImage& im, const HostChunk& c, uint32_t first, uin
 static hipError_t start_chunk(const HostImage& im, HostChunk& c)
 {
     const StagingCtx::Slot& slot = slot_of(im, c);
-    const uint32_t nblocks = im.bw * c.rows;
-    const size_t bytes = im.row_bytes * 4 * c.rows;
-    const uint8_t* const rows = im.input + (size_t)c.y0 * 4 * im.stride;
+    const uint32_t nblocks = c.cols * c.rows;
+    const size_t row_bytes = (size_t)c.cols * 16, bytes = row_bytes * 4 * c.rows;
+    const uint8_t* const rows = im.input + (size_t)c.y0 * 4 * im.stride + (size_t)c.x0 * 16;
     const bool fed = bytes >= (128u << 10) && !im.ctx->stage_first;
-    // parts of whole block rows
-    const uint32_t want = (uint32_t)std::max<size_t>(1, std::min<size_t>(kFeedParts, bytes / im.part_bytes));
-    const uint32_t prows = (c.rows + want - 1) / want, parts = (c.rows + prows - 1) / prows;
+    // Parts of whole block rows; where those have more than kWidePart, of
+    // blocks in order, so that several threads copy what one row holds and the
+    // kernel starts before all of it is staged (us per call, with parts of whole
+    // rows / so: 524288x16 1250 / 780, 4194288x8 5900 / 2730).
+    const bool wide = row_bytes * 4 > kWidePart;
+    const uint32_t want =
+        (uint32_t)(wide ? (bytes + kWidePart - 1) / kWidePart
+                        : std::max<size_t>(1, std::min<size_t>(kFeedParts, bytes / im.part_bytes)));
+    const uint32_t part_blocks = wide ? (nblocks + want - 1) / want : c.cols * ((c.rows + want - 1) / want);
+    const uint32_t parts = (nblocks + part_blocks - 1) / part_blocks;
     const auto stage = [&](uint32_t p) {
-        const size_t r0 = (size_t)p * prows * 4, n = std::min((size_t)prows * 4, (size_t)c.rows * 4 - r0);
-        copy_rows(slot.in + r0 * im.row_bytes, rows + r0 * im.stride, im.stride, im.row_bytes, n);
+        uint32_t b = p * part_blocks;
+        for (const uint32_t end = std::min(b + part_blocks, nblocks); b < end;) {
+            const uint32_t y = b / c.cols, x = b % c.cols;
+            // the rest of a block row, or all block rows of the part
+            const uint32_t n = wide ? std::min(end - b, c.cols - x) : end - b;
+            copy_rows(slot.in + (size_t)y * 4 * row_bytes + (size_t)x * 16, row_bytes,
+                      rows + (size_t)y * 4 * im.stride + (size_t)x * 16, im.stride,
+                      wide ? (size_t)n * 16 : row_bytes, wide ? 4 : (size_t)n / c.cols * 4);
+            b += n;
+        }
     };
     // one thread copies an image of 1 MiB at the link's rate, and waking others
     // takes longer (512x512: 38 us with one, 43 with them)
@@ -331,8 +349,8 @@ static hipError_t start_chunk(const HostImage& im, HostChunk& c)
     if (!fed) each_part(stage);
     c.call = ++im.ctx->call;
     const hipError_t e =
-        launch_fed(im.fmt, slot.in, im.row_bytes, slot.out, slot.out + nblocks * im.block_bytes, im.bw, nblocks,
-                   slot.feed, c.call, fed ? im.bw * prows : 0u, im.patience, stream_of(im, c));
+        launch_fed(im.fmt, slot.in, row_bytes, slot.out, slot.out + nblocks * im.block_bytes, c.cols, nblocks,
+                   slot.feed, c.call, fed ? part_blocks : 0u, im.patience, stream_of(im, c));
     if (e != hipSuccess || !fed) return e;
     const FeedGuard guard{slot.feed, c.call, parts};
     each_part([&](uint32_t p) {
@@ -345,7 +363,7 @@ static hipError_t start_chunk(const HostImage& im, HostChunk& c)
 // Collects the groups of a chunk that are marked, in order.
 static bool collect_marked(const HostImage& im, HostChunk& c)
 {
-    const uint32_t nblocks = im.bw * c.rows, groups = feed_groups(nblocks);
+    const uint32_t nblocks = c.cols * c.rows, groups = feed_groups(nblocks);
     const HostFeed* const feed = slot_of(im, c).feed;
     uint32_t to = c.got;
     while (to < std::min(groups, kFeedMarks) && __atomic_load_n(&feed->done[to], __ATOMIC_ACQUIRE) == c.call) ++to;
@@ -362,14 +380,14 @@ static hipError_t finish_chunk(const HostImage& im, HostChunk& c)
     for (uint32_t look = 1; !collect_marked(im, c); ++look) {
         if (c.got == kFeedMarks || (look % 64 == 0 && std::chrono::steady_clock::now() > end)) break;
     }
-    if (c.got == feed_groups(im.bw * c.rows)) return hipSuccess;
+    if (c.got == feed_groups(c.cols * c.rows)) return hipSuccess;
     const StagingCtx::Slot& slot = slot_of(im, c);
     const hipStream_t stream = stream_of(im, c);
-    const uint32_t nblocks = im.bw * c.rows;
+    const uint32_t nblocks = c.cols * c.rows;
     hipError_t e = hipStreamSynchronize(stream);
     if (e == hipSuccess && __atomic_load_n(&slot.feed->gave_up, __ATOMIC_ACQUIRE) == c.call) {
-        e = launch_any(im.fmt, im.cfg, slot.in, im.row_bytes, slot.out, slot.out + nblocks * im.block_bytes, im.bw,
-                       nblocks, stream);
+        e = launch_any(im.fmt, im.cfg, slot.in, (size_t)c.cols * 16, slot.out, slot.out + nblocks * im.block_bytes,
+                       c.cols, nblocks, stream);
         if (e == hipSuccess) e = hipStreamSynchronize(stream);
     }
     if (e == hipSuccess) collect(im, c, c.got * kFeedBlocks, nblocks);
@@ -412,14 +430,15 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
         }
     } rel{ctx};
 
-    const size_t row_bytes = (size_t)width * 4;
-    const unsigned chunk_brows = (unsigned)std::max<size_t>(1, (size_t(8) << 20) / (row_bytes * 4));  // ~8 MiB
-    const unsigned cb = std::min(std::min(chunk_brows, bh), max_rows);
+    // Chunks of about 8 MiB: block rows, or, where one has more, pieces of one.
+    const size_t row_bytes = (size_t)width * 4, chunk = (size_t)8 << 20;
+    const unsigned cb = std::min(std::min((unsigned)std::max<size_t>(1, chunk / (row_bytes * 4)), bh), max_rows);
+    const uint32_t pieces = (uint32_t)((row_bytes * 4 + chunk - 1) / chunk), cols = (bw + pieces - 1) / pieces;
     // dual: a chunk's staging output holds its blocks of the first format, then
     // those of the second
     const size_t outs = dual ? 2 : 1;
     const size_t bb = dual_alpha ? 16 : (dual ? 8 : block_bytes(fmt));
-    if ((rc = ensure_ctx(ctx, row_bytes * 4 * cb, outs * bw * cb * bb)) != GOOFY_OK) return rc;
+    if ((rc = ensure_ctx(ctx, (size_t)cols * 64 * cb, outs * cols * cb * bb)) != GOOFY_OK) return rc;
     // Parts of an image of one chunk: 64 KiB, or a thirty-second of it, so that
     // the kernel can start early.  Of larger ones: 1 MiB, copied as streams by
     // the threads; pieces of 256 KiB take 2 to 3 times as long from an image
@@ -427,16 +446,21 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
     // ms, in 1 MiB pieces 1.5) and are 1-2% faster on one that lies in the
     // caches.
     const size_t part_bytes = cb < bh ? (size_t)1 << 20 : (size_t)1 << 16;
-    const HostImage im{ctx,    fmt,       auto_cfg((uint64_t)bw * cb, di.num_cus), result, dual ? result2 : nullptr, input,
-                       stride, row_bytes, bb, bw, part_bytes, patience};
+    const HostImage im{ctx, fmt, auto_cfg((uint64_t)cols * cb, di.num_cus), result, dual ? result2 : nullptr, input,
+                       stride, bb, bw, part_bytes, patience};
     HostChunk ring[kSlots];  // chunks [oldest, k) are launched and not yet collected
     hipError_t e = hipSuccess;
     uint32_t k = 0, oldest = 0;
-    for (uint64_t y0 = 0; y0 < bh && e == hipSuccess; y0 += cb, ++k) {
+    for (uint64_t y0 = 0, x0 = 0; y0 < bh && e == hipSuccess; ++k) {
         if (k - oldest == kSlots && (e = finish_chunk(im, ring[oldest++ % kSlots])) != hipSuccess) break;
-        ring[k % kSlots] = HostChunk{k, (uint32_t)y0, std::min<uint32_t>(cb, bh - (uint32_t)y0)};
+        ring[k % kSlots] = HostChunk{k, (uint32_t)y0, std::min<uint32_t>(cb, bh - (uint32_t)y0), (uint32_t)x0,
+                                     std::min<uint32_t>(cols, bw - (uint32_t)x0)};
         e = start_chunk(im, ring[k % kSlots]);
         if (oldest < k) collect_marked(im, ring[oldest % kSlots]);
+        if ((x0 += cols) >= bw) {
+            x0 = 0;
+            y0 += cb;
+        }
     }
     // a marker behind the kernels while they run, for a caller that goes on to
     // wait for the device

@@ -205,3 +205,18 @@ def test_quality_calls_on_host(quality_host, name):
     r = subprocess.run([str(quality_host), name], capture_output=True, text=True, timeout=120,
                        env={**os.environ, "ASAN_OPTIONS": "detect_leaks=0"})  # work areas are kept for good
     assert r.returncode == 0 and "errors=0" in r.stdout, r.stdout + r.stderr
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_dropin_staging_on_host(tmp_path):
+    """tests/native/dropin_host_test.cpp: the drop-in's staging with threads
+    in place of its kernels, under ThreadSanitizer: every path and format, and
+    very wide rows in parts that several threads share."""
+    exe = tmp_path / "dropin_host_test"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=thread", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", f"-I{ROOT / 'include'}", f"-I{ROOT / 'goofy_amd' / 'csrc'}",
+                    str(ROOT / "tests" / "native" / "dropin_host_test.cpp"),
+                    str(ROOT / "goofy_amd" / "csrc" / "capi.cpp"), "-pthread", "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "errors=0" in r.stdout, r.stdout + r.stderr
+    assert "WARNING: ThreadSanitizer" not in r.stderr, r.stderr
