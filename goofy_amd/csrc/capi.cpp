@@ -49,10 +49,12 @@ void clear_error() { t_last_error.clear(); }
 
 // ---- device -------------------------------------------------------------------
 
+constexpr int kMaxDevices = 64;
+
 int device_info(DeviceInfo* out)
 {
     static std::mutex mu;
-    static DeviceInfo cache[64];
+    static DeviceInfo cache[kMaxDevices];
     int count = 0;
     if (hipGetDeviceCount(&count) != hipSuccess || count <= 0) {
         (void)hipGetLastError();
@@ -61,7 +63,7 @@ int device_info(DeviceInfo* out)
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return fail_hip(e, "hipGetDevice");
-    if (dev < 0 || dev >= 64) return fail(GOOFY_ERR_INVALID, "device index out of range");
+    if (dev < 0 || dev >= kMaxDevices) return fail(GOOFY_ERR_INVALID, "device index out of range");
     std::lock_guard<std::mutex> lock(mu);
     if (cache[dev].device != dev) {
         hipDeviceProp_t prop;
@@ -108,8 +110,8 @@ bool cfg_valid(const LaunchCfg& c)
 // rows is staged, reads the slot over PCIe part by part as the host marks the
 // parts, writes its blocks to pinned memory over PCIe and marks them group by
 // group, so that the link runs from the first part staged to the last block,
-// and the host copies rows in and blocks out meanwhile.  Chunks alternate
-// between two streams: the next chunk's kernel is waiting when one ends.  DXT1 /
+// and the host copies rows in and blocks out meanwhile (a caller's chunks behind
+// the one that is so launched, and other callers' chunks: StagingLink).  DXT1 /
 // ETC2 RGBA8 in us per call; in the middle images up to 8 MiB with a fed kernel
 // and a stream synchronisation before the blocks were copied out, larger ones by
 // copy engines both ways (8 MiB chunks, plain kernels); on the left images up to
@@ -149,9 +151,29 @@ static bool launches_block()
     return false;
 }
 
+// A device's link, and who of its callers may have a kernel there that waits for
+// its host thread (a turn, from the launch to the last block collected): one
+// chunk of 2 MiB and more at a time, on stream[0], or up to three smaller ones.
+// Chunks that get no turn are staged first; the large ones then follow one
+// another on stream[1], so that two at most share the link.  With the kernels
+// of all callers beside each other, callers that had started together ended
+// together, and the link stood still while they staged their next images.  In
+// us per image with 1 / 2 / 4 threads, copy engines -> every chunk launched
+// before it is staged -> with turns:
+//    512x512      53 / 44 / 29       ->    35 / 30 / 22       ->    36 / 30 / 22
+//   1024x1024    150 / 115 / 97      ->   107 / 97 / 86       ->   107 / 94 / 83
+//   2048x2048    498 / 324 / 326     ->   410 / 365 / 335     ->   408 / 318 / 318
+//   4096x4096   1508 / 1300 / 1308   ->  1390 / 1355 / 1340   ->  1370 / 1250 / 1250
+// 512x512 with all chunks in turn on the two streams: 35 / 36 / 24.
+struct StagingLink {
+    std::atomic<int> turns{0};
+    hipStream_t stream[2] = {};
+};
+
 struct StagingCtx {
     int device = -1;
-    hipStream_t stream[2] = {};
+    StagingLink* link = nullptr;
+    hipStream_t stream = nullptr;  // of chunks below 2 MiB
     hipEvent_t ended[2] = {};
     struct Slot {
         uint8_t* in = nullptr;     // staged rows
@@ -160,7 +182,21 @@ struct StagingCtx {
     } slot[kSlots];
     size_t in_cap = 0, out_cap = 0;
     uint64_t call = 0;  // the number of the last launch
-    bool stage_first = launches_block();
+    bool turn = false;  // this call has one of the link's turns
+    const bool stage_first = launches_block();
+
+    bool take_turn(int limit)  // false too where an earlier chunk of this call has one
+    {
+        if (turn) return false;
+        if (link->turns.fetch_add(1, std::memory_order_acquire) < limit) return turn = true;
+        link->turns.fetch_sub(1, std::memory_order_relaxed);
+        return false;
+    }
+    void give_turn()
+    {
+        if (turn) link->turns.fetch_sub(1, std::memory_order_release);
+        turn = false;
+    }
 };
 
 class StagingPool {
@@ -176,7 +212,17 @@ public:
             }
         StagingCtx* c = new StagingCtx();
         c->device = device;
+        c->link = &links_[device];
         return c;
+    }
+    // Makes the streams of a link.
+    hipError_t ensure_link(StagingLink* l)
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        hipError_t e = hipSuccess;
+        for (hipStream_t& s : l->stream)
+            if (!s && e == hipSuccess) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+        return e;
     }
     void release(StagingCtx* c)
     {
@@ -187,6 +233,7 @@ public:
 private:
     std::mutex mu_;
     std::vector<StagingCtx*> free_;
+    StagingLink links_[kMaxDevices];
 };
 
 static StagingPool& staging_pool()
@@ -198,14 +245,16 @@ static StagingPool& staging_pool()
 static int ensure_ctx(StagingCtx* c, size_t in_bytes, size_t out_bytes)
 {
     hipError_t e;
-    for (int i = 0; i < 2; ++i) {
-        if (!c->stream[i] && (e = hipStreamCreateWithFlags(&c->stream[i], hipStreamNonBlocking)) != hipSuccess)
+    if (!c->stream) {
+        if ((e = staging_pool().ensure_link(c->link)) != hipSuccess ||
+            (e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess)
             return fail_hip(e, "hipStreamCreate");
-        if (!c->ended[i] && (e = hipEventCreateWithFlags(&c->ended[i], hipEventDisableTiming)) != hipSuccess)
-            return fail_hip(e, "hipEventCreate");
     }
+    for (hipEvent_t& ev : c->ended)
+        if (!ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess)
+            return fail_hip(e, "hipEventCreate");
     if (c->in_cap < in_bytes || c->out_cap < out_bytes) {
-        for (hipStream_t s : c->stream) (void)hipStreamSynchronize(s);
+        for (hipStream_t s : {c->stream, c->link->stream[0], c->link->stream[1]}) (void)hipStreamSynchronize(s);
         const size_t ni = std::max(in_bytes, c->in_cap), no = std::max(out_bytes, c->out_cap);
         for (StagingCtx::Slot& s : c->slot) {
             if (s.in) (void)hipHostFree(s.in);
@@ -279,16 +328,17 @@ struct HostImage {
 
 // The k-th chunk: `rows` block rows from the y0-th on, of them the `cols` block
 // columns from the x0-th on (all of them unless rows is 1), launched as number
-// `call`; of its groups of kFeedBlocks blocks the first `got` are in the
-// caller's memory.
+// `call` on `stream`; of its groups of kFeedBlocks blocks the first `got` are in
+// the caller's memory.  fed: it has a turn.
 struct HostChunk {
     uint32_t k = 0, y0 = 0, rows = 0, x0 = 0, cols = 0;
+    hipStream_t stream = nullptr;
     uint64_t call = 0;
     uint32_t got = 0;
+    bool fed = false;
 };
 
 static const StagingCtx::Slot& slot_of(const HostImage& im, const HostChunk& c) { return im.ctx->slot[c.k % kSlots]; }
-static hipStream_t stream_of(const HostImage& im, const HostChunk& c) { return im.ctx->stream[c.k & 1u]; }
 
 // Copies blocks [first, last) of a chunk from its slot to the caller, large
 // ranges split over the copy pool.
@@ -309,14 +359,17 @@ static void collect(const HostImage& im, const HostChunk& c, uint32_t first, uin
     });
 }
 
-// Launches a chunk's kernel and stages its rows.
+// Launches a chunk's kernel and stages its rows, in this order if it gets a
+// turn.
 static hipError_t start_chunk(const HostImage& im, HostChunk& c)
 {
     const StagingCtx::Slot& slot = slot_of(im, c);
     const uint32_t nblocks = c.cols * c.rows;
     const size_t row_bytes = (size_t)c.cols * 16, bytes = row_bytes * 4 * c.rows;
     const uint8_t* const rows = im.input + (size_t)c.y0 * 4 * im.stride + (size_t)c.x0 * 16;
-    const bool fed = bytes >= (128u << 10) && !im.ctx->stage_first;
+    const bool large = bytes >= (2u << 20) && !im.ctx->stage_first;
+    c.fed = bytes >= (128u << 10) && !im.ctx->stage_first && im.ctx->take_turn(large ? 1 : 3);
+    c.stream = large ? im.ctx->link->stream[c.fed ? 0 : 1] : im.ctx->stream;
     // Parts of whole block rows; where those have more than kWidePart, of
     // blocks in order, so that several threads copy what one row holds and the
     // kernel starts before all of it is staged (us per call, with parts of whole
@@ -346,12 +399,12 @@ static hipError_t start_chunk(const HostImage& im, HostChunk& c)
         else
             for (uint32_t p = 0; p < parts; ++p) f(p);
     };
-    if (!fed) each_part(stage);
+    if (!c.fed) each_part(stage);
     c.call = ++im.ctx->call;
     const hipError_t e =
         launch_fed(im.fmt, slot.in, row_bytes, slot.out, slot.out + nblocks * im.block_bytes, c.cols, nblocks,
-                   slot.feed, c.call, fed ? part_blocks : 0u, im.patience, stream_of(im, c));
-    if (e != hipSuccess || !fed) return e;
+                   slot.feed, c.call, c.fed ? part_blocks : 0u, im.patience, c.stream);
+    if (e != hipSuccess || !c.fed) return e;
     const FeedGuard guard{slot.feed, c.call, parts};
     each_part([&](uint32_t p) {
         stage(p);
@@ -372,25 +425,35 @@ static bool collect_marked(const HostImage& im, HostChunk& c)
     return c.got == groups;
 }
 
-// Waits for a chunk and collects it: by its marks, or, where they don't come
-// within 2 ms or don't reach, by its stream.
+// Waits for a chunk and collects it: by its marks, looking all the time for 2 ms
+// and then now and then, behind many other callers' chunks; or, where its kernel
+// gave up or no mark comes for 200 ms, by its stream.
 static hipError_t finish_chunk(const HostImage& im, HostChunk& c)
 {
-    const auto end = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
-    for (uint32_t look = 1; !collect_marked(im, c); ++look) {
-        if (c.got == kFeedMarks || (look % 64 == 0 && std::chrono::steady_clock::now() > end)) break;
-    }
-    if (c.got == feed_groups(c.cols * c.rows)) return hipSuccess;
+    using std::chrono::milliseconds;
     const StagingCtx::Slot& slot = slot_of(im, c);
-    const hipStream_t stream = stream_of(im, c);
     const uint32_t nblocks = c.cols * c.rows;
-    hipError_t e = hipStreamSynchronize(stream);
-    if (e == hipSuccess && __atomic_load_n(&slot.feed->gave_up, __ATOMIC_ACQUIRE) == c.call) {
-        e = launch_any(im.fmt, im.cfg, slot.in, (size_t)c.cols * 16, slot.out, slot.out + nblocks * im.block_bytes,
-                       c.cols, nblocks, stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    const auto gave_up = [&] { return __atomic_load_n(&slot.feed->gave_up, __ATOMIC_ACQUIRE) == c.call; };
+    const auto start = std::chrono::steady_clock::now();
+    hipError_t e = hipSuccess;
+    for (uint32_t look = 1; !collect_marked(im, c); ++look) {
+        if (look % 64 != 0) continue;
+        const auto waited = std::chrono::steady_clock::now() - start;
+        if (waited < milliseconds(2)) continue;
+        if (gave_up() || waited > milliseconds(200)) {
+            e = hipStreamSynchronize(c.stream);
+            if (e == hipSuccess && gave_up()) {
+                e = launch_any(im.fmt, im.cfg, slot.in, (size_t)c.cols * 16, slot.out,
+                               slot.out + nblocks * im.block_bytes, c.cols, nblocks, c.stream);
+                if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+            }
+            if (e == hipSuccess) collect(im, c, c.got * kFeedBlocks, nblocks);
+            break;
+        }
+        std::this_thread::sleep_for(std::chrono::microseconds(50));
+        look = 63;
     }
-    if (e == hipSuccess) collect(im, c, c.got * kFeedBlocks, nblocks);
+    if (c.fed) im.ctx->give_turn();
     return e;
 }
 
@@ -424,8 +487,9 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
         bool done = false;
         ~Release()
         {
-            for (hipStream_t s : c->stream)
+            for (hipStream_t s : {c->stream, c->link->stream[0], c->link->stream[1]})
                 if (s && !done) (void)hipStreamSynchronize(s);
+            c->give_turn();
             staging_pool().release(c);
         }
     } rel{ctx};
@@ -462,9 +526,9 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
             y0 += cb;
         }
     }
-    // a marker behind the kernels while they run, for a caller that goes on to
-    // wait for the device
-    for (uint32_t i = 0; i < std::min(k, 2u); ++i) (void)hipEventRecord(ctx->ended[i], ctx->stream[i]);
+    // a marker behind the last kernels while they run, for a caller that goes on
+    // to wait for the device
+    for (uint32_t i = 0; i < std::min(k, 2u); ++i) (void)hipEventRecord(ctx->ended[i], ring[(k - 1u - i) % kSlots].stream);
     while (e == hipSuccess && oldest < k) e = finish_chunk(im, ring[oldest++ % kSlots]);
     if (e != hipSuccess) return fail_hip(e, "drop-in staging");
     rel.done = true;

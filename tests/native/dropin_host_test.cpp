@@ -22,7 +22,7 @@
 
 using namespace goofy_impl;
 
-static int g_errors = 0;
+static std::atomic<int> g_errors{0};
 #define CHECK(cond, ...)                                           \
     do {                                                           \
         if (!(cond)) {                                             \
@@ -39,6 +39,7 @@ std::mutex g_mu;
 std::map<hipStream_t, std::vector<std::thread>> g_running;
 size_t g_largest_part = 0, g_largest_launch = 0, g_launches = 0;  // bytes of pixels
 bool g_late = false;                                              // fed kernels give up at once
+std::atomic<int> g_unstaged{0}, g_most_unstaged{0};               // kernels that wait for their hosts
 uintptr_t g_next = 0x1000;
 
 uint64_t digest(const uint8_t* src, size_t pitch, uint64_t bx, uint64_t by, int fmt)
@@ -114,6 +115,7 @@ hipError_t launch_fed(int fmt, const void* src, size_t pitch, void* dst, void* d
     g_largest_launch = std::max(g_largest_launch, (size_t)nblocks * 64);
     if (part_blocks) g_largest_part = std::max(g_largest_part, (size_t)part_blocks * 64);
     const bool late = g_late && part_blocks;
+    if (part_blocks) g_most_unstaged = std::max(g_most_unstaged.load(), ++g_unstaged);
     g_running[stream].emplace_back([=] {
         for (uint32_t group = 0; group < feed_groups(nblocks); ++group) {
             const uint32_t first = group * kFeedBlocks, end = std::min(first + kFeedBlocks, nblocks);
@@ -121,11 +123,13 @@ hipError_t launch_fed(int fmt, const void* src, size_t pitch, void* dst, void* d
                 for (uint32_t p = first / part_blocks; p <= (end - 1) / part_blocks; ++p)
                     while (__atomic_load_n(&feed->part[p].staged, __ATOMIC_ACQUIRE) != call) {
                         if (late) {
+                            --g_unstaged;
                             __atomic_store_n(&feed->gave_up, call, __ATOMIC_RELEASE);
                             return;
                         }
                         std::this_thread::yield();
                     }
+            if (part_blocks && end == nblocks) --g_unstaged;
             for (uint32_t b = first; b < end; ++b)
                 write_block(fmt, (uint8_t*)dst, (uint8_t*)dst2, b,
                             digest((const uint8_t*)src, pitch, b % bw, b / bw, fmt));
@@ -220,10 +224,40 @@ void wide()
     }
 }
 
+// Several threads at once: of all callers, one kernel of 2 MiB and more at a
+// time waits for its host thread, or three smaller ones, and the turns for that
+// come back from calls of every kind.
+void threads()
+{
+    for (int run : {0, 1, 2, 3}) {
+        const bool mixed = run & 1;
+        g_late = run & 2;
+        g_most_unstaged = 0;
+        std::vector<std::thread> t;
+        for (unsigned i = 0; i < 4; ++i)
+            t.emplace_back([i, mixed] {
+                for (unsigned r = 0; r < 3; ++r) {
+                    compare(0, 2048, 516 + 1024 * (i & 1), 0);
+                    compare(0, 64, 64, 0);
+                    for (unsigned k = 0; mixed && k < 20; ++k) compare(GOOFY_FORMAT_ETC1, 128 + 16 * i, 256, 16);
+                }
+            });
+        for (std::thread& x : t) x.join();
+        CHECK(g_most_unstaged >= 1 && g_most_unstaged <= (mixed ? 3 : 1), "%d kernels waited for their hosts at once",
+              g_most_unstaged.load());
+    }
+    g_late = false;
+    for (unsigned h : {512u, 2048u}) {
+        g_most_unstaged = 0;
+        compare(0, 512, h, 0);
+        CHECK(g_most_unstaged == 1, "a turn was lost");
+    }
+}
+
 const struct {
     const char* name;
     void (*go)();
-} kTests[] = {{"sizes", sizes}, {"wide", wide}};
+} kTests[] = {{"sizes", sizes}, {"wide", wide}, {"threads", threads}};
 
 }  // namespace
 
@@ -236,6 +270,6 @@ int main(int argc, char** argv)
     }
     for (auto& r : g_running)
         for (std::thread& t : r.second) t.join();
-    std::printf("errors=%d\n", g_errors);
+    std::printf("errors=%d\n", g_errors.load());
     return g_errors != 0;
 }

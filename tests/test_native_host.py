@@ -210,8 +210,9 @@ def test_quality_calls_on_host(quality_host, name):
 @pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
 def test_dropin_staging_on_host(tmp_path):
     """tests/native/dropin_host_test.cpp: the drop-in's staging with threads
-    in place of its kernels, under ThreadSanitizer: every path and format, and
-    very wide rows in parts that several threads share."""
+    in place of its kernels, under ThreadSanitizer: every path and format,
+    very wide rows in parts that several threads share, and several callers, few
+    of whose kernels wait for their host threads at a time."""
     exe = tmp_path / "dropin_host_test"
     subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=thread", "-D__HIP_PLATFORM_AMD__",
                     "-I/opt/rocm/include", f"-I{ROOT / 'include'}", f"-I{ROOT / 'goofy_amd' / 'csrc'}",
