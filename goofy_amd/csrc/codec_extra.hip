@@ -80,10 +80,6 @@ __device__ __forceinline__ uint4 load_block_fmt(const uint8_t* blocks, uint64_t 
     }
 }
 
-// Cache policies of the decoders' stores: streaming, streaming written through
-// (sc0 sc1 nt), and cached.
-constexpr int kStream = 2, kStreamThrough = 19, kCached = 0;
-
 template <int FMT, int STORE>
 __global__ __launch_bounds__(256) void k_decode(const uint8_t* __restrict__ blocks, uint8_t* __restrict__ dst,
                                                 uint64_t pitch, uint32_t bw, uint32_t nblocks, uint64_t magic,
@@ -457,27 +453,6 @@ static void decode_go(int store, dim3 grid, hipStream_t stream, const uint8_t* b
     else go(k_decode<FMT, kStream>);
 }
 
-// How a decode stores depends on how its rows lie on the 64-byte sectors.
-//   Rows on sectors: every store fills whole sectors, and writing them through
-// is fastest.  Other rows: neighbouring waves share a sector at their ends,
-// which their XCD's L2 has to bring together, so runs of workgroups per XCD and
-// no writing through; cached stores keep more of them together, but only
-// images too large to lie in the last-level cache gain by that.  Measured in us
-// (BC1 / ETC2 RGBA8), streaming in linear order -> as chosen here: 2048^2
-// 5.2 / 5.7 -> 4.2 / 4.5, 4096^2 13.8 / 15.7 -> 12.2 / 14.9, 8192^2 47.2 / 53.9
-// -> 45.8 / 52.9, with a pitch of 32896 55.3 / 59.7 -> 46.6 / 53.2; rows off the
-// sectors 3076^2 10.3 / 11.3 -> 9.8 / 10.9, 6004^2 36.9 / 35.9 -> 31.9 / 34.4,
-// 8196x8192 64.9 / 62.2 -> 54.4 / 57.8.  Cached against streaming there, both in
-// runs: 3076^2 10.1 / 11.7 and 9.8 / 10.9, 4100^2 14.6 / 17.2 and 15.3 / 17.1,
-// 6004^2 31.9 / 34.6 and 34.6 / 34.4, 7004^2 42.5 / 43.9 and 47.7 / 45.5; written
-// through at 8196x8192 61.4 / 67.6.
-static int decode_store(int fmt, const void* dst, size_t pitch, uint32_t height)
-{
-    if (pitch % 64 == 0 && (uintptr_t)dst % 64 == 0) return kStreamThrough;
-    const size_t large = fmt < 2 ? (size_t)64 << 20 : (size_t)160 << 20;
-    return pitch * height >= large ? kCached : kStream;
-}
-
 hipError_t launch_decode(int fmt, const void* blocks, void* dst, uint32_t width, uint32_t height, size_t pitch,
                          hipStream_t stream)
 {
@@ -487,7 +462,7 @@ hipError_t launch_decode(int fmt, const void* blocks, void* dst, uint32_t width,
     const uint64_t magic = div_magic(bw);
     const uint8_t* b = static_cast<const uint8_t*>(blocks);
     uint8_t* d = static_cast<uint8_t*>(dst);
-    const int store = decode_store(fmt, dst, pitch, height);
+    const int store = decode_store(fmt, bw, dst, pitch, height);
     switch (fmt) {
     case 0: decode_go<0>(store, grid, stream, b, d, pitch, bw, nblocks, magic); break;
     case 1: decode_go<1>(store, grid, stream, b, d, pitch, bw, nblocks, magic); break;

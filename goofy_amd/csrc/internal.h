@@ -152,6 +152,37 @@ hipError_t launch_synth(const void* params, void* dst, uint32_t width, uint32_t 
                         hipStream_t stream);
 hipError_t launch_decode(int fmt, const void* blocks, void* dst, uint32_t width, uint32_t height, size_t pitch,
                          hipStream_t stream);
+// Cache policies of the decoders' stores: streaming, streaming written through
+// (sc0 sc1 nt), and cached.
+constexpr int kStream = 2, kStreamThrough = 19, kCached = 0;
+
+// How a decode stores depends on how what its waves write (the pixels of 64
+// blocks in order) lies on the 64-byte sectors.
+//   Rows on sectors, of whole groups of 4 blocks: every wave begins and ends on a
+// sector, every store fills whole ones, and writing them through is fastest.
+// Otherwise neighbouring waves share a sector at their ends, which their XCD's
+// L2 has to bring together, so runs of workgroups per XCD and no writing
+// through; cached stores keep more of them together, but only images too large
+// to lie in the last-level cache gain by that.  Measured in us
+// (BC1 / ETC2 RGBA8), streaming in linear order -> as chosen here: 2048^2
+// 5.2 / 5.7 -> 4.2 / 4.5, 4096^2 13.8 / 15.7 -> 12.2 / 14.9, 8192^2 47.2 / 53.9
+// -> 45.8 / 52.9, with a pitch of 32896 55.3 / 59.7 -> 46.6 / 53.2; rows off the
+// sectors 3076^2 10.3 / 11.3 -> 9.8 / 10.9, 6004^2 36.9 / 35.9 -> 31.9 / 34.4,
+// 8196x8192 64.9 / 62.2 -> 54.4 / 57.8.  Cached against streaming there, both in
+// runs: 3076^2 10.1 / 11.7 and 9.8 / 10.9, 4100^2 14.6 / 17.2 and 15.3 / 17.1,
+// 6004^2 31.9 / 34.6 and 34.6 / 34.4, 7004^2 42.5 / 43.9 and 47.7 / 45.5; written
+// through at 8196x8192 61.4 / 67.6.  Rows on sectors with a width that is no
+// multiple of 16 pixels, streaming in linear order / written through / as chosen
+// here: 2052^2 5.5 5.9 / 5.9 6.3 / 5.0 5.5, 3076^2 10.2 11.3 / 11.2 11.4 / 9.6
+// 10.6, 4100^2 16.6 18.1 / 17.3 18.1 / 14.3 16.7, 6004^2 36.7 36.0 / 35.2 37.5 /
+// 33.0 33.9, 8196x8192 64.5 62.3 / 60.7 66.2 / 56.2 58.9.
+inline int decode_store(int fmt, uint32_t bw, const void* dst, size_t pitch, uint32_t height)
+{
+    if (pitch % 64 == 0 && (uintptr_t)dst % 64 == 0 && bw % 4 == 0) return kStreamThrough;
+    const size_t large = fmt < 2 ? (size_t)64 << 20 : (size_t)160 << 20;
+    return pitch * height >= large ? kCached : kStream;
+}
+
 // Quality sums: squared errors of bytes 0..3, then the sum of squared luma
 // differences times 10^4 (an exact integer with the harness's weights).
 struct QualitySums {

@@ -205,6 +205,15 @@ def test_decode_stores_by_row_alignment(gpu, w, h, pad, offset, fmt):
         assert np.array_equal(rows[y:y + n, :w * 4].reshape(-1), strip.download(w * 4 * n)), y
 
 
+@pytest.mark.parametrize("fmt", [W.DXT1, W.ETC1, W.DXT5, W.ETC2])
+@pytest.mark.parametrize("w,h,pad", [(1028, 272, 48), (36, 1028, 48), (4100, 4100, 48), (6500, 6500, 48)])
+def test_decode_stores_of_ragged_rows_on_sectors(gpu, w, h, pad, fmt):
+    """The same for rows that lie on 64-byte sectors but hold no whole groups
+    of 4 blocks, so that waves end inside a sector."""
+    assert (w * 4 + pad) % 64 == 0 and w % 16
+    test_decode_stores_by_row_alignment(gpu, w, h, pad, 0, fmt)
+
+
 def integer_sums(src, dec):
     """The round-trip sums in integers: squared error of bytes 0..3, and
     10^4 x the harness's luma error sum (its weights 0.21 / 0.72 / 0.07 on

@@ -221,3 +221,15 @@ def test_dropin_staging_on_host(tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and "errors=0" in r.stdout, r.stdout + r.stderr
     assert "WARNING: ThreadSanitizer" not in r.stderr, r.stderr
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_decode_store_rule_on_host(tmp_path):
+    """A decode writes its stores through exactly where every wave's pixels
+    begin and end on 64-byte sectors (tests/native/decode_store_rule.cpp)."""
+    exe = tmp_path / "decode_store_rule"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    f"-I{ROOT / 'include'}", f"-I{ROOT / 'goofy_amd' / 'csrc'}",
+                    str(ROOT / "tests" / "native" / "decode_store_rule.cpp"), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "decode store rule ok" in r.stdout, r.stdout + r.stderr
