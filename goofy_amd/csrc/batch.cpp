@@ -197,6 +197,12 @@ Key shape_key(const goofy_batch* b)
     return Key{b->arch, lb, lpt, (int)(dxt * 10 / (uint64_t)n + 11 * (alpha * 10 / (uint64_t)n))};
 }
 
+// First line of the tuning file.  The number goes up whenever a field of a shape
+// comes to mean something else, or the kernels change so that times of earlier
+// builds no longer rank the shapes: files of another number (and those of 1,
+// which had no such line) are not used, and written anew by the next autotune.
+constexpr int kTuneVersion = 2;  // 2: tile_order 1 is runs of tiles per XCD, no longer eighths
+
 void load_file_cache()
 {
     static bool loaded = false;
@@ -206,6 +212,11 @@ void load_file_cache()
     if (!path) return;
     FILE* f = std::fopen(path, "r");
     if (!f) return;
+    int version = 0;
+    if (std::fscanf(f, "goofy-tune %d", &version) != 1 || version != kTuneVersion) {
+        std::fclose(f);
+        return;
+    }
     char arch[64];
     int lb, lpt, mix, bpl, wg, wpc, nt, order;
     while (std::fscanf(f, "%63s %d %d %d %d %d %d %d %d", arch, &lb, &lpt, &mix, &bpl, &wg, &wpc, &nt, &order) == 9) {
@@ -221,6 +232,7 @@ void save_file_cache()
     if (!path) return;
     FILE* f = std::fopen(path, "w");
     if (!f) return;
+    std::fprintf(f, "goofy-tune %d\n", kTuneVersion);
     for (const auto& kv : tune_cache()) {
         const LaunchCfg& c = kv.second;
         std::fprintf(f, "%s %d %d %d %d %d %d %d %d\n", std::get<0>(kv.first).c_str(), std::get<1>(kv.first),

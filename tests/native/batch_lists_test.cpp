@@ -5,7 +5,7 @@
 // list the way the kernel does, but with every index checked, and marks the
 // blocks it covers.  So a list that is rewritten, resized or freed while a
 // launch or a captured graph still reads it shows as an error here, with no
-// GPU.  Arguments: the names of the tests to run (none: all).
+// GPU.  Arguments: the names of the tests to run.
 #include <hip/hip_runtime_api.h>
 
 #include <cstdio>
@@ -175,6 +175,7 @@ int device_info(DeviceInfo* out)
 {
     *out = DeviceInfo{};
     out->num_cus = 256;
+    std::snprintf(out->arch, sizeof out->arch, "test");
     return GOOFY_OK;
 }
 LaunchCfg auto_cfg(uint64_t, int) { return LaunchCfg{1, 4, 0, 1, 0}; }
@@ -332,17 +333,41 @@ void events()
     finish(b);
 }
 
+// The tuning file (GOOFY_TUNE_CACHE): rows of a build whose shapes meant
+// something else are left alone, those of this one are taken.  One process each,
+// as the file is read once.
+void expect(const char* what, const goofy_launch_config& want)
+{
+    goofy_batch* b = make_plan();
+    goofy_launch_config c{};
+    CHECK(goofy_batch_get_config(b, &c) == GOOFY_OK && !std::memcmp(&c, &want, sizeof c),
+          "%s: %d blocks per lane, %d waves, %d per CU, streaming %d, order %d", what, c.blocks_per_lane, c.wg_waves,
+          c.waves_per_cu, c.nontemporal, c.tile_order);
+    finish(b);
+}
+void tune_file_foreign() { expect("shape after a foreign file", shape(1)); }
+void tune_file_write()
+{
+    goofy_batch* b = make_plan();
+    CHECK(goofy_batch_autotune(b, nullptr, 1, nullptr, nullptr) == GOOFY_OK, "autotune");
+    advance(nullptr, g_ticket);
+    finish(b);
+}
+void tune_file_read() { expect("shape after our file", goofy_launch_config{1, 2, 0, 0, 0}); }  // all alike: the first
+
 const struct {
     const char* name;
     void (*go)();
-} kTests[] = {{"captured", captured}, {"streams", streams}, {"per_thread", per_thread}, {"events", events}};
+} kTests[] = {{"captured", captured}, {"streams", streams}, {"per_thread", per_thread}, {"events", events},
+             {"tune_file_foreign", tune_file_foreign}, {"tune_file_write", tune_file_write},
+             {"tune_file_read", tune_file_read}};
 
 }  // namespace
 
 int main(int argc, char** argv)
 {
     for (const auto& t : kTests) {
-        bool want = argc < 2;
+        bool want = false;
         for (int i = 1; i < argc; ++i) want |= !std::strcmp(argv[i], t.name);
         if (want) t.go();
     }

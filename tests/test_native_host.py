@@ -183,6 +183,26 @@ def test_batch_worklists_on_host(batch_lists, name):
     assert r.returncode == 0 and "errors=0" in r.stdout, r.stdout + r.stderr
 
 
+def test_batch_tune_file_on_host(batch_lists, tmp_path):
+    """A tuning file of a build that meant other shapes by its rows (no version
+    line, or another version) is not used; one that this build wrote is."""
+    import os
+    path = tmp_path / "tune"
+    env = {**os.environ, "GOOFY_TUNE_CACHE": str(path)}
+
+    def run(name):
+        r = subprocess.run([str(batch_lists), name], capture_output=True, text=True, timeout=120, env=env)
+        assert r.returncode == 0 and "errors=0" in r.stdout, r.stdout + r.stderr
+
+    rows = "".join(f"test {lb} {lpt} {mix} 4 8 16 1 1\n" for lb in range(8, 16) for lpt in range(4, 12) for mix in (0, 10))
+    for text in (rows, "goofy-tune 1\n" + rows, "goofy-tune\n" + rows, "", "goofy-tune 999\n" + rows):
+        path.write_text(text)
+        run("tune_file_foreign")
+    run("tune_file_write")
+    assert path.read_text().startswith("goofy-tune ")
+    run("tune_file_read")
+
+
 @pytest.fixture(scope="module")
 def quality_host(tmp_path_factory):
     """tests/native/quality_host_test.cpp: the host side of the quality calls
