@@ -176,6 +176,16 @@ static bool words_arrive(const QualityHost* h, uint32_t n)
     return true;
 }
 
+// A quality call reads its sums back, so it cannot be captured: a replay would
+// only write to a work area and to host memory that are no longer its own.
+static int refuse_capture(hipStream_t stream)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();  // the launch says why
+    return cap == hipStreamCaptureStatusNone ? GOOFY_OK
+                                             : fail(GOOFY_ERR_HIP, "quality call on a stream that is being captured");
+}
+
 // Runs `launch(y0, rows, dest)` on `stream` for the stripes [y0, y0 + rows) of
 // `height` rows, at most max_rows each, waits for the stream and fills `out`
 // with getMsePsnr's figures (Src/main.cpp:403-469) from the stripes' sums.
@@ -186,11 +196,7 @@ static int run_quality(uint64_t pixels, uint32_t height, uint32_t max_rows, hipS
     DeviceInfo di;
     int rc = device_info(&di);
     if (rc != GOOFY_OK) return rc;
-    // The figures are read back here, so the call cannot be captured: a replay
-    // would only add to a work area that other calls use by then.
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();  // the launch says why
-    if (cap != hipStreamCaptureStatusNone) return fail(GOOFY_ERR_HIP, "quality call on a stream that is being captured");
+    if ((rc = refuse_capture(stream)) != GOOFY_OK) return rc;
     struct Use {  // on every path, the launches are through with the slot before it is reused
         QualitySlot slot;
         hipStream_t s;
@@ -267,7 +273,7 @@ int goofy_hip_quality_device_noalloc(int format, const void* d_blocks, const voi
     if (quality_scratch_bytes(stripe_blocks) > kQualityNoAllocBytes)
         return fail(GOOFY_ERR_TOO_LARGE, "quality grid larger than the fixed work area");
     DeviceInfo di;
-    if ((rc = device_info(&di)) != GOOFY_OK) return rc;
+    if ((rc = device_info(&di)) != GOOFY_OK || (rc = refuse_capture((hipStream_t)stream)) != GOOFY_OK) return rc;
     void* work = nullptr;
     hipError_t e = noalloc_scratch_address(di.device, &work);
     if (e != hipSuccess) return fail_hip(e, "hipGetSymbolAddress(quality work area)");

@@ -27,8 +27,8 @@ static int g_errors = 0;
 namespace {
 
 struct Counts {
-    int memset, launch, record, sync;
-    int all() const { return memset + launch + record + sync; }
+    int memset, launch, record, sync, copy;
+    int all() const { return memset + launch + record + sync + copy; }
 } g_n;
 bool g_capturing = false;
 bool g_writes = true;  // launches write their words
@@ -36,7 +36,7 @@ bool g_writes = true;  // launches write their words
 hipError_t launched(const QualityDest& dest)
 {
     ++g_n.launch;
-    if (g_writes)
+    if (g_writes && dest.host)
         for (uint32_t k = 0; k < kQualityWords; ++k) dest.host->word[k] = k + 1;
     return hipSuccess;
 }
@@ -63,7 +63,12 @@ hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st)
     return hipSuccess;
 }
 hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void*, size_t n, hipMemcpyKind, hipStream_t)
+{
+    ++g_n.copy;
+    std::memset(d, 0, n);
+    return hipSuccess;
+}
 const char* hipGetErrorString(hipError_t) { return "error"; }
 }
 
@@ -107,6 +112,10 @@ namespace {
 void* const kMem = (void*)(uintptr_t)4096;
 
 int images(goofy_quality* q) { return goofy_hip_quality_images_device(kMem, 1024, kMem, 1024, 256, 64, nullptr, q); }
+int noalloc(goofy_quality* q)
+{
+    return goofy_hip_quality_device_noalloc(0, kMem, kMem, 256, 64, 1024, nullptr, q);
+}
 int blocks(goofy_quality* q) { return goofy_hip_quality_device(0, kMem, kMem, 256, 64, 1024, nullptr, q); }
 
 void right(int (*call)(goofy_quality*), const char* what)
@@ -132,6 +141,13 @@ void capture()
             g_capturing = false;
             right(call, "after a capture");
         }
+    goofy_quality q{};
+    g_capturing = true;
+    g_n = {};
+    CHECK(noalloc(&q) == GOOFY_ERR_HIP, "under capture");
+    CHECK(g_n.all() == 0, "queued under capture: %d launches, %d copies, %d waits", g_n.launch, g_n.copy, g_n.sync);
+    g_capturing = false;
+    CHECK(noalloc(&q) == GOOFY_OK && g_n.launch == 1 && g_n.copy == 1, "after a capture");
 }
 
 // Words that are still unwritten when the stream has drained are an error, not
