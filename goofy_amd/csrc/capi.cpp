@@ -419,7 +419,7 @@ static bool collect_marked(const HostImage& im, HostChunk& c)
     const uint32_t nblocks = c.cols * c.rows, groups = feed_groups(nblocks);
     const HostFeed* const feed = slot_of(im, c).feed;
     uint32_t to = c.got;
-    while (to < std::min(groups, kFeedMarks) && __atomic_load_n(&feed->done[to], __ATOMIC_ACQUIRE) == c.call) ++to;
+    while (to < groups && __atomic_load_n(&feed->done[to], __ATOMIC_ACQUIRE) == c.call) ++to;
     if (to != c.got) collect(im, c, c.got * kFeedBlocks, std::min(to * kFeedBlocks, nblocks));
     c.got = to;
     return c.got == groups;
@@ -494,8 +494,9 @@ static int compress_host(int fmt, unsigned char* result, const unsigned char* in
         }
     } rel{ctx};
 
-    // Chunks of about 8 MiB: block rows, or, where one has more, pieces of one.
-    const size_t row_bytes = (size_t)width * 4, chunk = (size_t)8 << 20;
+    // Chunks of at most 8 MiB, as far as a launch's marks reach: block rows, or,
+    // where one has more, pieces of one.
+    const size_t row_bytes = (size_t)width * 4, chunk = (size_t)kFeedMarks * kFeedBlocks * 64;
     const unsigned cb = std::min(std::min((unsigned)std::max<size_t>(1, chunk / (row_bytes * 4)), bh), max_rows);
     const uint32_t pieces = (uint32_t)((row_bytes * 4 + chunk - 1) / chunk), cols = (bw + pieces - 1) / pieces;
     // dual: a chunk's staging output holds its blocks of the first format, then
