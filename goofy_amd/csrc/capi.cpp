@@ -105,8 +105,7 @@ bool cfg_valid(const LaunchCfg& c)
 // ---- host-memory drop-in: pinned staging, read by the kernels themselves ------
 //
 // goofy::compressDXT1/ETC1 take pageable host buffers.  The image goes in
-// chunks of block rows (about 8 MiB of pixels each) through three pinned
-// staging slots.  A chunk's kernel (k_encode_fed) is launched before any of its
+// chunks of at most 8 MiB of pixels through three pinned staging slots.  A chunk's kernel (k_encode_fed) is launched before any of its
 // rows is staged, reads the slot over PCIe part by part as the host marks the
 // parts, writes its blocks to pinned memory over PCIe and marks them group by
 // group, so that the link runs from the first part staged to the last block,
@@ -118,10 +117,10 @@ bool cfg_valid(const LaunchCfg& c)
 // 8 MiB with a plain kernel per 512 KiB staged:
 //     64x64      18 / 18     ->    17 / 17     ->    14 / 15
 //    512x512     55 / 59     ->    45 / 49     ->    38 / 40
-//   1440x1448   274 / 328    ->   227 / 274    ->   194 / 200
-//   2048x2048   490 / 532    ->   494 / 535    ->   408 / 410
-//   4096x4096  1485 / 1540   ->  1490 / 1545   ->  1385 / 1410
-//   8192x8192  5455 / 5860   ->  5450 / 5820   ->  5140 / 5180
+//   1440x1448   274 / 328    ->   227 / 274    ->   194 / 198
+//   2048x2048   490 / 532    ->   494 / 535    ->   400 / 405
+//   4096x4096  1485 / 1540   ->  1490 / 1545   ->  1350 / 1385
+//   8192x8192  5455 / 5860   ->  5450 / 5820   ->  5140 / 5170
 // The kernels read 52 GB/s over the link.  With the first chunk fed and copy
 // engines for the others the calls were bound by the host (4096x4096 1473 /
 // 1617, 8192x8192 5530 / 6790).

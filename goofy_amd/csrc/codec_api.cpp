@@ -187,8 +187,9 @@ static int refuse_capture(hipStream_t stream)
 }
 
 // Runs `launch(y0, rows, dest)` on `stream` for the stripes [y0, y0 + rows) of
-// `height` rows, at most max_rows each, waits for the stream and fills `out`
-// with getMsePsnr's figures (Src/main.cpp:403-469) from the stripes' sums.
+// `height` rows, at most max_rows each, waits for their words (words_arrive) and
+// fills `out` with getMsePsnr's figures (Src/main.cpp:403-469) from the stripes'
+// sums.
 extern "C++" template <typename Launch>
 static int run_quality(uint64_t pixels, uint32_t height, uint32_t max_rows, hipStream_t stream, goofy_quality* out,
                        Launch&& launch)

@@ -334,8 +334,8 @@ __device__ __forceinline__ void sqerr_loop(const uint8_t* __restrict__ blocks, c
 // pixels, ey = sum of squared luma differences x 10^4 with the harness's
 // weights (0.21, 0.72, 0.07 on bytes 2, 1, 0 -- getMsePsnr reads a pixel as a
 // little-endian word and takes bits 16..23 as "red").  Grid-stride over the
-// blocks (at most 1536 workgroups), one partial per workgroup; k_sums_final
-// adds the partials.
+// blocks (at most 1536 workgroups); finish_sums brings the workgroups' sums
+// together, or, for the allocation-free call, leaves them for k_sums_final.
 template <int FMT>
 __global__ __launch_bounds__(256) void k_sqerr(const uint8_t* __restrict__ blocks, const uint8_t* __restrict__ src,
                                                uint64_t pitch, uint32_t bw, uint32_t nblocks, uint64_t magic,
