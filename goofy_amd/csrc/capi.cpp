@@ -253,7 +253,8 @@ static int ensure_ctx(StagingCtx* c, size_t in_bytes, size_t out_bytes)
         if (!ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess)
             return fail_hip(e, "hipEventCreate");
     if (c->in_cap < in_bytes || c->out_cap < out_bytes) {
-        for (hipStream_t s : {c->stream, c->link->stream[0], c->link->stream[1]}) (void)hipStreamSynchronize(s);
+        if (c->in_cap)  // its last kernels have marked their blocks, but may not have ended
+            for (hipStream_t s : {c->stream, c->link->stream[0], c->link->stream[1]}) (void)hipStreamSynchronize(s);
         const size_t ni = std::max(in_bytes, c->in_cap), no = std::max(out_bytes, c->out_cap);
         for (StagingCtx::Slot& s : c->slot) {
             if (s.in) (void)hipHostFree(s.in);

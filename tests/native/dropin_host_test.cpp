@@ -18,6 +18,7 @@
 #include <thread>
 #include <vector>
 
+
 #include "internal.h"
 
 using namespace goofy_impl;
@@ -39,6 +40,7 @@ std::mutex g_mu;
 std::map<hipStream_t, std::vector<std::thread>> g_running;
 size_t g_largest_part = 0, g_largest_launch = 0, g_launches = 0;  // bytes of pixels
 bool g_late = false;                                              // fed kernels give up at once
+std::atomic<int> g_fed_us{0};                                      // how long kernels take that are launched before staging
 std::atomic<int> g_unstaged{0}, g_most_unstaged{0};               // kernels that wait for their hosts
 uintptr_t g_next = 0x1000;
 
@@ -130,6 +132,7 @@ hipError_t launch_fed(int fmt, const void* src, size_t pitch, void* dst, void* d
                         std::this_thread::yield();
                     }
             if (part_blocks && end == nblocks) --g_unstaged;
+            if (part_blocks && end == nblocks) std::this_thread::sleep_for(std::chrono::microseconds(g_fed_us));
             for (uint32_t b = first; b < end; ++b)
                 write_block(fmt, (uint8_t*)dst, (uint8_t*)dst2, b,
                             digest((const uint8_t*)src, pitch, b % bw, b / bw, fmt));
@@ -254,17 +257,37 @@ void threads()
     }
 }
 
+// A caller with a new context does not wait for a kernel whose rows another
+// caller has not staged, or which takes long.
+void waiting()
+{
+    const unsigned w = 1024, h = 512;  // 2 MiB
+    std::vector<uint8_t> img((size_t)w * h * 4, 1), out((size_t)w * h / 2), out2(out.size());
+    const auto call = [&](std::vector<uint8_t>& o) {
+        CHECK(goofy_hip_compress(0, o.data(), img.data(), w, h, w * 4) == GOOFY_OK, "call");
+    };
+    g_fed_us = 1500000;
+    std::thread other([&] { call(out2); });  // has the turn meanwhile
+    std::this_thread::sleep_for(std::chrono::milliseconds(50));
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int i = 0; i < 5; ++i) call(out);
+    const double wall = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+    CHECK(wall < 1.2, "%.0f ms: waited for the other caller", wall * 1e3);
+    other.join();
+    g_fed_us = 0;
+}
+
 const struct {
     const char* name;
     void (*go)();
-} kTests[] = {{"sizes", sizes}, {"wide", wide}, {"threads", threads}};
+} kTests[] = {{"sizes", sizes}, {"wide", wide}, {"threads", threads}, {"waiting", waiting}};
 
 }  // namespace
 
 int main(int argc, char** argv)
 {
-    for (const auto& t : kTests) {
-        bool want = argc < 2;
+    for (const auto& t : kTests) {  // "waiting" in a process of its own: it needs new contexts
+        bool want = argc < 2 && t.go != waiting;
         for (int i = 1; i < argc; ++i) want |= !std::strcmp(argv[i], t.name);
         if (want) t.go();
     }

@@ -238,9 +238,10 @@ def test_dropin_staging_on_host(tmp_path):
                     "-I/opt/rocm/include", f"-I{ROOT / 'include'}", f"-I{ROOT / 'goofy_amd' / 'csrc'}",
                     str(ROOT / "tests" / "native" / "dropin_host_test.cpp"),
                     str(ROOT / "goofy_amd" / "csrc" / "capi.cpp"), "-pthread", "-o", str(exe)], check=True)
-    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
-    assert r.returncode == 0 and "errors=0" in r.stdout, r.stdout + r.stderr
-    assert "WARNING: ThreadSanitizer" not in r.stderr, r.stderr
+    for args in ([], ["waiting"]):
+        r = subprocess.run([str(exe), *args], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0 and "errors=0" in r.stdout, r.stdout + r.stderr
+        assert "WARNING: ThreadSanitizer" not in r.stderr, r.stderr
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
